@@ -15,8 +15,9 @@
 //      direction) and h0 quantisation (codes + masks), h[0] dequantised;
 //   3. code_gemm     : the time-parallel input projection W_q x_q summed exactly on int8 MFMA
 //      over pre-packed byte planes and rounded once to fp32 (exact_gemm.h);
-//   4. recurrence    : both directions' T steps in one clustered cooperative launch
-//      (recurrence_cl; cluster.h): a batch tile's hidden units split over a cluster of
+//   4. recurrence    : up to H = 256 one workgroup per two or four sequences with all of R_q in
+//      its VGPRs (recurrence_res: no exchange between workgroups); above that both directions'
+//      T steps in one clustered cooperative launch (recurrence_cl; cluster.h): a batch tile's hidden units split over a cluster of
 //      workgroups, the new h codes exchanged through global memory each step.  R_q lives in
 //      VGPRs as int8 MFMA fragments for the whole kernel; h_t arrives as int8 planes (16-bit
 //      codes as a high and a low byte plane); the pointwise update (bias rescale, gate
@@ -378,6 +379,25 @@ __device__ __forceinline__ float gate_tab(float q, const int *tab, float lo, uin
   return static_cast<float>(e >> 1);
 }
 
+// Fills the three gate tables from the LUT in LDS (every thread of the workgroup; the caller
+// synchronises before they are read).
+__device__ __forceinline__ void fill_gate_tables(const StepParams &p, const float *lut_f,
+                                                 const int *lut_n, int *gtab) {
+  for (int i = threadIdx.x; i < 3 * kGateTabMax; i += blockDim.x) {
+    const int g = i / kGateTabMax, e = i % kGateTabMax;
+    // selected, not indexed: a local array indexed by g would live in scratch memory
+    const Bounds gi = g == 0 ? p.zin : (g == 1 ? p.rin : p.nin);
+    const Bounds go = g == 0 ? p.zout : (g == 1 ? p.rout : p.nout);
+    const float zpx = g == 0 ? p.lut[0].zp_x : (g == 1 ? p.lut[1].zp_x : p.lut[2].zp_x);
+    if (e <= static_cast<int>(gi.hi - gi.lo)) {
+      uint8_t k = 0;
+      const float v = pwl_eval(gi.lo + static_cast<float>(e), lut_f + 48 * g, lut_f + 48 * g + 16,
+                               lut_n + 16 * g, lut_f + 48 * g + 32, zpx, go, k);
+      gtab[i] = static_cast<int>(v) * 2 | k;
+    }
+  }
+}
+
 // One (sequence, unit) step of the FP carrier (gru_forward_gpu_quant_fp.cu:138-393): both
 // linears from their exact sums (zero-point and bias terms, rescale, clamp), the three gates
 // through the PWL LUTs (thresholds, slopes, offsets in lut_f, shifts in lut_n; 48 floats and
@@ -491,6 +511,262 @@ __device__ __forceinline__ void store_point(const RecArgs &a, const StepParams &
       a.gout_m[m + g * H] = o.k_go[g];
     }
     a.h_m[stepH + oH] = o.k_h;
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// 4a. resident recurrence (H <= 256)
+// ---------------------------------------------------------------------------------
+// One workgroup owns NS sequences and all H units, and holds all of R_q in its VGPRs as int8
+// MFMA operands (H = 256: 192 KB of the CU's 512), so a step needs no other workgroup: the new
+// h codes go to the other waves through LDS, and the step's only synchronisation is one
+// workgroup barrier.  The clustered kernel below spends most of a step on the exchange through
+// the coherence point (4.1 us per step at the size below; this kernel 1.6).
+//
+// MFMA rows: 16x16x64 multiplies 16 rows, and NS <= 4 sequences have NS * NPL byte planes, so
+// the planes are rows too: row 4 s + q is plane q of sequence s, and lane group s (lanes 16 s ..
+// 16 s + 15) receives in its accumulator words 0 .. NPL - 1 the plane sums of sequence s for 16
+// units.  The idle rows cost nothing: the matrix units are busy 20% of a step.  A wave owns UPW
+// tiles of 16 units, all three gates, the whole K range, so no sums meet across waves.  With two
+// sequences and two tiles the second tile's sums move to the upper 32 lanes
+// (v_permlane32_swap) and each lane finishes exactly one (sequence, unit).
+//
+// The step's outputs are stored straight from registers, without branches (rows past B get an
+// offset outside the buffer), and the barrier waits for LDS only, so neither the stores nor the
+// input-projection loads (issued two steps ahead) are waited for early.
+//
+// Measured (both directions of B = 256, T = 200, H = 256; 8-bit gates, 16-bit h, saved codes):
+// 818 us clustered -> 322 us; one direction of B = 32, T = 98, H = 64 (inference): 283 -> 73 us.
+// What bounds it: the chain of one step (LDS reads, 24 MFMA per wave at H = 256, about 200 VALU of
+// the pointwise update, the barrier), with two waves per SIMD to overlap.
+enum { kResInfer = 0, kResCodes = 1, kResFloat = 2 };
+constexpr unsigned kResSkip = 0x80000000u;  // an offset past every buffer: the store is dropped
+
+struct ResArgs {
+  int nblk;      // workgroups per direction
+  int gate_tab;  // gate activations by table
+};
+
+// LDS: LUT floats and ints (1 KB), two h buffers [NS * NPL][64 KS + 16], gate tables.
+constexpr size_t res_lds_bytes(int npl, int ks, int ns, bool tab) {
+  return 1024 + static_cast<size_t>(2) * ns * npl * (64 * ks + 16) +
+         (tab ? sizeof(int) * 3 * kGateTabMax : 0);
+}
+
+// All of the workgroup's LDS accesses are complete; memory accesses stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+__device__ __forceinline__ void buf_f32(__amdgpu_buffer_rsrc_t r, float v, unsigned off) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, 0, 0);
+}
+__device__ __forceinline__ void buf_u16(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned off) {
+  __builtin_amdgcn_raw_buffer_store_b16(static_cast<unsigned short>(v), r, off, 0, 0);
+}
+__device__ __forceinline__ void buf_u8(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned off) {
+  __builtin_amdgcn_raw_buffer_store_b8(static_cast<unsigned char>(v), r, off, 0, 0);
+}
+
+template <int NPL, int KS, int UPW, int NS, int MODE>
+__global__ __launch_bounds__(512) void recurrence_res(RecArgs a0, RecArgs a1,
+                                                      const StepParams *__restrict__ ps,
+                                                      ResArgs ra) {
+  constexpr bool kMerge = UPW == 2 && NS == 2;  // two tiles' sums share one pass of the lanes
+  constexpr int NP = UPW == 2 && !kMerge ? 2 : 1;
+  constexpr int ROW = 64 * KS + 16, HB = NS * NPL * ROW;
+  extern __shared__ __align__(16) unsigned char smem[];
+  float *lut_f = reinterpret_cast<float *>(smem);
+  int *lut_n = reinterpret_cast<int *>(lut_f + 3 * 16 * 3);
+  int8_t *hs = reinterpret_cast<int8_t *>(smem + 1024);
+  int *gtab = reinterpret_cast<int *>(smem + 1024 + 2 * HB);  // 16-byte aligned
+  const int d = blockIdx.x / ra.nblk, blk = blockIdx.x % ra.nblk;
+  const RecArgs &a = d == 0 ? a0 : a1;
+  const StepParams &p = ps[d];
+  const int H = a.H, C = 3 * H, B = a.B, T = a.T, UT = H / 16;
+  const int tid = threadIdx.x, w = tid / 64, l = tid % 64, grp = l / 16, e = l % 16;
+
+  for (int i = tid; i < 3 * 16; i += blockDim.x) {
+    const int g = i / 16, s = i % 16;
+    lut_f[g * 48 + s] = p.lut[g].thr[s];
+    lut_f[g * 48 + 16 + s] = p.lut[g].qb[s];
+    lut_f[g * 48 + 32 + s] = p.lut[g].c[s];
+    lut_n[g * 16 + s] = p.lut[g].n[s];
+  }
+  for (int i = tid; i < 2 * HB / 4; i += blockDim.x) reinterpret_cast<int *>(hs)[i] = 0;
+  __syncthreads();
+  const int *tab = nullptr;
+  if (ra.gate_tab) {
+    fill_gate_tables(p, lut_f, lut_n, gtab);
+    tab = gtab;
+  }
+
+  // R_q fragments: tile UPW w + u, gate g, K-step s (zero beyond the tiles and H)
+  v4i rfr[UPW][3][KS];
+#pragma unroll
+  for (int u = 0; u < UPW; ++u)
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int ut = UPW * w + u;
+        rfr[u][g][s] = ut < UT && s < a.KS ? a.rfrag[((ut * 3 + g) * a.KS + s) * 64 + l]
+                                           : v4i{0, 0, 0, 0};
+      }
+
+  // the elements this lane finishes: pass k, (sequence b, unit j); offsets of its outputs within
+  // one step's rows, kResSkip where the element does not exist
+  float cst[NP][3][kChanParams], hold[NP];
+  unsigned og[NP], oh[NP], oc[NP], ov[NP], om[NP];
+  int8_t *hw[NP];
+  bool own[NP];
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    const int seq = kMerge ? grp % 2 : grp, ut = UPW * w + (kMerge ? grp / 2 : k);
+    const int b = NS * blk + seq, j = 16 * ut + e;
+    own[k] = seq < NS && ut < UT;
+    const bool ok = own[k] && b < B;
+    const unsigned row = static_cast<unsigned>(b) * H + j;
+    og[k] = ok ? 4u * (static_cast<unsigned>(b) * C + j) : kResSkip;
+    oh[k] = ok ? 4u * row : kResSkip;
+    if (MODE == kResCodes) {
+      const unsigned cr = ok ? codes_row(0, b, j, B, H) : 0;
+      oc[k] = ok ? 128u * cr + 2u * e : kResSkip;
+      om[k] = ok ? 32u * cr + 2u * e : kResSkip;
+    }
+    if (MODE == kResFloat) {
+      ov[k] = ok ? 4u * (4u * static_cast<unsigned>(b) * H + j) : kResSkip;
+      om[k] = ok ? static_cast<unsigned>(b) * C + j : kResSkip;
+      oc[k] = ok ? row : kResSkip;
+    }
+    const int jc = ut < UT ? j : 0;
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+#pragma unroll
+      for (int q = 0; q < kChanParams; ++q) cst[k][g][q] = a.chan[q * C + g * H + jc];
+    hold[k] = ok ? a.h0codes[row] : p.zp_h;
+    hw[k] = hs + (own[k] ? seq * NPL * ROW + j : 0);
+  }
+  auto put_h = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const int hc = static_cast<int>(hold[k] - a.h_offset);
+      if (own[k]) {
+        int8_t *dst = hw[k] + buf * HB;
+        dst[0] = static_cast<int8_t>(NPL == 1 ? hc : (hc & 255) - 128);
+        if (NPL == 2) dst[ROW] = static_cast<int8_t>(hc >> 8);
+      }
+    }
+  };
+  put_h(0);
+
+  // A operand: row l % 16 = 4 s + q; rows without a sequence or plane repeat plane 0 of the
+  // first (their sums are not read)
+  const int ar = e / 4 < NS && e % 4 < NPL ? (e / 4) * NPL + e % 4 : 0;
+  const int8_t *hr = hs + ar * ROW + 16 * grp;
+
+  const unsigned step_g = 4u * static_cast<unsigned>(B) * C, step_h = 4u * static_cast<unsigned>(B) * H;
+  const unsigned step_blk = static_cast<unsigned>((B + 15) / 16) * H;  // x 128 B of v codes, x 32 B
+  auto load_gih = [&](int t, float (&gi)[NP][3]) {
+    const auto r = cluster::buffer_rsrc(
+        a.gih + static_cast<size_t>(t < T ? t : T - 1) * B * C, step_g);
+#pragma unroll
+    for (int k = 0; k < NP; ++k)
+#pragma unroll
+      for (int g = 0; g < 3; ++g)
+        gi[k][g] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(r, og[k] + 4u * g * H, 0, 0));
+  };
+  const float plane_off = 128.0f + a.h_offset;
+
+  auto step = [&](int t, int par, float (&gi)[NP][3]) {
+    v4i acc[UPW][3];
+#pragma unroll
+    for (int u = 0; u < UPW; ++u)
+#pragma unroll
+      for (int g = 0; g < 3; ++g) acc[u][g] = v4i{0, 0, 0, 0};
+    v4i hf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      hf[s] = *reinterpret_cast<const v4i *>(hr + par * HB + 64 * s);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int u = 0; u < UPW; ++u)
+#pragma unroll
+        for (int g = 0; g < 3; ++g) acc[u][g] = mfma_i8(hf[s], rfr[u][g][s], acc[u][g]);
+    PointOut o[NP];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      float gh3[3];
+#pragma unroll
+      for (int g = 0; g < 3; ++g) {
+        int sum[2] = {acc[k][g][0], acc[k][g][NPL - 1]};
+        if constexpr (kMerge) {
+#pragma unroll
+          for (int q = 0; q < NPL; ++q)
+            sum[q] = __builtin_amdgcn_permlane32_swap(acc[0][g][q], acc[1][g][q], false, false)[0];
+          if (NPL == 1) sum[1] = sum[0];
+        }
+        gh3[g] = recombine_rh<NPL>(a.wide_acc, sum[0], sum[1], plane_off, a.h_offset, cst[k][g][6]);
+      }
+      o[k] = gru_point(gi[k], gh3, cst[k], p, lut_f, lut_n, hold[k], tab);
+      hold[k] = o[k].h;
+    }
+    put_h(par ^ 1);
+    lds_barrier();
+    // everything below is independent of the next step's reads
+    load_gih(t + 2, gi);
+    const size_t t64 = static_cast<size_t>(t);
+    const auto rh = cluster::buffer_rsrc(a.hout + (t64 + 1) * B * H, step_h);
+#pragma unroll
+    for (int k = 0; k < NP; ++k) buf_f32(rh, (o[k].h - p.zp_h) * p.eff_h, oh[k]);
+    if constexpr (MODE == kResCodes) {
+      const auto rc = cluster::buffer_rsrc(a.vc + t64 * step_blk * 64, step_blk * 128);
+      const auto rm = cluster::buffer_rsrc(a.mb + t64 * step_blk * 16, step_blk * 32);
+#pragma unroll
+      for (int k = 0; k < NP; ++k) {
+        buf_u16(rc, code_u16(o[k].z, p.zout.lo), oc[k]);
+        buf_u16(rc, code_u16(o[k].r, p.rout.lo), oc[k] + 32);
+        buf_u16(rc, code_u16(o[k].n, p.nout.lo), oc[k] + 64);
+        buf_u16(rc, code_u16(o[k].rh_n, p.rh.lo), oc[k] + 96);
+        buf_u16(rm, code_mask_bits(o[k]), om[k]);
+      }
+    } else if constexpr (MODE == kResFloat) {
+      const auto rv = cluster::buffer_rsrc(a.v + 4 * t64 * B * H, 4u * step_h);
+      const unsigned mb = static_cast<unsigned>(B) * C;
+      const auto ri = cluster::buffer_rsrc(a.ih_m + t64 * mb, mb);
+      const auto rr = cluster::buffer_rsrc(a.hh_m + t64 * mb, mb);
+      const auto rgi = cluster::buffer_rsrc(a.gin_m + t64 * mb, mb);
+      const auto rgo = cluster::buffer_rsrc(a.gout_m + t64 * mb, mb);
+      const auto rhm = cluster::buffer_rsrc(a.h_m + t64 * B * H, static_cast<unsigned>(B) * H);
+#pragma unroll
+      for (int k = 0; k < NP; ++k) {
+        buf_f32(rv, (o[k].z - p.zp_zout) * p.eff_zout, ov[k]);
+        buf_f32(rv, (o[k].r - p.zp_rout) * p.eff_rout, ov[k] + 4u * H);
+        buf_f32(rv, (o[k].n - p.zp_nout) * p.eff_nout, ov[k] + 8u * H);
+        buf_f32(rv, (o[k].rh_n - p.zp_rh) * p.eff_rh, ov[k] + 12u * H);
+#pragma unroll
+        for (int g = 0; g < 3; ++g) {
+          buf_u8(ri, o[k].k_ih[g], om[k] + g * H);
+          buf_u8(rr, o[k].k_hh[g], om[k] + g * H);
+          buf_u8(rgi, o[k].k_gi[g], om[k] + g * H);
+          buf_u8(rgo, o[k].k_go[g], om[k] + g * H);
+        }
+        buf_u8(rhm, o[k].k_h, oc[k]);
+      }
+    }
+  };
+  // two steps per turn: each keeps its own input registers and h buffer
+  float ga[NP][3], gb[NP][3];
+  load_gih(0, ga);
+  load_gih(1, gb);
+  lds_barrier();  // the h buffers, the LUT and the tables are in LDS
+  for (int t = 0;;) {
+    step(t, 0, ga);
+    if (++t >= T) break;
+    step(t, 1, gb);
+    if (++t >= T) break;
   }
 }
 
@@ -748,19 +1024,7 @@ __device__ __forceinline__ void recurrence_cl_pair(const RecArgs &a, const StepP
   const int *tab = nullptr;
   if (!STAGE && cl.gate_tab) {
     __syncthreads();  // the LUT is in LDS
-    for (int i = tid; i < 3 * kGateTabMax; i += blockDim.x) {
-      const int g = i / kGateTabMax, e = i % kGateTabMax;
-      // selected, not indexed: a local array indexed by g would live in scratch memory
-      const Bounds gi = g == 0 ? p.zin : (g == 1 ? p.rin : p.nin);
-      const Bounds go = g == 0 ? p.zout : (g == 1 ? p.rout : p.nout);
-      const float zpx = g == 0 ? p.lut[0].zp_x : (g == 1 ? p.lut[1].zp_x : p.lut[2].zp_x);
-      if (e <= static_cast<int>(gi.hi - gi.lo)) {
-        uint8_t k = 0;
-        const float v = pwl_eval(gi.lo + static_cast<float>(e), lut_f + 48 * g, lut_f + 48 * g + 16,
-                                 lut_n + 16 * g, lut_f + 48 * g + 32, zpx, go, k);
-        gtab[i] = static_cast<int>(v) * 2 | k;
-      }
-    }
+    fill_gate_tables(p, lut_f, lut_n, gtab);
     tab = gtab;  // read after the first cluster barrier (a workgroup barrier as well)
   }
   v4i rfr[kClMaxKPerWave][3];
@@ -1278,6 +1542,63 @@ static int forward_prologue(bool training, int T, int B, int I, int H, const rxm
   return 0;
 }
 
+// Resident recurrence of every direction (H <= 256): one ordinary launch of one workgroup per NS
+// sequences.  Returns 1 when launched, 0 when the caller takes another form.  Two sequences per
+// workgroup while that leaves every workgroup a CU of its own, else four (a second pass of the
+// lanes costs less than a second round of workgroups).  A forced poll limit (the timeout tests)
+// asks for the clustered form, the one that polls.
+template <int NPL, int KS, int UPW, int NS>
+static const void *res_kernel(int mode) {
+  if (mode == kResInfer) return reinterpret_cast<const void *>(&recurrence_res<NPL, KS, UPW, NS, kResInfer>);
+  if (mode == kResCodes) return reinterpret_cast<const void *>(&recurrence_res<NPL, KS, UPW, NS, kResCodes>);
+  return reinterpret_cast<const void *>(&recurrence_res<NPL, KS, UPW, NS, kResFloat>);
+}
+
+template <int NPL, int NS>
+static const void *res_kernel(int ks, int mode) {
+  if (ks == 1) return res_kernel<NPL, 1, 1, NS>(mode);
+  if (ks == 2) return res_kernel<NPL, 2, 1, NS>(mode);
+  return res_kernel<NPL, 4, 2, NS>(mode);
+}
+
+static int forward_recurrence_resident(FwdPlan *plans, int ndir, int T, int B, int I, int H,
+                                       hipStream_t stream) {
+  const int npl = plans[0].npl;
+  for (int k = 1; k < ndir; ++k)
+    if (plans[k].npl != npl || plans[k].ra.training != plans[0].ra.training) return 0;
+  if (H > kMaxH || std::getenv("RXMET_NO_CLUSTER") != nullptr ||
+      cluster::spin_limit() != cluster::kSpinLimit)
+    return 0;
+  // one step's rows are addressed with 31-bit byte offsets (v: 16 bytes per element)
+  if (16.0 * ((B + kTileB - 1) / kTileB * kTileB) * H >= 2147483648.0) return 0;
+  int device = 0, ncu = 0;
+  RXMET_CHECK_HIP(hipGetDevice(&device));
+  RXMET_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
+  const int ns = static_cast<int64_t>(ndir) * ((B + 1) / 2) <= ncu ? 2 : 4;
+  const int KS = plans[0].ra.KS, ks = KS <= 2 ? KS : 4, upw = ks == 4 ? 2 : 1;
+  ResArgs ra;
+  ra.nblk = (B + ns - 1) / ns;
+  ra.gate_tab = 1;
+  for (int k = 0; k < ndir; ++k) {
+    const StepParams &sp = plans[k].sp;
+    for (const Bounds &g : {sp.zin, sp.rin, sp.nin})
+      if (!(g.hi - g.lo < static_cast<float>(kGateTabMax))) ra.gate_tab = 0;
+  }
+  const int mode = !plans[0].ra.training ? kResInfer : (plans[0].ra.vc ? kResCodes : kResFloat);
+  const void *fn = npl == 1 ? (ns == 2 ? res_kernel<1, 2>(ks, mode) : res_kernel<1, 4>(ks, mode))
+                            : (ns == 2 ? res_kernel<2, 2>(ks, mode) : res_kernel<2, 4>(ks, mode));
+  const int waves = (H / 16 + upw - 1) / upw;
+  const FwdWorkspace ws(T, B, I, H);
+  StepParams host_ps[2] = {plans[0].sp, plans[ndir > 1 ? 1 : 0].sp};
+  StepParams *ps = reinterpret_cast<StepParams *>(plans[0].wsb + ws.sparams);
+  RXMET_CHECK_HIP(hipMemcpyAsync(ps, host_ps, sizeof(host_ps), hipMemcpyHostToDevice, stream));
+  void *args[] = {&plans[0].ra, &plans[ndir > 1 ? 1 : 0].ra, &ps, &ra};
+  rxmet::prof::Scope ps__("gru_fwd_recurrence", stream);
+  RXMET_CHECK_HIP(hipLaunchKernel(fn, dim3(ndir * ra.nblk), dim3(64 * waves), args,
+                                  res_lds_bytes(npl, ks, ns, ra.gate_tab != 0), stream));
+  return 1;
+}
+
 // Clustered launch over every direction when the grid can be resident at once; returns 1
 // when launched, 0 when the caller must use the per-tile recurrence.
 static int forward_recurrence_clustered(FwdPlan *plans, int ndir, int T, int B, int I, int H,
@@ -1458,7 +1779,8 @@ static int forward_dirs(int ndir, bool training, int T, int B, int I, int H,
       if (int r = forward_recurrence_stepped(plans[k], *dirs[k].params, T, B, I, H, stream)) return r;
     return 0;
   }
-  const int rc = forward_recurrence_clustered(plans, ndir, T, B, I, H, stream);
+  int rc = forward_recurrence_resident(plans, ndir, T, B, I, H, stream);
+  if (rc == 0) rc = forward_recurrence_clustered(plans, ndir, T, B, I, H, stream);
   if (rc < 0) return rc;
   if (rc == 1) return 0;
   RXMET_CHECK_ARG(H <= kMaxH,
