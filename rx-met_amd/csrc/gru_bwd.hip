@@ -10,7 +10,10 @@
 // Here:
 //   1. prologue    : x, h_prev and W codes as bf16 operand planes for the weight-gradient
 //                    GEMMs (h codes recovered exactly from the dequantised h);
-//   2. recurrence  : both directions walk t = T-1..0 in one clustered launch
+//   2. recurrence  : up to H = 256 with 8-bit R one workgroup per two or four sequences with
+//                    all of R_q in its VGPRs (bwd_recurrence_res: dq as 31-bit fixed point
+//                    in four byte digits, dh += R_q dq on int8 MFMA, exact sums); else both
+//                    directions walk t = T-1..0 in one clustered launch
 //                    (bwd_recurrence_cl: a batch tile's hidden units split over a cluster of
 //                    workgroups, dq * scale_R exchanged through global memory each step and
 //                    dh += R_deq dq summed on bf16 MFMA, dq split exactly into three bf16
@@ -69,7 +72,7 @@ __global__ __launch_bounds__(64) void pack_rt_frags(int H, int KS2, const float 
     wd[q] = pack4_i8(by[0], by[1], by[2], by[3]);
   }
   frag[static_cast<size_t>(idx) * 64 + lane] = v4i{wd[0], wd[1], wd[2], wd[3]};
-  if (s == 0 && lane < 16 && k < H) {
+  if (rowsum != nullptr && s == 0 && lane < 16 && k < H) {
     int sum = 0;
     for (int c = 0; c < C; ++c) sum += static_cast<int>(Rq[static_cast<size_t>(k) * C + c]);
     rowsum[k] = static_cast<float>(sum);
@@ -656,6 +659,354 @@ __global__ __launch_bounds__(256 * UT) void bwd_recurrence_cl(BwdArgs a0, BwdArg
 }
 
 // ---------------------------------------------------------------------------------
+// 2a. resident backward recurrence (H <= 256, R_q of signed 8 bits)
+// ---------------------------------------------------------------------------------
+// One workgroup owns NS sequences and all H units and holds all of R_q in its VGPRs as int8 MFMA
+// operands, as the resident forward does; a step exchanges nothing with other workgroups.  Per
+// step a lane finishes the STE pointwise of one (sequence, unit), the gate gradients scaled by
+// R's channel scales become 31-bit fixed point on one exponent per sequence (the step's largest
+// magnitude, met through LDS), split into four signed byte digits, and dh += R_q dq runs on
+// v_mfma_i32_16x16x64_i8 with row 4 s + q = digit q of sequence s: the four digit sums of a
+// (sequence, unit) arrive in one lane's accumulator and are combined exactly in double.  Each
+// term is off by at most 2^-30 of the sequence's largest, and the sum itself is exact (the three
+// bf16 terms of the clustered form are exact, but accumulate in fp32): against 64-bit sums the
+// error of a whole step's gradients is no larger (training steps at H = 100 and 256: 2.8e-7 and
+// 4.8e-7 here, 2.9e-7 and 4.9e-7 clustered; the later fp32 weight products dominate).
+//
+// A digit must sit next to its neighbours' along K: a lane holds the four digits of one channel,
+// four lanes of a quad hold four consecutive channels, and two DPP exchanges transpose the 4 x 4
+// bytes so that each lane writes one aligned word of one digit row.
+//
+// Measured (both directions of B = 256, T = 200, H = 256, saved codes): 1021 us clustered ->
+// 345 us.  Bound: the chain of one step (two LDS exchanges, 24 MFMA per wave, about 200 VALU).
+constexpr unsigned kResSkip = 0x80000000u;  // an offset past every buffer: the store is dropped
+constexpr int kResMaxH = 256;
+
+constexpr size_t bwd_res_lds(int ks2, int ns) {
+  return 256 + static_cast<size_t>(4) * ns * (64 * ks2 + 16);
+}
+
+// All of the workgroup's LDS accesses are complete; memory accesses stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Largest of the 16 lanes of a row, in every lane of it.
+__device__ __forceinline__ unsigned row16_max(unsigned v) {
+  const int i0 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xf, 0xf, true);  // lane ^ 1
+  v = max(v, static_cast<unsigned>(i0));
+  const int i1 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xf, 0xf, true);  // lane ^ 2
+  v = max(v, static_cast<unsigned>(i1));
+  const int i2 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x141, 0xf, 0xf, true);  // half mirror
+  v = max(v, static_cast<unsigned>(i2));
+  const int i3 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x140, 0xf, 0xf, true);  // mirror
+  return max(v, static_cast<unsigned>(i3));
+}
+
+// Byte i of the four lanes of a quad, to lane i of the quad (its byte k from lane k); s1, s2: the
+// lane's selectors (odd lanes, upper pairs).
+__device__ __forceinline__ unsigned quad_transpose(unsigned v, unsigned s1, unsigned s2) {
+  const unsigned x = static_cast<unsigned>(
+      __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xf, 0xf, true));
+  v = __builtin_amdgcn_perm(x, v, s1);
+  const unsigned y = static_cast<unsigned>(
+      __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xf, 0xf, true));
+  return __builtin_amdgcn_perm(y, v, s2);
+}
+
+// One element's step inputs as they are in memory.
+template <bool CODES>
+struct BwdRaw {
+  float g, h;
+  float v[CODES ? 1 : 4];
+  unsigned c[CODES ? 5 : 13];  // v codes and mask bits, or the 13 mask bytes
+};
+
+// The element's STE pointwise: bwd_point's operations in its order, the 0 / 1 masks that meet on
+// one value combined before the product.
+template <bool CODES>
+__device__ __forceinline__ float bwd_point_raw(const BwdRaw<CODES> &r, const BwdArgs &a, float dhc,
+                                               float (&dpv)[3], float (&dqv)[3]) {
+  float z, rr, g, qg;
+  unsigned bits;
+  if constexpr (CODES) {
+    z = (static_cast<float>(r.c[0]) - a.vzl[0]) * a.veff[0];
+    rr = (static_cast<float>(r.c[1]) - a.vzl[1]) * a.veff[1];
+    g = (static_cast<float>(r.c[2]) - a.vzl[2]) * a.veff[2];
+    qg = (static_cast<float>(r.c[3]) - a.vzl[3]) * a.veff[3];
+    bits = r.c[4];
+  } else {
+    z = r.v[0]; rr = r.v[1]; g = r.v[2]; qg = r.v[3];
+    // the order of the saved mask bits: ih 0-2, hh 3-5, gate in 6-8, gate out 9-11, h 12
+    bits = 0;
+#pragma unroll
+    for (int k = 0; k < 13; ++k) bits |= (r.c[k] & 1u) << k;
+  }
+  const unsigned gm = (bits >> 6) & (bits >> 9);  // gate in and gate out
+  const unsigned mp = gm & bits, mq = gm & (bits >> 3);
+  auto bit = [](unsigned w, int k) { return static_cast<float>((w >> k) & 1u); };
+  const float dht = (r.g + dhc) * bit(bits, 12);
+  const float dg = (1.0f - z) * dht;
+  const float dz = (r.h - g) * dht;
+  const float dpg = (1.0f - g * g) * dg * bit(gm, 2);
+  const float dqg = dpg * rr;
+  const float dr = dpg * qg;
+  const float dpr = rr * (1.0f - rr) * dr;
+  const float dpz = z * (1.0f - z) * dz;
+  dpv[0] = dpz * bit(mp, 0); dpv[1] = dpr * bit(mp, 1); dpv[2] = dpg * bit(bits, 2);
+  dqv[0] = dpz * bit(mq, 0); dqv[1] = dpr * bit(mq, 1); dqv[2] = dqg * bit(bits, 5);
+  return z * dht;
+}
+
+template <int KS2, int UPW, int NS, bool CODES>
+__global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1, int nblk) {
+  constexpr bool kMerge = UPW == 2 && NS == 2;  // two tiles' sums share one pass of the lanes
+  constexpr int NP = UPW == 2 && !kMerge ? 2 : 1;
+  constexpr int ROW = 64 * KS2 + 16;
+  extern __shared__ __align__(16) unsigned char smem[];
+  unsigned *smax = reinterpret_cast<unsigned *>(smem);  // [NS][8]: a wave's largest per sequence
+  int8_t *pl = reinterpret_cast<int8_t *>(smem + 256);  // [4 NS][ROW] digit rows
+  const int dir = blockIdx.x / nblk, blk = blockIdx.x % nblk;
+  const BwdArgs &a = dir == 0 ? a0 : a1;
+  const int H = a.H, C = 3 * H, B = a.B, T = a.T, UT = H / 16;
+  const int tid = threadIdx.x, w = tid / 64, l = tid % 64, grp = l / 16, e = l % 16;
+
+  for (int i = tid; i < NS * ROW; i += blockDim.x) reinterpret_cast<int *>(pl)[i] = 0;
+  if (tid < NS * 8) smax[tid] = 0u;
+
+  v4i rfr[UPW][KS2];
+#pragma unroll
+  for (int u = 0; u < UPW; ++u)
+#pragma unroll
+    for (int s = 0; s < KS2; ++s) {
+      const int ut = UPW * w + u;
+      rfr[u][s] = ut < UT && s < a.KS2 ? a.rfrag[(static_cast<size_t>(ut) * a.KS2 + s) * 64 + l]
+                                       : v4i{0, 0, 0, 0};
+    }
+
+  // the elements this lane finishes: pass k, (sequence b, unit j)
+  const int seq = kMerge ? grp % 2 : grp;
+  const int b = NS * blk + seq, bc = b < B ? b : B - 1;  // loads of absent rows repeat the last
+  float dhc[NP], effr[NP][3];
+  double sbw[NP][3], sbr[NP][3];
+  unsigned od[NP], ol[NP], oc[NP], om[NP];  // dp / dq stores; h, v codes (or v), mask loads
+  const float *gp[NP];
+  int8_t *pw[NP];
+  bool own[NP], ok[NP];
+  const float *gbase = a.gv_on ? (a.gv ? a.gv : a.h) : a.dh_new + static_cast<size_t>(B) * H;
+  const int64_t gst = a.gv_on ? (a.gv ? a.gv_t : 0) : static_cast<int64_t>(B) * H;
+  const bool rev = a.gv_on && a.gv_rev, nog = a.gv_on && a.gv == nullptr;
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    const int ut = UPW * w + (kMerge ? grp / 2 : k), j = 16 * ut + e, jc = ut < UT ? j : 0;
+    own[k] = seq < NS && ut < UT;
+    ok[k] = own[k] && b < B;
+    const unsigned row = static_cast<unsigned>(bc) * H + jc;
+    od[k] = ok[k] ? 4u * (static_cast<unsigned>(b) * C + j) : kResSkip;
+    ol[k] = 4u * row;
+    if (CODES) {
+      const unsigned cr = (static_cast<unsigned>(bc / 16) * (H / 16) + jc / 16) * 16 + bc % 16;
+      oc[k] = 128u * cr + 2u * e;
+      om[k] = 32u * cr + 2u * e;
+    } else {
+      oc[k] = 4u * (4u * static_cast<unsigned>(bc) * H + jc);
+      om[k] = static_cast<unsigned>(bc) * C + jc;
+    }
+    gp[k] = gbase + (a.gv_on ? (a.gv ? bc * a.gv_b + (a.gv_col0 + jc) * a.gv_k : 0)
+                             : static_cast<int64_t>(row));
+    dhc[k] = a.gv_on && a.gv_hn && ok[k] ? a.gv_hn[row] : 0.0f;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      effr[k][g] = a.eff_r[g * H + jc];
+      sbw[k][g] = sbr[k][g] = 0.0;
+    }
+    // this lane writes digit row 4 seq + e % 4, channels of the quad's four units
+    pw[k] = pl + (own[k] ? (4 * seq + e % 4) * ROW + 16 * ut + (e & ~3) : 0);
+  }
+  const unsigned sel1 = e & 1 ? 0x03070105u : 0x06020400u;
+  const unsigned sel2 = e & 2 ? 0x03020706u : 0x05040100u;
+  // A operand: row l % 16 = 4 s + q (rows without a sequence repeat one that exists)
+  const int8_t *ar = pl + (e % (4 * NS)) * ROW + 16 * grp;
+
+  const unsigned step_c = 4u * static_cast<unsigned>(B) * C, step_h = 4u * static_cast<unsigned>(B) * H;
+  const unsigned step_blk = static_cast<unsigned>((B + 15) / 16) * H;  // x 128 B of v codes, x 32 B
+  const unsigned step_m = static_cast<unsigned>(B) * C;
+  auto load = [&](int t, BwdRaw<CODES> (&r)[NP]) {
+    const size_t tt = static_cast<size_t>(t > 0 ? t : 0);
+    const int64_t go = (rev ? T - 1 - static_cast<int64_t>(tt) : static_cast<int64_t>(tt)) * gst;
+    const auto rh = cluster::buffer_rsrc(a.h + tt * B * H, step_h);
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      r[k].g = gp[k][go];
+      r[k].h = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rh, ol[k], 0, 0));
+    }
+    if constexpr (CODES) {
+      const auto rc = cluster::buffer_rsrc(a.vc + tt * step_blk * 64, step_blk * 128);
+      const auto rm = cluster::buffer_rsrc(a.mb + tt * step_blk * 16, step_blk * 32);
+#pragma unroll
+      for (int k = 0; k < NP; ++k) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          r[k].c[q] = static_cast<unsigned short>(
+              __builtin_amdgcn_raw_buffer_load_b16(rc, oc[k] + 32u * q, 0, 0));
+        r[k].c[4] = static_cast<unsigned short>(__builtin_amdgcn_raw_buffer_load_b16(rm, om[k], 0, 0));
+      }
+    } else {
+      const auto rv = cluster::buffer_rsrc(a.v + 4 * tt * B * H, 4u * step_h);
+      // an absent mask reads v's bytes (its buffer is larger) and counts as ones
+      auto masks = [&](const uint8_t *m, unsigned bytes) {
+        return cluster::buffer_rsrc(m ? m + tt * bytes : reinterpret_cast<const uint8_t *>(a.v), bytes);
+      };
+      const auto r0 = masks(a.ih_m, step_m), r1 = masks(a.hh_m, step_m), r2 = masks(a.gin_m, step_m),
+                 r3 = masks(a.gout_m, step_m), r4 = masks(a.h_m, step_h / 4);
+#pragma unroll
+      for (int k = 0; k < NP; ++k) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          r[k].v[q] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(rv, oc[k] + 4u * q * H, 0, 0));
+#pragma unroll
+        for (int g = 0; g < 3; ++g) {
+          r[k].c[g] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r0, om[k] + g * H, 0, 0));
+          r[k].c[3 + g] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r1, om[k] + g * H, 0, 0));
+          r[k].c[6 + g] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r2, om[k] + g * H, 0, 0));
+          r[k].c[9 + g] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r3, om[k] + g * H, 0, 0));
+        }
+        r[k].c[12] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r4, ol[k] / 4, 0, 0));
+      }
+    }
+  };
+  // masks that are absent, as ones over the loaded bytes
+  const unsigned ones = CODES ? 0u : (a.ih_m ? 0u : 1u) | (a.hh_m ? 0u : 2u) | (a.gin_m ? 0u : 4u) |
+                                         (a.gout_m ? 0u : 8u) | (a.h_m ? 0u : 16u);
+
+  auto step = [&](int t, BwdRaw<CODES> (&r)[NP]) {
+    float dpv[NP][3], dqv[NP][3], dhl[NP], sv[NP][3];
+    unsigned mx = 0u;
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      if (nog) r[k].g = 0.0f;
+      if constexpr (!CODES) {
+#pragma unroll
+        for (int q = 0; q < 12; ++q) r[k].c[q] |= (ones >> (q / 3)) & 1u;
+        r[k].c[12] |= ones >> 4;
+      }
+      dhl[k] = bwd_point_raw<CODES>(r[k], a, dhc[k], dpv[k], dqv[k]);
+#pragma unroll
+      for (int g = 0; g < 3; ++g) {
+        sbw[k][g] += static_cast<double>(dpv[k][g]);
+        sbr[k][g] += static_cast<double>(dqv[k][g]);
+        sv[k][g] = dqv[k][g] * effr[k][g];
+        // magnitudes as integers: a NaN is the largest
+        const unsigned m = __builtin_bit_cast(unsigned, sv[k][g]) & 0x7fffffffu;
+        if (own[k]) mx = max(mx, m);
+      }
+    }
+    mx = row16_max(mx);
+    if constexpr (kMerge) {
+      const auto sw = __builtin_amdgcn_permlane32_swap(mx, mx, false, false);
+      mx = max(sw[0], sw[1]);
+    }
+    if (e == 0 && (kMerge ? grp < 2 : grp < NS)) smax[seq * 8 + w] = mx;
+    lds_barrier();
+    load(t - 2, r);
+    {
+      const size_t tt = static_cast<size_t>(t);
+      const auto rp = cluster::buffer_rsrc(a.dp + tt * B * C, step_c);
+      const auto rq = cluster::buffer_rsrc(a.dq + tt * B * C, step_c);
+#pragma unroll
+      for (int k = 0; k < NP; ++k)
+#pragma unroll
+        for (int g = 0; g < 3; ++g) {
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dpv[k][g]), rp,
+                                                od[k] + 4u * g * H, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dqv[k][g]), rq,
+                                                od[k] + 4u * g * H, 0, 0);
+        }
+    }
+    const uint4 m0 = *reinterpret_cast<const uint4 *>(smax + (seq < NS ? seq : 0) * 8);
+    const uint4 m1 = *reinterpret_cast<const uint4 *>(smax + (seq < NS ? seq : 0) * 8 + 4);
+    const unsigned top = max(max(max(m0.x, m0.y), max(m0.z, m0.w)), max(max(m1.x, m1.y), max(m1.z, m1.w)));
+    // the largest is below 2^(ex - 126): scaled by 2^ex2 everything is below 2^30
+    const int ex2 = 156 - static_cast<int>(top >> 23);
+    const bool bad = top >= 0x7f800000u;
+#pragma unroll
+    for (int k = 0; k < NP; ++k)
+#pragma unroll
+      for (int g = 0; g < 3; ++g) {
+        const int q = bad ? 0 : static_cast<int>(rintf(ldexpf(sv[k][g], ex2)));
+        // four signed digits: adding 128 to the three low bytes carries into the next, and
+        // flipping their top bits subtracts it again
+        const unsigned dg = (static_cast<unsigned>(q) + 0x00808080u) ^ 0x00808080u;
+        const unsigned tr = quad_transpose(dg, sel1, sel2);
+        if (own[k]) *reinterpret_cast<unsigned *>(pw[k] + g * H) = tr;
+      }
+    lds_barrier();
+    v4i acc[UPW];
+#pragma unroll
+    for (int u = 0; u < UPW; ++u) acc[u] = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < KS2; ++s) {
+      const v4i af = *reinterpret_cast<const v4i *>(ar + 64 * s);
+#pragma unroll
+      for (int u = 0; u < UPW; ++u) acc[u] = mfma_i8(af, rfr[u][s], acc[u]);
+    }
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      int sum[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        sum[q] = acc[k][q];
+        if constexpr (kMerge)
+          sum[q] = __builtin_amdgcn_permlane32_swap(acc[0][q], acc[UPW - 1][q], false, false)[0];
+      }
+      // |sum| < 2^24, so the low pair and the high pair are exact in int32, the whole in double
+      const double s = 65536.0 * static_cast<double>(256LL * sum[3] + sum[2]) +
+                       static_cast<double>(256LL * sum[1] + sum[0]);
+      const float add = bad ? NAN : static_cast<float>(ldexp(s, -ex2));
+      dhc[k] = dhl[k] + add;
+    }
+  };
+  BwdRaw<CODES> ra[NP], rb[NP];
+  load(T - 1, ra);
+  load(T - 2, rb);
+  lds_barrier();  // the zeroed rows are in LDS
+  for (int t = T - 1;;) {
+    step(t, ra);
+    if (--t < 0) break;
+    step(t, rb);
+    if (--t < 0) break;
+  }
+
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    if (ok[k]) {
+      const unsigned o = ol[k] / 4;
+      a.dh0[o] = a.h0_m ? dhc[k] * static_cast<float>(a.h0_m[o]) : dhc[k];
+    }
+    // bias partials of the workgroup's sequences, in lane order
+    const int ut = UPW * w + (kMerge ? grp / 2 : k), j = 16 * ut + e;
+    double *p = a.bias_partial + static_cast<size_t>(blk) * 2 * C;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      double x = ok[k] ? sbw[k][g] : 0.0, y = ok[k] ? sbr[k][g] : 0.0;
+      x += __shfl_xor(x, 16, 64);
+      y += __shfl_xor(y, 16, 64);
+      if (!kMerge) {
+        x += __shfl_xor(x, 32, 64);
+        y += __shfl_xor(y, 32, 64);
+      }
+      if (ut < UT && (kMerge ? grp % 2 == 0 : grp == 0)) {
+        const double mw = a.bw_m ? static_cast<double>(a.bw_m[g * H + j]) : 1.0;
+        const double mr = a.br_m ? static_cast<double>(a.br_m[g * H + j]) : 1.0;
+        p[g * H + j] = x * mw;
+        p[C + g * H + j] = y * mr;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------
 // stepped backward (H > 256): per step one pointwise launch and one dh GEMM launch
 // ---------------------------------------------------------------------------------
 // Step t: every (sequence, unit) takes dh_c = dhl + gsum of step t + 1 (zero at t = T - 1),
@@ -742,18 +1093,31 @@ __global__ __launch_bounds__(256) void zero_floats(int64_t n, float *p) {
 }
 
 
-// swap_h > 0: written in the (r, z, n) gate order (the first two blocks of swap_h swapped).
+// Bias gradients: the partials of the nwg workgroups (or 16-row chunks) summed in a fixed order,
+// 16 interleaved chains per channel: 128 partials of the resident recurrence take 5.5 us (one
+// chain over the clustered form's 16 took 7.6).  swap_h > 0: written in the (r, z, n) gate order (the first two blocks of swap_h
+// swapped).
 __global__ __launch_bounds__(256) void fold_bias(int nwg, int C, const double *__restrict__ part,
                                                  float *__restrict__ dbw, float *__restrict__ dbr,
                                                  int swap_h) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= C) return;
-  const int co = swap_h > 0 ? (c < swap_h ? c + swap_h : (c < 2 * swap_h ? c - swap_h : c)) : c;
+  __shared__ double red[16][16][2];
+  const int lc = threadIdx.x % 16, ch = threadIdx.x / 16;
+  const int c = blockIdx.x * 16 + lc;
   double x = 0.0, y = 0.0;
-  for (int k = 0; k < nwg; ++k) {
-    x += part[static_cast<size_t>(k) * 2 * C + c];
-    y += part[static_cast<size_t>(k) * 2 * C + C + c];
+  if (c < C)
+    for (int k = ch; k < nwg; k += 16) {
+      x += part[static_cast<size_t>(k) * 2 * C + c];
+      y += part[static_cast<size_t>(k) * 2 * C + C + c];
+    }
+  red[ch][lc][0] = x;
+  red[ch][lc][1] = y;
+  __syncthreads();
+  if (ch != 0 || c >= C) return;
+  for (int k = 1; k < 16; ++k) {
+    x += red[k][lc][0];
+    y += red[k][lc][1];
   }
+  const int co = swap_h > 0 ? (c < swap_h ? c + swap_h : (c < 2 * swap_h ? c - swap_h : c)) : c;
   dbw[co] = static_cast<float>(x);
   dbr[co] = static_cast<float>(y);
 }
@@ -807,7 +1171,8 @@ struct BwdWorkspace {
     o += al(sizeof(float) * (2 * C + I + H));
     rfrag = o; o += al(sizeof(v4i) * 64 * ((H + 15) / 16) * KS2);
     rowsum = o; o += al(sizeof(float) * H);
-    bias = o; o += al(sizeof(double) * 2 * C * nwg);
+    // one partial per 16 sequences, or per two in the resident recurrence
+    bias = o; o += al(sizeof(double) * 2 * C * (H <= kResMaxH ? (static_cast<size_t>(B) + 1) / 2 : nwg));
     for (int np = 0; np < 2; ++np)
       wgrad::tn_plan(static_cast<int>(M), static_cast<int>(C), I, np + 1, &S_w[np], &kper_w[np]);
     for (int np = 0; np < 2; ++np)
@@ -837,6 +1202,7 @@ struct BwdPlan {
   char *wsb;
   int npx, nph, npw;  // bf16 planes of the x, h and W codes
   bool torch_layout;  // dW, dR, dbw, dbr in PyTorch's layout and (r, z, n) gate order
+  int nbias;          // bias partials the recurrence left
 };
 
 static int backward_prologue(int T, int B, int I, int H, const rxmet_gru_bwd_dir &d,
@@ -946,7 +1312,56 @@ static int backward_prologue(int T, int B, int I, int H, const rxmet_gru_bwd_dir
   ba.rt = reinterpret_cast<uint4 *>(wsb + ws.rt);
   plan->d = &d;
   plan->wsb = wsb;
+  plan->nbias = (B + kBTile - 1) / kBTile;
   return 0;
+}
+
+template <int NS, bool CODES>
+static const void *bwd_res_kernel(int ks2) {
+  if (ks2 <= 3) return reinterpret_cast<const void *>(&bwd_recurrence_res<3, 1, NS, CODES>);
+  if (ks2 <= 6) return reinterpret_cast<const void *>(&bwd_recurrence_res<6, 1, NS, CODES>);
+  // four sequences in the float format would need more than the 256 VGPRs of a wave
+  return reinterpret_cast<const void *>(&bwd_recurrence_res<12, 2, (CODES ? NS : 2), CODES>);
+}
+
+// Resident recurrence of every direction in one ordinary launch; returns 1 when launched, 0 when
+// the caller takes another form.  Two sequences per workgroup while every workgroup then has a CU
+// of its own, else four, as in the forward.  A forced poll limit (the timeout tests) asks for the
+// clustered form.
+static int backward_recurrence_resident(BwdPlan *plans, int ndir, int T, int B, int I, int H,
+                                        hipStream_t stream) {
+  const int KS2 = (3 * H + 63) / 64;
+  if (H > kResMaxH || std::getenv("RXMET_NO_CLUSTER") != nullptr ||
+      cluster::spin_limit() != cluster::kSpinLimit)
+    return 0;
+  for (int k = 0; k < ndir; ++k) {
+    const rxmet_gru_qparams *q = plans[k].d->params;
+    if (q->chan_bits[RXMET_GRU_R] > 8 || q->chan_unsigned[RXMET_GRU_R] != 0) return 0;
+  }
+  // one step's rows are addressed with 31-bit byte offsets (v: 16 bytes per element)
+  if (16.0 * ((B + kBTile - 1) / kBTile * kBTile) * H >= 2147483648.0) return 0;
+  int device = 0, ncu = 0;
+  RXMET_CHECK_HIP(hipGetDevice(&device));
+  RXMET_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
+  const bool codes = plans[0].ba.vc != nullptr;
+  const int ns = static_cast<int64_t>(ndir) * ((B + 1) / 2) <= ncu || (!codes && KS2 > 6) ? 2 : 4;
+  int nblk = (B + ns - 1) / ns;
+  for (int k = 0; k < ndir; ++k) {
+    plans[k].nbias = nblk;
+    hipLaunchKernelGGL(pack_rt_frags, dim3((H / 16) * KS2), dim3(64), 0, stream, H, KS2,
+                       plans[k].d->R_q, const_cast<v4i *>(plans[k].ba.rfrag),
+                       static_cast<float *>(nullptr));
+    RXMET_CHECK_LAUNCH();
+  }
+  const void *fn = ns == 2 ? (codes ? bwd_res_kernel<2, true>(KS2) : bwd_res_kernel<2, false>(KS2))
+                           : (codes ? bwd_res_kernel<4, true>(KS2) : bwd_res_kernel<4, false>(KS2));
+  const int ks = KS2 <= 3 ? 3 : (KS2 <= 6 ? 6 : 12), upw = ks == 12 ? 2 : 1;
+  const int waves = (H / 16 + upw - 1) / upw;
+  void *args[] = {&plans[0].ba, &plans[ndir > 1 ? 1 : 0].ba, &nblk};
+  rxmet::prof::Scope ps__("gru_bwd_recurrence", stream);
+  RXMET_CHECK_HIP(hipLaunchKernel(fn, dim3(ndir * nblk), dim3(64 * waves), args,
+                                  bwd_res_lds(ks, ns), stream));
+  return 1;
 }
 
 // Clustered recurrence over every direction; 1 when launched, 0 when the caller must use the
@@ -1088,9 +1503,8 @@ static int backward_epilogue(int T, int B, int I, int H, BwdPlan &plan, hipStrea
   const rxmet_gru_bwd_dir &d = *plan.d;
   const int C = 3 * H;
   const BwdWorkspace ws(T, B, I, H);
-  const int nwg = (B + kBTile - 1) / kBTile;
   const int swap_h = plan.torch_layout ? H : 0;
-  hipLaunchKernelGGL(fold_bias, dim3((C + 255) / 256), dim3(256), 0, stream, nwg, C,
+  hipLaunchKernelGGL(fold_bias, dim3((C + 15) / 16), dim3(256), 0, stream, plan.nbias, C,
                      plan.ba.bias_partial, d.dbw, d.dbr, swap_h);
   RXMET_CHECK_LAUNCH();
   const int M = T * B;
@@ -1170,9 +1584,9 @@ static int backward_dirs(int ndir, int T, int B, int I, int H, const rxmet_gru_b
   // RXMET_BWD_STEPPED set: one pointwise and one GEMM launch per step
   const bool stepped = H > 256 || std::getenv("RXMET_BWD_STEPPED") != nullptr;
   int *timeout_flag = nullptr;
-  const int rc = stepped ? 0
-                         : backward_recurrence_clustered(plans, ndir, T, B, I, H, stream,
-                                                         &timeout_flag);
+  int rc = stepped ? 0 : backward_recurrence_resident(plans, ndir, T, B, I, H, stream);
+  if (rc == 0 && !stepped)
+    rc = backward_recurrence_clustered(plans, ndir, T, B, I, H, stream, &timeout_flag);
   if (rc < 0) return rc;
   // the per-tile recurrence holds R as int8 fragments: wider recurrent weights step instead
   bool wide_r = false;

@@ -55,3 +55,57 @@ def test_resident_forward_matches_oracle_and_clustered(cuda, case, monkeypatch):
             u, v = (np.ascontiguousarray(gru_ops.unblock_codes(o[k].cpu().numpy(), B, H, f))
                     for o in (a, b))
             np.testing.assert_array_equal(u, v)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_resident_backward_matches_oracle_and_clustered(cuda, case, monkeypatch):
+    """Gradients within 1e-5 of the oracle's 64-bit sums, relative to each tensor's norm (32-bit
+    sums over at most 3 H and T B terms: a few 1e-7 expected), in both saved formats; the two
+    formats agree bit for bit, and the clustered form to the same bound."""
+    T, B, I, H, cfg = case
+    print(f"[gru resident bwd] {case}", flush=True)
+    args = _dirs(cuda, case)
+    ref = gru_ops.forward_quant_float_storage_dirs(True, T, B, I, H, args)
+    cod = gru_ops.forward_quant_codes_dirs(True, T, B, I, H, args)
+    g = np.random.default_rng(5)
+    dh = [torch.from_numpy((g.standard_normal((T + 1, B, H)) * 1e-2).astype(np.float32)).to(cuda)
+          for _ in range(2)]
+    pack = lambda outs: [(o[2], o[3], o[4], o[5], o[6], dh[d], o[0], o[1], args[d][6], o[7:])
+                         for d, o in enumerate(outs)]
+    f = gru_ops.backward_quant_float_storage_dirs(T, B, I, H, pack(ref))
+    c = gru_ops.backward_quant_codes_dirs(T, B, I, H, pack(cod), torch_layout=False)
+    monkeypatch.setenv("RXMET_TEST_SPIN_LIMIT", OTHER_LIMIT)
+    k = gru_ops.backward_quant_codes_dirs(T, B, I, H, pack(cod), torch_layout=False)
+    torch.cuda.synchronize()
+    for d in range(2):
+        W, R, bw, br, x, h0, qp = _case(T, B, I, H, cfg, 31 + d, d == 1)
+        fwd = GO.forward_quant(W, R, bw, br, x, qp, h0=h0, training=True)
+        exp = GO.backward_quant(fwd, dh[d].cpu().numpy(), qp)
+        for n, a, b, q in zip(("dx", "dW", "dR", "dbw", "dbr", "dh0"), f[d], c[d], k[d]):
+            assert torch.equal(a, b), (d, n)
+            e = np.asarray(exp[n], np.float64)
+            scale = np.linalg.norm(e) + 1e-30
+            assert np.linalg.norm(b.cpu().numpy() - e) <= 1e-5 * scale, (d, n)
+            assert np.linalg.norm(q.cpu().numpy() - e) <= 1e-5 * scale, (d, n)
+
+
+def test_resident_backward_keeps_nan_in_its_sequence(cuda):
+    """A NaN and an infinity in two sequences' output gradients reach every unit's dh0 and the
+    weight gradients, and leave the other sequences' dx and dh0 as they are without them."""
+    case = (4, 5, 3, 64, "c3")
+    T, B, I, H, _ = case
+    args = _dirs(cuda, case)[:1]
+    o = gru_ops.forward_quant_codes_dirs(True, T, B, I, H, args)[0]
+    res = []
+    for bad in (False, True):
+        dh = torch.full((T + 1, B, H), 1e-2, device=cuda)
+        if bad:
+            dh[2, 1, 7], dh[3, 2, 9] = float("nan"), float("inf")
+        res.append(gru_ops.backward_quant_codes_dirs(
+            T, B, I, H, [(o[2], o[3], o[4], o[5], o[6], dh, o[0], o[1], args[0][6], o[7:])],
+            torch_layout=False)[0])
+    torch.cuda.synchronize()
+    (dx0, _, _, _, _, h00), (dx1, dW1, _, _, _, h01) = res
+    keep = [0, 3, 4]
+    assert torch.equal(dx0[:, keep], dx1[:, keep]) and torch.equal(h00[keep], h01[keep])
+    assert torch.isnan(h01[1]).all() and torch.isnan(h01[2]).all() and torch.isnan(dW1).any()
