@@ -15,18 +15,22 @@
 //   4. lstm_input_gemm    : the input linear of all T steps as an exact integer GEMM with
 //      the whole input branch fused in its epilogue (bias, rescale, clamp + mask, and the
 //      rescale to each gate-input grid), so the recurrence only adds the recurrent branch;
-//   5. lstm_recurrence_cl : (H a multiple of 64) a cluster of H/64 workgroups per 16-sequence
+//   5. lstm_recurrence_res : (W_hh of 8 bits, H up to 512, activations as tables) W_hh in the
+//      registers of one workgroup, or of a cluster of up to four above H = 256
+//      (lstm_resident.h);
+//   5'. lstm_recurrence_cl : otherwise (H a multiple of 64; W_hh up to 16 bits) a cluster of H/64 workgroups per 16-sequence
 //      batch tile in one cooperative launch.  Each member keeps the W_hh fragments of its 64
 //      units resident in LDS, computes the recurrent linear on v_mfma_i32_16x16x64_i8, the
 //      gates through precomputed activation tables (exact: the activation is a function of
 //      the integer gate-input code), the cell and hidden update, every clamp mask and the
 //      checkpoints; the new h codes are exchanged through global memory and the members meet
 //      at a counter barrier once per step (cluster.h);
-//   5'. lstm_recurrence   : otherwise, one persistent workgroup per 16 sequences walks the T
+//   5''. lstm_recurrence  : otherwise, one persistent workgroup per 16 sequences walks the T
 //      steps with h in LDS and W_hh fragments streamed from L2.
 //
 // Activations: sigmoid keeps the reference's float op order around exp, with exp and tanh
 // evaluated in double and rounded once to float.
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -1187,6 +1191,14 @@ __global__ __launch_bounds__(256) void lstm_poison_on_timeout(const int *timeout
   }
 }
 
+}  // namespace lstm
+}  // namespace rxmet
+
+#include "lstm_resident.h"
+
+namespace rxmet {
+namespace lstm {
+
 size_t recurrence_lds(int H, int KS, int npl) {
   return sizeof(float4) * 4 * static_cast<size_t>(H) + sizeof(float) * kBT * static_cast<size_t>(H) +
          static_cast<size_t>(2) * npl * kBT * (KS * 64 + 16);
@@ -1214,7 +1226,7 @@ struct FwdWorkspace {
     // clustered recurrence: h exchange planes (two parities, up to two planes) and counters
     const size_t Bpad = (static_cast<size_t>(B) + 15) / 16 * 16;
     hx = o; o += al(2 * 2 * Bpad * H);
-    sync = o; o += al(sizeof(unsigned) * cluster::kCounterStride * (Bpad / 16 + 1));
+    sync = o; o += al(sizeof(unsigned) * cluster::kCounterStride * (Bpad / kLresTile + 1));
     lut = o; o += al(sizeof(uint32_t) * 2 * kLutMaxEntries);
     glut = o; o += al(sizeof(uint32_t) * 5 * static_cast<size_t>(kGlobalLutMaxCodes));
     // reference activation exceptions: keys, then entries, of at most 5 full 16-bit grids
@@ -1232,6 +1244,166 @@ struct FwdWorkspace {
     total = o;
   }
 };
+
+// The gate and tanh tables of lut (LDS-sized ones from lut_table, the others from gtab) built on
+// the stream, the reference's exception codes included.
+static int build_act_tables(const StepParams &sp, const ActLut &lut, uint32_t *lut_table,
+                            uint32_t *gtab, int n_exc, hipStream_t stream) {
+  ActLut gl{};
+  for (int g = 0; g < 4; ++g) {
+    gl.off[g] = lut.goff[g];
+    gl.n[g] = lut.gn[g];
+  }
+  gl.tanh_off = lut.gtanh_off;
+  gl.tanh_n = lut.gtanh_n;
+  gl.total = lut.gtotal;
+  const ActLut *l[2] = {&lut, &gl};
+  uint32_t *t[2] = {lut_table, gtab};
+  for (int k = 0; k < 2; ++k) {
+    if (l[k]->total == 0) continue;
+    hipLaunchKernelGGL(lstm_build_act_lut, dim3((l[k]->total + 255) / 256), dim3(256), 0, stream, sp,
+                       *l[k], t[k]);
+    RXMET_CHECK_LAUNCH();
+    if (n_exc > 0) {
+      hipLaunchKernelGGL(lstm_act_lut_exceptions, dim3((n_exc + 255) / 256), dim3(256), 0, stream, sp,
+                         *l[k], t[k]);
+      RXMET_CHECK_LAUNCH();
+    }
+  }
+  return 0;
+}
+
+// Resident recurrence (lstm_resident.h) for W_hh of 8 bits, H <= 512 and grids whose activations
+// are tables (at most 2^16 codes); 1 when launched, 0 when another form takes the call.  Up to
+// H = 256: two sequences per workgroup while every workgroup then has a CU of its own, else
+// four.  Above: clusters of ceil(H / 128) workgroups on eight sequences.  A forced poll limit
+// (the timeout tests) asks for the clustered form up to H = 256, where this one never polls.
+static int lstm_res_launch(const RecArgs &ra, const StepParams &sp, int npl, int n_exc,
+                           const FwdWorkspace &ws, char *wsb, hipStream_t stream) {
+  const int H = ra.H, B = ra.B;
+  if (H > kMaxH || std::getenv("RXMET_NO_CLUSTER") != nullptr ||
+      (H <= 256 && cluster::spin_limit() != cluster::kSpinLimit) || sp.cell_fp[0] || sp.cell_fp[1])
+    return 0;
+  // one step's rows are addressed with 31-bit byte offsets (gates: 16 bytes per unit)
+  if (16.0 * ((B + 15) / 16 * 16) * H >= 2147483648.0) return 0;
+  int64_t n[4], tot = 0;
+  for (int g = 0; g < 4; ++g) {
+    n[g] = static_cast<int64_t>(sp.gin[g].hi) - sp.gin[g].lo + 1;
+    if (n[g] > kGlobalLutMaxCodes) return 0;
+    tot += n[g];
+  }
+  const int64_t nc = static_cast<int64_t>(sp.c.hi) - sp.c.lo + 1;
+  if (nc > kGlobalLutMaxCodes) return 0;
+  LresParams p{};
+  int tab = kTabLds;
+  ActLut lut{};
+  uint32_t *lut_table = reinterpret_cast<uint32_t *>(wsb + ws.lut);
+  uint32_t *gtab = reinterpret_cast<uint32_t *>(wsb + ws.glut);
+  const bool lds_gates = tot <= kLutMaxEntries;
+  for (int g = 0, o = 0; g < 4; ++g) {
+    (lds_gates ? lut.off : lut.goff)[g] = o;
+    (lds_gates ? lut.n : lut.gn)[g] = static_cast<int>(n[g]);
+    o += static_cast<int>(n[g]);
+  }
+  (lds_gates ? lut.total : lut.gtotal) = static_cast<int>(tot);
+  if (lds_gates && tot + nc <= kLutMaxEntries) {
+    tab = kTabLds;
+    lut.tanh_off = lut.total;
+    lut.tanh_n = static_cast<int>(nc);
+    lut.total += lut.tanh_n;
+  } else {
+    // 16-bit entries (output code and mask) when the output grid leaves room for the mask bit
+    tab = !lds_gates ? kTabGlobal
+          : sp.tanh_c.hi - sp.tanh_c.lo < (1 << 15) ? kTabLds16 : kTabGlobalTanh;
+    lut.gtanh_off = lut.gtotal;
+    lut.gtanh_n = static_cast<int>(nc);
+    lut.gtotal += lut.gtanh_n;
+  }
+  p.tanh_n = static_cast<int>(nc);
+  p.lds_gates = lut.total;
+  p.lds_src = lut_table;
+  p.gate_tab = gtab;
+  p.tanh_tab = gtab + lut.gtanh_off;
+  for (int g = 0; g < 4; ++g) {
+    LresGate &q = p.g[g];
+    q.h2g_mult = sp.hh_to_gate[g].mult;
+    q.h2g_shift = sp.hh_to_gate[g].shift;
+    q.in_zp = static_cast<float>(sp.gin[g].zp);
+    q.in_lo = sp.gin[g].flo;
+    q.in_hi = sp.gin[g].fhi;
+    q.base = (lds_gates ? lut.off[g] : lut.goff[g]) - sp.gin[g].lo;
+    q.out_c = sp.gout[g].lo - sp.gout[g].zp;
+    q.out_lo = sp.gout[g].lo;
+  }
+  p.lin_zp = static_cast<float>(sp.hh_lin.zp);
+  p.lin_lo = sp.hh_lin.flo;
+  p.lin_hi = sp.hh_lin.fhi;
+  p.c_zp = static_cast<float>(sp.c.zp);
+  p.c_lo = sp.c.flo;
+  p.c_hi = sp.c.fhi;
+  p.c_scale = sp.c.scale;
+  p.c_min = sp.c.lo;
+  p.ratio_f = sp.cell_ratio[0];
+  p.ratio_i = sp.cell_ratio[1];
+  p.t_base = (tab == kTabLds ? lut.tanh_off : 0) - sp.c.lo;
+  p.t_c = sp.tanh_c.lo - sp.tanh_c.zp;
+  p.t_lo = sp.tanh_c.lo;
+  p.h_zp = static_cast<float>(sp.h.zp);
+  p.h_lo = sp.h.flo;
+  p.h_hi = sp.h.fhi;
+  p.h_scale = sp.h.scale;
+  p.hid_mult = sp.hidden.mult;
+  p.hid_shift = sp.hidden.shift;
+
+  int device = 0, ncu = 0;
+  RXMET_CHECK_HIP(hipGetDevice(&device));
+  RXMET_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
+  const bool clustered = H > 256;
+  const int ns = clustered ? kLresTile : ((B + 1) / 2 <= ncu ? 2 : 4);
+  const int mode = ra.hidden == nullptr ? kLresInfer : (ra.ckb ? kLresCodes : kLresFloat);
+  const void *fn = npl == 1 ? (mode == kLresInfer   ? lres_kernel<1, kLresInfer>(H, ns, tab)
+                               : mode == kLresCodes ? lres_kernel<1, kLresCodes>(H, ns, tab)
+                                                    : lres_kernel<1, kLresFloat>(H, ns, tab))
+                            : (mode == kLresInfer   ? lres_kernel<2, kLresInfer>(H, ns, tab)
+                               : mode == kLresCodes ? lres_kernel<2, kLresCodes>(H, ns, tab)
+                                                    : lres_kernel<2, kLresFloat>(H, ns, tab));
+  const int ks = H > 256 ? 8 : (H > 128 ? 4 : (H > 64 ? 2 : 1)), upw = ks == 4 ? 2 : 1;
+  const size_t lds = lres_lds_bytes(npl, ks, ns, p.lds_gates, tab == kTabLds16 ? p.tanh_n : 0);
+  RXMET_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      static_cast<int>(lds)));
+  if (int rc = build_act_tables(sp, lut, lut_table, gtab, n_exc, stream)) return rc;
+  void *args[] = {const_cast<RecArgs *>(&ra), &p};
+  if (!clustered) {
+    const int waves = (H / 16 + upw - 1) / upw;
+    rxmet::prof::Scope ps__("lstm_fwd_recurrence", stream);
+    RXMET_CHECK_HIP(hipLaunchKernel(fn, dim3((B + ns - 1) / ns), dim3(64 * waves), args, lds, stream));
+    return 1;
+  }
+  p.G = (H + kLresMember - 1) / kLresMember;
+  p.ntiles = (B + kLresTile - 1) / kLresTile;
+  int per_cu = 0;
+  RXMET_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 512, lds));
+  p.ncl = std::min(per_cu * ncu / p.G, p.ntiles);
+  if (p.ncl < 1) return 0;
+  if (p.ncl >= 8) p.ncl -= p.ncl % 8;
+  p.hx = reinterpret_cast<int8_t *>(wsb + ws.hx);
+  p.counters = reinterpret_cast<unsigned *>(wsb + ws.sync);
+  p.timeout = reinterpret_cast<int *>(p.counters + cluster::kCounterStride * p.ncl);
+  p.spin_limit = cluster::spin_limit();
+  hipLaunchKernelGGL(cluster::zero_words, dim3(1), dim3(256), 0, stream, p.counters,
+                     cluster::kCounterStride * p.ncl + 1);
+  RXMET_CHECK_LAUNCH();
+  {
+    rxmet::prof::Scope ps__("lstm_fwd_recurrence", stream);
+    RXMET_CHECK_HIP(cluster::launch(fn, dim3(p.ncl * p.G), dim3(512), args,
+                                    static_cast<unsigned>(lds), stream));
+  }
+  const int64_t n_out = static_cast<int64_t>(ra.T) * B * H, n_state = static_cast<int64_t>(B) * H;
+  hipLaunchKernelGGL(lstm_poison_on_timeout, dim3(64), dim3(256), 0, stream, p.timeout, n_out,
+                     ra.output, n_state, ra.h_n, ra.c_n);
+  RXMET_CHECK_LAUNCH();
+  return 1;
+}
 
 }  // namespace lstm
 }  // namespace rxmet
@@ -1507,6 +1679,10 @@ static int lstm_forward_impl(int32_t T, int32_t B, int32_t I, int32_t H, const f
     return 0;
   };
   if (stepped) return run_stepped();
+  if (pw == 1 && f32_grids) {
+    const int rc = lstm_res_launch(ra, sp, npl, static_cast<int>(exc.key.size()), ws, wsb, stream);
+    if (rc != 0) return rc < 0 ? rc : 0;
+  }
   if (may_cluster) {
     // clustered path when the whole grid can be resident at once
     const bool has_exc = !exc.key.empty();
@@ -1598,36 +1774,9 @@ static int lstm_forward_impl(int32_t T, int32_t B, int32_t I, int32_t H, const f
       hipLaunchKernelGGL(cluster::zero_words, dim3(1), dim3(256), 0, stream, cl.counters,
                      cluster::kCounterStride * ncl + 1);
       RXMET_CHECK_LAUNCH();
-      const int n_exc = static_cast<int>(exc.key.size());
-      if (lut.total > 0) {
-        hipLaunchKernelGGL(lstm_build_act_lut, dim3((lut.total + 255) / 256), dim3(256), 0, stream,
-                           sp, lut, lut_table);
-        RXMET_CHECK_LAUNCH();
-        if (n_exc > 0) {
-          hipLaunchKernelGGL(lstm_act_lut_exceptions, dim3((n_exc + 255) / 256), dim3(256), 0,
-                             stream, sp, lut, lut_table);
-          RXMET_CHECK_LAUNCH();
-        }
-      }
-      if (lut.gtotal > 0) {  // the builder on the global tables' layout
-        ActLut gl{};
-        for (int g = 0; g < 4; ++g) {
-          gl.off[g] = lut.goff[g];
-          gl.n[g] = lut.gn[g];
-        }
-        gl.tanh_off = lut.gtanh_off;
-        gl.tanh_n = lut.gtanh_n;
-        gl.total = lut.gtotal;
-        uint32_t *gt = reinterpret_cast<uint32_t *>(wsb + ws.glut);
-        hipLaunchKernelGGL(lstm_build_act_lut, dim3((gl.total + 255) / 256), dim3(256), 0, stream,
-                           sp, gl, gt);
-        RXMET_CHECK_LAUNCH();
-        if (n_exc > 0) {
-          hipLaunchKernelGGL(lstm_act_lut_exceptions, dim3((n_exc + 255) / 256), dim3(256), 0,
-                             stream, sp, gl, gt);
-          RXMET_CHECK_LAUNCH();
-        }
-      }
+      if (int rc = build_act_tables(sp, lut, lut_table, reinterpret_cast<uint32_t *>(wsb + ws.glut),
+                                    static_cast<int>(exc.key.size()), stream))
+        return rc;
       void *args[] = {&ra, &sp, &cl};
       {
         rxmet::prof::Scope ps__("lstm_fwd_recurrence", stream);
