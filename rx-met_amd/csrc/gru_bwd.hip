@@ -12,7 +12,7 @@
 //                    GEMMs (h codes recovered exactly from the dequantised h);
 //   2. recurrence  : up to H = 256 with 8-bit R one workgroup per two or four sequences with
 //                    all of R_q in its VGPRs (bwd_recurrence_res: dq as 31-bit fixed point
-//                    in four byte digits, dh += R_q dq on int8 MFMA, exact sums); else both
+//                    in four byte digits, dh += R_q dq on int8 MFMA); else both
 //                    directions walk t = T-1..0 in one clustered launch
 //                    (bwd_recurrence_cl: a batch tile's hidden units split over a cluster of
 //                    workgroups, dq * scale_R exchanged through global memory each step and
@@ -36,6 +36,7 @@
 #include "cluster.h"
 #include "gru_internal.h"
 #include "mfma_frag.h"
+#include "resident.h"
 #include "rxmet_common.h"
 #include "rxmet_gru.h"
 #include "wgrad_gemm.h"
@@ -667,11 +668,12 @@ __global__ __launch_bounds__(256 * UT) void bwd_recurrence_cl(BwdArgs a0, BwdArg
 // R's channel scales become 31-bit fixed point on one exponent per sequence (the step's largest
 // magnitude, met through LDS), split into four signed byte digits, and dh += R_q dq runs on
 // v_mfma_i32_16x16x64_i8 with row 4 s + q = digit q of sequence s: the four digit sums of a
-// (sequence, unit) arrive in one lane's accumulator and are combined exactly in double.  Each
-// term is off by at most 2^-30 of the sequence's largest, and the sum itself is exact (the three
-// bf16 terms of the clustered form are exact, but accumulate in fp32): against 64-bit sums the
-// error of a whole step's gradients is no larger (training steps at H = 100 and 256: 2.8e-7 and
-// 4.8e-7 here, 2.9e-7 and 4.9e-7 clustered; the later fp32 weight products dominate).
+// (sequence, unit) arrive in one lane's accumulator.  Each term is off by at most 2^-30 of the
+// sequence's largest, the digit sums are exact and their combination is within two units in the
+// last place of fp32 (the three bf16 terms of the clustered form are exact, but accumulate over 3H
+// products in fp32): the error of a whole step's gradients against 64 bits is no larger (training
+// steps at H = 100 and 256: 2.9e-7 and 4.8e-7 here, 2.9e-7 and 4.9e-7 clustered; the later fp32
+// weight products dominate).
 //
 // A digit must sit next to its neighbours' along K: a lane holds the four digits of one channel,
 // four lanes of a quad hold four consecutive channels, and two DPP exchanges transpose the 4 x 4
@@ -679,39 +681,10 @@ __global__ __launch_bounds__(256 * UT) void bwd_recurrence_cl(BwdArgs a0, BwdArg
 //
 // Measured (both directions of B = 256, T = 200, H = 256, saved codes): 1021 us clustered ->
 // 345 us.  Bound: the chain of one step (two LDS exchanges, 24 MFMA per wave, about 200 VALU).
-constexpr unsigned kResSkip = 0x80000000u;  // an offset past every buffer: the store is dropped
 constexpr int kResMaxH = 256;
 
 constexpr size_t bwd_res_lds(int ks2, int ns) {
   return 256 + static_cast<size_t>(4) * ns * (64 * ks2 + 16);
-}
-
-// All of the workgroup's LDS accesses are complete; memory accesses stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// Largest of the 16 lanes of a row, in every lane of it.
-__device__ __forceinline__ unsigned row16_max(unsigned v) {
-  const int i0 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xf, 0xf, true);  // lane ^ 1
-  v = max(v, static_cast<unsigned>(i0));
-  const int i1 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xf, 0xf, true);  // lane ^ 2
-  v = max(v, static_cast<unsigned>(i1));
-  const int i2 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x141, 0xf, 0xf, true);  // half mirror
-  v = max(v, static_cast<unsigned>(i2));
-  const int i3 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x140, 0xf, 0xf, true);  // mirror
-  return max(v, static_cast<unsigned>(i3));
-}
-
-// Byte i of the four lanes of a quad, to lane i of the quad (its byte k from lane k); s1, s2: the
-// lane's selectors (odd lanes, upper pairs).
-__device__ __forceinline__ unsigned quad_transpose(unsigned v, unsigned s1, unsigned s2) {
-  const unsigned x = static_cast<unsigned>(
-      __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xf, 0xf, true));
-  v = __builtin_amdgcn_perm(x, v, s1);
-  const unsigned y = static_cast<unsigned>(
-      __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xf, 0xf, true));
-  return __builtin_amdgcn_perm(y, v, s2);
 }
 
 // One element's step inputs as they are in memory.
@@ -823,8 +796,6 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
     // this lane writes digit row 4 seq + e % 4, channels of the quad's four units
     pw[k] = pl + (own[k] ? (4 * seq + e % 4) * ROW + 16 * ut + (e & ~3) : 0);
   }
-  const unsigned sel1 = e & 1 ? 0x03070105u : 0x06020400u;
-  const unsigned sel2 = e & 2 ? 0x03020706u : 0x05040100u;
   // A operand: row l % 16 = 4 s + q (rows without a sequence repeat one that exists)
   const int8_t *ar = pl + (e % (4 * NS)) * ROW + 16 * grp;
 
@@ -838,7 +809,7 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
       r[k].g = gp[k][go];
-      r[k].h = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rh, ol[k], 0, 0));
+      r[k].h = buf_load_f32(rh, ol[k]);
     }
     if constexpr (CODES) {
       const auto rc = cluster::buffer_rsrc(a.vc + tt * step_blk * 64, step_blk * 128);
@@ -847,9 +818,8 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
       for (int k = 0; k < NP; ++k) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          r[k].c[q] = static_cast<unsigned short>(
-              __builtin_amdgcn_raw_buffer_load_b16(rc, oc[k] + 32u * q, 0, 0));
-        r[k].c[4] = static_cast<unsigned short>(__builtin_amdgcn_raw_buffer_load_b16(rm, om[k], 0, 0));
+          r[k].c[q] = buf_load_u16(rc, oc[k] + 32u * q);
+        r[k].c[4] = buf_load_u16(rm, om[k]);
       }
     } else {
       const auto rv = cluster::buffer_rsrc(a.v + 4 * tt * B * H, 4u * step_h);
@@ -863,16 +833,15 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
       for (int k = 0; k < NP; ++k) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          r[k].v[q] = __builtin_bit_cast(
-              float, __builtin_amdgcn_raw_buffer_load_b32(rv, oc[k] + 4u * q * H, 0, 0));
+          r[k].v[q] = buf_load_f32(rv, oc[k] + 4u * q * H);
 #pragma unroll
         for (int g = 0; g < 3; ++g) {
-          r[k].c[g] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r0, om[k] + g * H, 0, 0));
-          r[k].c[3 + g] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r1, om[k] + g * H, 0, 0));
-          r[k].c[6 + g] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r2, om[k] + g * H, 0, 0));
-          r[k].c[9 + g] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r3, om[k] + g * H, 0, 0));
+          r[k].c[g] = buf_load_u8(r0, om[k] + g * H);
+          r[k].c[3 + g] = buf_load_u8(r1, om[k] + g * H);
+          r[k].c[6 + g] = buf_load_u8(r2, om[k] + g * H);
+          r[k].c[9 + g] = buf_load_u8(r3, om[k] + g * H);
         }
-        r[k].c[12] = static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(r4, ol[k] / 4, 0, 0));
+        r[k].c[12] = buf_load_u8(r4, ol[k] / 4);
       }
     }
   };
@@ -918,27 +887,20 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
       for (int k = 0; k < NP; ++k)
 #pragma unroll
         for (int g = 0; g < 3; ++g) {
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dpv[k][g]), rp,
-                                                od[k] + 4u * g * H, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dqv[k][g]), rq,
-                                                od[k] + 4u * g * H, 0, 0);
+          buf_f32(rp, dpv[k][g], od[k] + 4u * g * H);
+          buf_f32(rq, dqv[k][g], od[k] + 4u * g * H);
         }
     }
     const uint4 m0 = *reinterpret_cast<const uint4 *>(smax + (seq < NS ? seq : 0) * 8);
     const uint4 m1 = *reinterpret_cast<const uint4 *>(smax + (seq < NS ? seq : 0) * 8 + 4);
     const unsigned top = max(max(max(m0.x, m0.y), max(m0.z, m0.w)), max(max(m1.x, m1.y), max(m1.z, m1.w)));
-    // the largest is below 2^(ex - 126): scaled by 2^ex2 everything is below 2^30
-    const int ex2 = 156 - static_cast<int>(top >> 23);
-    const bool bad = top >= 0x7f800000u;
+    const int ex2 = fixed_exp(top);
+    const bool bad = fixed_bad(top);
 #pragma unroll
     for (int k = 0; k < NP; ++k)
 #pragma unroll
       for (int g = 0; g < 3; ++g) {
-        const int q = bad ? 0 : static_cast<int>(rintf(ldexpf(sv[k][g], ex2)));
-        // four signed digits: adding 128 to the three low bytes carries into the next, and
-        // flipping their top bits subtracts it again
-        const unsigned dg = (static_cast<unsigned>(q) + 0x00808080u) ^ 0x00808080u;
-        const unsigned tr = quad_transpose(dg, sel1, sel2);
+        const unsigned tr = quad_transpose8(bad ? 0u : fixed_digits(sv[k][g], ex2), e);
         if (own[k]) *reinterpret_cast<unsigned *>(pw[k] + g * H) = tr;
       }
     lds_barrier();
@@ -960,10 +922,7 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
         if constexpr (kMerge)
           sum[q] = __builtin_amdgcn_permlane32_swap(acc[0][q], acc[UPW - 1][q], false, false)[0];
       }
-      // |sum| < 2^24, so the low pair and the high pair are exact in int32, the whole in double
-      const double s = 65536.0 * static_cast<double>(256LL * sum[3] + sum[2]) +
-                       static_cast<double>(256LL * sum[1] + sum[0]);
-      const float add = bad ? NAN : static_cast<float>(ldexp(s, -ex2));
+      const float add = bad ? NAN : fixed_sum(sum[0], sum[1], sum[2], sum[3], ex2);
       dhc[k] = dhl[k] + add;
     }
   };

@@ -32,6 +32,7 @@
 #include "exact_gemm.h"
 #include "gru_internal.h"
 #include "mfma_frag.h"
+#include "resident.h"
 #include "rxmet_common.h"
 #include "rxmet_gru.h"
 
@@ -540,7 +541,6 @@ __device__ __forceinline__ void store_point(const RecArgs &a, const StepParams &
 // What bounds it: the chain of one step (LDS reads, 24 MFMA per wave at H = 256, about 200 VALU of
 // the pointwise update, the barrier), with two waves per SIMD to overlap.
 enum { kResInfer = 0, kResCodes = 1, kResFloat = 2 };
-constexpr unsigned kResSkip = 0x80000000u;  // an offset past every buffer: the store is dropped
 
 struct ResArgs {
   int nblk;      // workgroups per direction
@@ -551,21 +551,6 @@ struct ResArgs {
 constexpr size_t res_lds_bytes(int npl, int ks, int ns, bool tab) {
   return 1024 + static_cast<size_t>(2) * ns * npl * (64 * ks + 16) +
          (tab ? sizeof(int) * 3 * kGateTabMax : 0);
-}
-
-// All of the workgroup's LDS accesses are complete; memory accesses stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-__device__ __forceinline__ void buf_f32(__amdgpu_buffer_rsrc_t r, float v, unsigned off) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, 0, 0);
-}
-__device__ __forceinline__ void buf_u16(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned off) {
-  __builtin_amdgcn_raw_buffer_store_b16(static_cast<unsigned short>(v), r, off, 0, 0);
-}
-__device__ __forceinline__ void buf_u8(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned off) {
-  __builtin_amdgcn_raw_buffer_store_b8(static_cast<unsigned char>(v), r, off, 0, 0);
 }
 
 template <int NPL, int KS, int UPW, int NS, int MODE>
@@ -674,8 +659,7 @@ __global__ __launch_bounds__(512) void recurrence_res(RecArgs a0, RecArgs a1,
     for (int k = 0; k < NP; ++k)
 #pragma unroll
       for (int g = 0; g < 3; ++g)
-        gi[k][g] = __builtin_bit_cast(
-            float, __builtin_amdgcn_raw_buffer_load_b32(r, og[k] + 4u * g * H, 0, 0));
+        gi[k][g] = buf_load_f32(r, og[k] + 4u * g * H);
   };
   const float plane_off = 128.0f + a.h_offset;
 

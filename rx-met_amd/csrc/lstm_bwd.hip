@@ -10,7 +10,9 @@
 //   1. prologue  : x and h_prev codes and the W_ih codes as bf16 operand planes for the
 //                  weight-gradient GEMMs; W_hh codes packed as int8 MFMA fragments of the
 //                  transposed product, with their column sums;
-//   2. recurrence: a batch tile's dh product over a cluster of workgroups
+//   2. recurrence: W_hh of 8 bits and H up to 512: W_hh in the registers of one workgroup, or
+//                  of a cluster of up to four above H = 256 (lstm_bwd_resident.h); else a batch
+//                  tile's dh product over a cluster of workgroups
 //                  (lstm_bwd_recurrence_cl; the per-tile fallback lstm_bwd_recurrence keeps
 //                  one workgroup per 16 sequences).  Per step: the pointwise backward with
 //                  every mask family in the reference's operation order; dgates_hh * scale_W
@@ -869,6 +871,14 @@ __global__ __launch_bounds__(512) void lstm_bwd_recurrence_cl(BwdArgs a, BwdClAr
   }
 }
 
+}  // namespace lstm
+}  // namespace rxmet
+
+#include "lstm_bwd_resident.h"
+
+namespace rxmet {
+namespace lstm {
+
 size_t bwd_cl_lds() {
   return sizeof(double) * 8 * 4 * 64 * 4 + 2 * sizeof(int) * kBB + sizeof(float) * kBB * 8 * kBcUnits +
          kCkBytes;
@@ -940,11 +950,11 @@ struct BwdWorkspace {
     gsum = o; o += al(sizeof(float) * 4 * C * std::max(sih, shh));
     // clustered recurrence (H a multiple of 64)
     const size_t Bpad = (static_cast<size_t>(B) + kBB - 1) / kBB * kBB, G = H / kBcUnits + 1;
-    wfrag_cl = o; o += al(sizeof(v4i) * 64 * (H / 16) * KS2);
+    wfrag_cl = o; o += al(sizeof(v4i) * std::max(64 * (H / 16) * KS2, bres_frags(H)));
     csum = o; o += al(sizeof(float) * KS2 * H);
-    xp = o; o += al(2 * 3 * Bpad * C);
+    xp = o; o += al(std::max(2 * 3 * Bpad * C, sizeof(float) * bres_exchange(B, H)));
     xe = o; o += al(sizeof(int) * 2 * Bpad * G);
-    sync = o; o += al(sizeof(unsigned) * cluster::kCounterStride * (Bpad / kBB + 1));
+    sync = o; o += al(sizeof(unsigned) * cluster::kCounterStride * (Bpad / kBresTile + 1));
     // stepped recurrence: K-split parts of dh, the cell gradient, W_hh codes as bf16 planes
     dhr = o; o += al(sizeof(float) * kBStepMaxSplit * static_cast<size_t>(B) * H);
     dcs = o; o += al(sizeof(float) * static_cast<size_t>(B) * H);
@@ -1121,7 +1131,15 @@ static int lstm_backward_impl(int32_t T, int32_t B, int32_t I, int32_t H,
                   a16(grad_output) && a16(sv.ih_linear_m) && a16(sv.hh_linear_m) &&
                   a16(sv.gate_in_m) && a16(sv.gate_out_m) && a16(sv.cell_m) &&
                   a16(sv.cell_tanh_m) && a16(sv.hidden_m);
-  if (!stepped && H % (2 * kBcUnits) == 0 && KS2 <= 8 * kBcMaxKs && ck_aligned &&
+  if (!stepped && ck_aligned) {
+    const int rc = lstm_bwd_res_launch(ba, sp, sv.w_hh_q, reinterpret_cast<v4i *>(wsb + ws.wfrag_cl),
+                                       reinterpret_cast<float *>(wsb + ws.xp),
+                                       reinterpret_cast<unsigned *>(wsb + ws.sync), stream,
+                                       &timeout_flag);
+    if (rc < 0) return rc;
+    recurrence_done = rc == 1;
+  }
+  if (!stepped && !recurrence_done && H % (2 * kBcUnits) == 0 && KS2 <= 8 * kBcMaxKs && ck_aligned &&
       6.0 * ((B + kBB - 1) / kBB * kBB) * C < 2147483648.0 &&
       std::getenv("RXMET_NO_CLUSTER") == nullptr) {
     const void *fn = codes ? reinterpret_cast<const void *>(&lstm_bwd_recurrence_cl<true>)

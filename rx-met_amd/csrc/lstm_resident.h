@@ -24,6 +24,8 @@
 // elements per lane.  Packing the saved codes into 8-byte stores by quad transposes: no gain.
 #pragma once
 
+#include "resident.h"
+
 namespace rxmet {
 namespace lstm {
 
@@ -31,7 +33,6 @@ enum { kLresInfer = 0, kLresCodes = 1, kLresFloat = 2 };
 // gates and tanh in LDS; gates and a 16-bit tanh table in LDS; gates in LDS, tanh in global memory;
 // both in global memory
 enum { kTabLds = 0, kTabLds16 = 1, kTabGlobalTanh = 2, kTabGlobal = 3 };
-constexpr unsigned kLresSkip = 0x80000000u;  // an offset past every buffer: the store is dropped
 constexpr int kLresMember = 128;             // units of a cluster member (8 waves x 16)
 constexpr int kLresTile = 8;                 // sequences of a cluster
 
@@ -60,19 +61,6 @@ struct LresParams {
   int *timeout;
   unsigned spin_limit;
 };
-
-__device__ __forceinline__ void lres_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-__device__ __forceinline__ void lres_f32(__amdgpu_buffer_rsrc_t r, float v, unsigned off) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, 0, 0);
-}
-__device__ __forceinline__ void lres_u16(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned off) {
-  __builtin_amdgcn_raw_buffer_store_b16(static_cast<unsigned short>(v), r, off, 0, 0);
-}
-__device__ __forceinline__ void lres_u8(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned off) {
-  __builtin_amdgcn_raw_buffer_store_b8(static_cast<unsigned char>(v), r, off, 0, 0);
-}
 
 // s clamped to [lo, hi]; bit is set where it was outside.
 __device__ __forceinline__ float lres_clamp(float s, float lo, float hi, unsigned bit, unsigned &m) {
@@ -169,14 +157,14 @@ __global__ __launch_bounds__(512) void lstm_recurrence_res(RecArgs a, LresParams
       uj[k] = j;
       const bool ok = own[k] && b < B;
       const unsigned row = static_cast<unsigned>(b) * H + j;
-      oi[k] = ok ? 4u * (static_cast<unsigned>(b) * C + j) : kLresSkip;
-      oh[k] = ok ? 4u * row : kLresSkip;
+      oi[k] = ok ? 4u * (static_cast<unsigned>(b) * C + j) : kResSkip;
+      oh[k] = ok ? 4u * row : kResSkip;
       // codes: the block's offset and the element's place in it; float format: mask offsets
       const unsigned blk = static_cast<unsigned>(b / 16) * (H / 16) + ut;
-      ob[k] = MODE == kLresCodes ? (ok ? blk * kLckBlock : kLresSkip)
-                                 : (ok ? static_cast<unsigned>(b) * C + j : kLresSkip);
-      oq[k] = MODE == kLresCodes ? (ok ? 2u * (blk * kLcellBlock + (b % 16) * 16 + e) : kLresSkip)
-                                 : (ok ? row : kLresSkip);
+      ob[k] = MODE == kLresCodes ? (ok ? blk * kLckBlock : kResSkip)
+                                 : (ok ? static_cast<unsigned>(b) * C + j : kResSkip);
+      oq[k] = MODE == kLresCodes ? (ok ? 2u * (blk * kLcellBlock + (b % 16) * 16 + e) : kResSkip)
+                                 : (ok ? row : kResSkip);
       cst[k] = ok ? a.c0q[row] : p.c_zp;
       hv[k] = ok ? a.h0q[row] : p.h_zp;
       hw[k] = hs + (own[k] ? seq * NPL * ROW + j : 0);
@@ -198,10 +186,8 @@ __global__ __launch_bounds__(512) void lstm_recurrence_res(RecArgs a, LresParams
           for (int q = 0; q < NPL; ++q) {
             // four lanes of a quad hold four consecutive bytes: lane 0 of it stores the word
             unsigned v = static_cast<unsigned>(NPL == 1 ? hc : (q == 0 ? (hc & 255) - 128 : hc >> 8)) & 255u;
-            const int b1 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xf, 0xf, true);
-            v |= static_cast<unsigned>(b1) << 8;
-            const int b2 = __builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xf, 0xf, true);
-            v |= static_cast<unsigned>(b2) << 16;
+            v |= quad_xor1(v) << 8;
+            v |= quad_xor2(v) << 16;
             if (own[k] && e % 4 == 0)
               cluster::store_coherent(reinterpret_cast<unsigned *>(dst + q * plane_stride), v);
           }
@@ -229,8 +215,7 @@ __global__ __launch_bounds__(512) void lstm_recurrence_res(RecArgs a, LresParams
       for (int k = 0; k < NP; ++k)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          lh[k][g] = __builtin_bit_cast(
-              float, __builtin_amdgcn_raw_buffer_load_b32(r, oi[k] + 4u * g * H, 0, 0));
+          lh[k][g] = buf_load_f32(r, oi[k] + 4u * g * H);
     };
 
     auto step = [&](int t, int par, float (&lh)[NP][4]) {
@@ -309,18 +294,18 @@ __global__ __launch_bounds__(512) void lstm_recurrence_res(RecArgs a, LresParams
         cluster::arrive(counter);
         ++epoch;
       } else {
-        lres_barrier();
+        lds_barrier();
       }
       // everything below is independent of the next step's reads
       load_in(t + (kDeep ? 2 : 1), lh);
       const size_t t64 = static_cast<size_t>(t);
       const auto ro = cluster::buffer_rsrc(a.output + t64 * B * H, step_h);
 #pragma unroll
-      for (int k = 0; k < NP; ++k) lres_f32(ro, (hv[k] - p.h_zp) * p.h_scale, oh[k]);
+      for (int k = 0; k < NP; ++k) buf_f32(ro, (hv[k] - p.h_zp) * p.h_scale, oh[k]);
       if constexpr (MODE != kLresInfer) {
         const auto rhd = cluster::buffer_rsrc(a.hidden + t64 * B * H, step_h);
 #pragma unroll
-        for (int k = 0; k < NP; ++k) lres_f32(rhd, hv[k], oh[k]);
+        for (int k = 0; k < NP; ++k) buf_f32(rhd, hv[k], oh[k]);
       }
       if constexpr (MODE == kLresCodes) {
         const auto rb = cluster::buffer_rsrc(a.ckb + t64 * nblk * kLckBlock, nblk * kLckBlock);
@@ -331,12 +316,12 @@ __global__ __launch_bounds__(512) void lstm_recurrence_res(RecArgs a, LresParams
           const unsigned R = static_cast<unsigned>(R0 + sq[k]) % 16;
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
-            lres_u16(rb, ge[k][g] >> 1, ob[k] + 2u * ((R * 4 + g) * 16 + e));
-            lres_u8(rb, gm[k][g], ob[k] + kLckGm + (g * 16 + R) * 16 + e);
+            buf_u16(rb, ge[k][g] >> 1, ob[k] + 2u * ((R * 4 + g) * 16 + e));
+            buf_u8(rb, gm[k][g], ob[k] + kLckGm + (g * 16 + R) * 16 + e);
           }
-          lres_u16(rb, te[k] >> 1, ob[k] + kLckTanh + 2u * (R * 16 + e));
-          lres_u8(rb, cm[k], ob[k] + kLckCm + R * 16 + e);
-          lres_u16(rc, static_cast<unsigned>(static_cast<int>(cnew[k]) - p.c_min), oq[k]);
+          buf_u16(rb, te[k] >> 1, ob[k] + kLckTanh + 2u * (R * 16 + e));
+          buf_u8(rb, cm[k], ob[k] + kLckCm + R * 16 + e);
+          buf_u16(rc, static_cast<unsigned>(static_cast<int>(cnew[k]) - p.c_min), oq[k]);
         }
       } else if constexpr (MODE == kLresFloat) {
         const auto rg = cluster::buffer_rsrc(a.gate_out + t64 * B * C, step_c);
@@ -352,24 +337,24 @@ __global__ __launch_bounds__(512) void lstm_recurrence_res(RecArgs a, LresParams
         for (int k = 0; k < NP; ++k) {
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
-            lres_f32(rg, static_cast<float>(static_cast<int>(ge[k][g] >> 1) + p.g[g].out_lo),
+            buf_f32(rg, static_cast<float>(static_cast<int>(ge[k][g] >> 1) + p.g[g].out_lo),
                      oi[k] + 4u * g * H);
-            lres_u8(r0, gm[k][g] & 1u, ob[k] + g * H);
-            lres_u8(r1, (gm[k][g] >> 1) & 1u, ob[k] + g * H);
-            lres_u8(r2, gm[k][g] >> 2, ob[k] + g * H);
+            buf_u8(r0, gm[k][g] & 1u, ob[k] + g * H);
+            buf_u8(r1, (gm[k][g] >> 1) & 1u, ob[k] + g * H);
+            buf_u8(r2, gm[k][g] >> 2, ob[k] + g * H);
           }
-          lres_f32(rc, cnew[k], oh[k]);
-          lres_f32(rt, static_cast<float>(static_cast<int>(te[k] >> 1) + p.t_lo), oh[k]);
-          lres_u8(m0, cm[k] & 1u, oq[k]);
-          lres_u8(m1, (cm[k] >> 1) & 1u, oq[k]);
-          lres_u8(m2, cm[k] >> 2, oq[k]);
+          buf_f32(rc, cnew[k], oh[k]);
+          buf_f32(rt, static_cast<float>(static_cast<int>(te[k] >> 1) + p.t_lo), oh[k]);
+          buf_u8(m0, cm[k] & 1u, oq[k]);
+          buf_u8(m1, (cm[k] >> 1) & 1u, oq[k]);
+          buf_u8(m2, cm[k] >> 2, oq[k]);
         }
       }
       if constexpr (kCluster) {
         alive = cluster::wait(counter, epoch * p.G, p.timeout, p.spin_limit);
         if (alive && t + 1 < T) {
           get_h(par ^ 1);
-          lres_barrier();
+          lds_barrier();
         }
       }
     };
@@ -383,7 +368,7 @@ __global__ __launch_bounds__(512) void lstm_recurrence_res(RecArgs a, LresParams
       if (!alive) break;
       get_h(0);
     }
-    lres_barrier();  // h, the zeroed rows and the tables are in LDS
+    lds_barrier();  // h, the zeroed rows and the tables are in LDS
     if constexpr (kDeep) {
       for (int t = 0;;) {
         step(t, 0, la);
@@ -398,8 +383,8 @@ __global__ __launch_bounds__(512) void lstm_recurrence_res(RecArgs a, LresParams
     const auto rhn = cluster::buffer_rsrc(a.h_n, step_h), rcn = cluster::buffer_rsrc(a.c_n, step_h);
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      lres_f32(rhn, (hv[k] - p.h_zp) * p.h_scale, oh[k]);
-      lres_f32(rcn, (cst[k] - p.c_zp) * p.c_scale, oh[k]);
+      buf_f32(rhn, (hv[k] - p.h_zp) * p.h_scale, oh[k]);
+      buf_f32(rcn, (cst[k] - p.c_zp) * p.c_scale, oh[k]);
     }
   }
 }

@@ -60,3 +60,66 @@ def test_cluster_timeout_poisons_the_outputs(cuda, monkeypatch):
     again = _gpu_forward(cuda, args, p, False)
     for r, b, a in zip(ref[:3], bad[:3], again[:3]):
         assert torch.isnan(b).all() and torch.equal(r, a)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_resident_backward_matches_oracle(cuda, case):
+    """Gradients within 1e-5 of the oracle's 64-bit sums relative to each tensor's norm (32-bit
+    sums over at most 4 H and T B terms: a few 1e-7 expected); the saved formats agree bit for
+    bit."""
+    T, B, I, H, cfg, state = case
+    print(f"[lstm resident bwd] {case}", flush=True)
+    args, _, p = _case(T, B, I, H, cfg, 11, True, state)
+    exp_f = LO.forward_quant(*args[:5], p, args[5], args[6], mode=LO.ACT_LIBM_EXACT)
+    g = np.random.default_rng(9)
+    go, gh, gc = ((g.standard_normal(s) * 0.1).astype(np.float32)
+                  for s in ((T, B, H), (B, H), (B, H)))
+    exp = LO.backward_quant(exp_f, p, go, gh, gc)
+    Wi, Wh, bi, bh, x, h0, c0 = (_dev(a, cuda) for a in args)
+    prm, res = _wrap(p), []
+    for codes in (False, True):
+        saved = lstm_ops.forward_quant(x, Wi, Wh, bi, bh, h0, c0, prm, True, codes=codes)[3]
+        res.append(lstm_ops.backward_quant(saved, prm, *(_dev(a, cuda) for a in (go, gh, gc))))
+    torch.cuda.synchronize()
+    for n, a, b in zip(("dx", "dW_ih", "dW_hh", "db_ih", "db_hh", "dh0", "dc0"), *res):
+        assert torch.equal(a, b), n
+        e = np.asarray(exp[n], np.float64)
+        assert np.linalg.norm(a.cpu().numpy() - e) <= 1e-5 * (np.linalg.norm(e) + 1e-30), n
+
+
+@pytest.mark.parametrize("H", [64, 512])
+def test_resident_backward_keeps_nan_in_its_sequence(cuda, H):
+    """A NaN and an infinity in two sequences' output gradients reach every unit's dh0 of those
+    sequences, and leave the others' dx and dh0 as they are without them."""
+    args, _, p = _case(4, 12, 3, H, "default", 14, True, True)
+    Wi, Wh, bi, bh, x, h0, c0 = (_dev(a, cuda) for a in args)
+    prm = _wrap(p)
+    saved = lstm_ops.forward_quant(x, Wi, Wh, bi, bh, h0, c0, prm, True, codes=True)[3]
+    res = []
+    for bad in (False, True):
+        go = torch.full((4, 12, H), 1e-2, device=cuda)
+        if bad:
+            go[1, 1, 7], go[2, 9, 9] = float("nan"), float("inf")
+        res.append(lstm_ops.backward_quant(saved, prm, go, None, None))
+    torch.cuda.synchronize()
+    keep = [b for b in range(12) if b not in (1, 9)]
+    for k in (0, 5):
+        a, b = res[0][k], res[1][k]
+        assert torch.equal(*((t[:, keep] if k == 0 else t[keep]) for t in (a, b)))
+    assert torch.isnan(res[1][5][1]).all() and torch.isnan(res[1][5][9]).all()
+
+
+def test_cluster_timeout_poisons_the_gradients(cuda, monkeypatch):
+    args, _, p = _case(6, 24, 5, 384, "default", 15, True, False)
+    Wi, Wh, bi, bh, x, h0, c0 = (_dev(a, cuda) for a in args)
+    prm = _wrap(p)
+    saved = lstm_ops.forward_quant(x, Wi, Wh, bi, bh, h0, c0, prm, True, codes=True)[3]
+    go = torch.full((6, 24, 384), 1e-2, device=cuda)
+    run = lambda: lstm_ops.backward_quant(saved, prm, go, None, None)
+    ref = run()
+    monkeypatch.setenv("RXMET_TEST_SPIN_LIMIT", "0")
+    bad = run()
+    monkeypatch.delenv("RXMET_TEST_SPIN_LIMIT")
+    again = run()
+    for r, b, a in zip(ref, bad, again):
+        assert torch.isnan(b).all() and torch.equal(r, a)
