@@ -11,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -98,6 +99,41 @@ def build_ort_ops(verbose: bool = True) -> Path | None:
     return ORT_LIB
 
 
+# The autograd node of the learnable min / max path (torch_ext/rxmet_torch.cpp): host code over
+# PyTorch's C++ headers, without a link to librxmet.so (it is handed the entry points of the
+# loaded one).  Users of the C ABI alone need no PyTorch: without it this module is not built.
+TORCH_SRC = PKG / "torch_ext" / "rxmet_torch.cpp"
+TORCH_LIB = PKG / ("rxmet_torch" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def build_torch_ext(verbose: bool = True) -> Path | None:
+    try:
+        import torch
+        from torch.utils import cpp_extension
+    except ImportError:
+        if verbose:
+            print(f"PyTorch not found; {TORCH_LIB.name} not built")
+        return None
+    BUILD.mkdir(exist_ok=True)
+    tmp = TORCH_LIB.with_suffix(".so.tmp")
+    torch_lib = Path(torch.__file__).parent / "lib"
+    cmd = [shutil.which("g++") or "g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall",
+           "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{ROOT / 'include'}", f"-I{sysconfig.get_paths()['include']}",
+           *(f"-isystem{p}" for p in cpp_extension.include_paths("cuda")), "-o", str(tmp),
+           str(TORCH_SRC), f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+           "-ltorch"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"PyTorch module build failed: {' '.join(cmd)}\n{proc.stdout}\n"
+                           f"{proc.stderr}")
+    os.replace(tmp, TORCH_LIB)
+    if verbose:
+        print(f"built {TORCH_LIB}")
+    return TORCH_LIB
+
+
 def build(verbose: bool = True) -> Path:
     BUILD.mkdir(exist_ok=True)
     sources = sorted(list(CSRC.glob("*.hip")) + list(CSRC.glob("*.cpp")))
@@ -105,7 +141,9 @@ def build(verbose: bool = True) -> Path:
         raise RuntimeError(f"no sources in {CSRC}")
     jobs = min(len(sources), max(1, min(8, os.cpu_count() or 1)))
     with cf.ThreadPoolExecutor(jobs) as ex:
+        ext = ex.submit(build_torch_ext, verbose)
         objs = list(ex.map(_compile, sources))
+        ext.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs),
            "-Wl,--no-undefined"]

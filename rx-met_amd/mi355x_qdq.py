@@ -524,26 +524,66 @@ def quantize_dequantize_minmax(tensor: torch.Tensor, mn: torch.Tensor, mx: torch
             and mx.dtype == torch.float32 and mn.is_contiguous() and mx.is_contiguous()
             and mn.shape == mx.shape and tensor.dtype in _IO_CODE and qmax > qmin):
         return None
-    _validate_arguments(tensor, mn, qmin, qmax, block_size)
-    internal = _internal_dtype(tensor.dtype, qmin, qmax)
+    call = _minmax_call(tensor.shape, tensor.dtype, mn.shape,
+                        None if block_size is None else tuple(block_size), int(qmin), int(qmax),
+                        bool(symmetric), float(sym_offset), float(min_scale),
+                        float(zero_point_shift))
+    if call is None:
+        return None
+    if call.native is not None and tensor.is_contiguous() and _native_node(tensor, mn, mx):
+        return _rx.torch_ext().qdq_minmax(tensor, mn, mx, call.native)
+    t = reshape_tensor_for_blocks(tensor, mn.shape, block_size)
+    y = _QuantDequantMinMax.apply(t, mn, mx, int(qmin), int(qmax),
+                                  (bool(symmetric), float(sym_offset), float(min_scale)),
+                                  call.plan, call.numerics)
+    return y.view(tensor.shape)
+
+
+def _native_node(*tensors) -> bool:
+    """Whether these tensors take the C++ autograd node: ordinary tensors of one device, outside
+    tracing and function transforms (the Python Function is recorded, or refused, there)."""
+    dev = tensors[0].device
+    return (torch._C._get_tracing_state() is None
+            and not torch._C._are_functorch_transforms_active()
+            and not torch.compiler.is_compiling()
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == dev
+                    for t in tensors))
+
+
+class _MinMaxCall:
+    """What a call of the fused form derives from shapes, types and options."""
+
+    __slots__ = ("plan", "numerics", "native")
+
+    def __init__(self, plan, numerics, native):
+        self.plan, self.numerics, self.native = plan, numerics, native
+
+
+# Keyed by values alone (nothing of a tensor's identity or content); the bound keeps a program
+# whose shapes change from call to call from collecting plans.
+@functools.lru_cache(maxsize=1024)
+def _minmax_call(shape, dtype, enc_shape, block_size, qmin: int, qmax: int, symmetric: bool,
+                 sym_offset: float, min_scale: float, shift: float) -> Optional[_MinMaxCall]:
+    tensor = torch.empty(shape, dtype=dtype, device="meta")
+    _validate_arguments(tensor, torch.empty(enc_shape, device="meta"), qmin, qmax, block_size)
+    internal = _internal_dtype(dtype, qmin, qmax)
     if not _is_grid_representable(internal, qmin, qmax):
         raise RuntimeError(
             f"{internal} is unable to represent quantized output of range [{qmin}, {qmax}].")
-    if max(abs(int(qmin)), abs(int(qmax))) > 1 << 24:
+    if max(abs(qmin), abs(qmax)) > 1 << 24:
         return None
-    orig_shape = tensor.shape
-    t = reshape_tensor_for_blocks(tensor, mn.shape, block_size)
-    enc_view = get_encoding_shape_with_blocks(mn.shape, block_size)
-    enc_shape = (1,) * (t.dim() - len(enc_view)) + tuple(enc_view)
-    plan = _Plan(t.shape, enc_shape)
-    if plan.C != mn.numel() or t.numel() == 0:
+    t = reshape_tensor_for_blocks(tensor, enc_shape, block_size)
+    enc_view = get_encoding_shape_with_blocks(enc_shape, block_size)
+    plan = _Plan(t.shape, (1,) * (t.dim() - len(enc_view)) + tuple(enc_view))
+    if plan.C != math.prod(enc_shape) or t.numel() == 0:
         return None
-    scalar = mn.dim() == 0 and t.dim() > 0 and internal != t.dtype
-    fn = _QuantDequantMinMax
-    y = fn.apply(t, mn, mx, int(qmin), int(qmax),
-                 (bool(symmetric), float(sym_offset), float(min_scale)), plan,
-                 _numerics(t.dtype, internal, zero_point_shift, scalar))
-    return y.view(orig_shape)
+    scalar = len(enc_shape) == 0 and t.dim() > 0 and internal != dtype
+    native = None
+    if plan.perm is None:  # a permuted layout copies its tensors: the Python Function does that
+        native = _rx.torch_ext().make_plan(list(plan.layout), _IO_CODE[dtype],
+                                           _INTERNAL_CODE[internal], shift, scalar, qmin, qmax,
+                                           symmetric, sym_offset, min_scale)
+    return _MinMaxCall(plan, _numerics(dtype, internal, shift, scalar), native)
 
 
 def minmax(tensor: torch.Tensor, enc_shape) -> Tuple[torch.Tensor, torch.Tensor]:

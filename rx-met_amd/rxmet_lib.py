@@ -16,6 +16,7 @@ _PKG = Path(__file__).resolve().parent
 LIB_PATH = Path(os.environ.get("RXMET_LIB", _PKG / "librxmet.so"))
 
 _lib: Optional[ctypes.CDLL] = None
+_torch_ext = None
 
 c_i64 = ctypes.c_int64
 c_int = ctypes.c_int
@@ -125,6 +126,28 @@ def load() -> ctypes.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def torch_ext():
+    """The autograd nodes in C++ (module ``rxmet_torch``, built by build.py), bound to the entry
+    points of the loaded library; raises if it has not been built."""
+    global _torch_ext
+    if _torch_ext is not None:
+        return _torch_ext
+    lib = load()
+    import torch  # noqa: F401  (the module's symbols come from PyTorch's libraries)
+
+    try:
+        import rxmet_torch
+    except ImportError as e:
+        raise RxmetError(
+            f"the module rxmet_torch cannot be imported ({e}): build it with "
+            "`python rx-met_amd/build.py`") from e
+    rxmet_torch.bind(*(ctypes.cast(getattr(lib, n), c_ptr).value for n in (
+        "rxmet_qdq_forward_minmax", "rxmet_qdq_backward_minmax", "rxmet_qdq_workspace_bytes_ex",
+        "rxmet_last_error")))
+    _torch_ext = rxmet_torch
+    return rxmet_torch
 
 
 def register(name: str, restype, argtypes) -> None:
