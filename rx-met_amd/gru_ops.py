@@ -445,12 +445,83 @@ def _padded_params(qp: "GRUQuantParams", H: int, Hp: int) -> "GRUQuantParams":
     for k in range(A.NCHAN):
         out._qp.chan_bits[k] = src.chan_bits[k]
         out._qp.chan_unsigned[k] = src.chan_unsigned[k]
-        dst = A.qparams_chan(out._qp, k)
-        dst[:] = 1.0
-        s = A.qparams_chan(src, k)
-        for g in range(3):
-            dst[g * Hp:g * Hp + H] = s[g * H:(g + 1) * H]
+        dst = A.qparams_chan(out._qp, k).reshape(3, Hp)
+        dst[:, :H] = A.qparams_chan(src, k)[:3 * H].reshape(3, H)
+        dst[:, H:] = 1.0
     out.bitwidth_config_ = qp.bitwidth_config_
+    return out
+
+
+# The module's own calls (PyTorch's weight layout, state saved as codes) keep the whole-tile form
+# between forward and backward, so that each direction of a pass widens its operands and narrows
+# its results in one launch (rxmet_block_copy).  A training step at T 61, B 50, I 23, H 100 took
+# 1280 - 1450 us with pad_blocks / unpad_blocks around each call and takes 590 us.
+
+def padded_hidden(H: int) -> int:
+    """H rounded up to whole unit tiles."""
+    return _padded_hidden(H)
+
+
+def widen_dirs(dirs, I: int, H: int, B: int):
+    """``dirs`` (lists of (W, R, bw, br, x, h0, quant_params), weights in PyTorch's layout) with
+    W, R, bw, br, h0 and the grids for padded_hidden(H) units; padded units have zero weights,
+    biases and states, so they reach no other unit."""
+    Hp = _padded_hidden(H)
+    jobs, out = [], []
+    dev = dirs[0][4].device
+
+    def wide(t, shape, *geo):
+        _check_f32_cuda("weight, bias or state", t)
+        w = torch.empty(shape, dtype=torch.float32, device=dev)
+        jobs.append((t, w, *geo))
+        return w
+
+    for (W, R, bw, br, x, h0, qp) in dirs:
+        Wp = wide(W, (3 * Hp, I), 3, (H, Hp), 1, (I, I))
+        Rp = wide(R, (3 * Hp, Hp), 3, (H, Hp), 1, (H, Hp))
+        bwp, brp = (wide(b, (3 * Hp,), 3, (1, 1), 1, (H, Hp)) for b in (bw, br))
+        h0p = h0
+        if h0 is not None and h0.numel() > 0:
+            if tuple(h0.shape) != (B, H):
+                raise RuntimeError("h0 must have shape [batch_size, hidden_size]")
+            h0p = wide(h0, (B, Hp), B, (1, 1), 1, (H, Hp))
+        out.append((Wp, Rp, bwp, brp, x, h0p, _padded_params(qp, H, Hp)))
+    _rx.block_copy(jobs, dev)
+    return out
+
+
+def resize_units(tensors, H_from: int, H_to: int, groups=(1, 1)):
+    """Tensor k [.., groups[k] * H_from] as [.., groups[k] * H_to] (zeros added, or the units
+    beyond H_to dropped), all in one launch; None and empty tensors are passed through."""
+    jobs, out = [], []
+    for t, n in zip(tensors, groups):
+        if t is None or t.numel() == 0:
+            out.append(t)
+            continue
+        _check_f32_cuda("gradient or state", t)
+        t = t.contiguous()
+        w = torch.empty((*t.shape[:-1], n * H_to), dtype=torch.float32, device=t.device)
+        jobs.append((t, w, t.numel() // (n * H_from), (1, 1), n, (H_from, H_to)))
+        out.append(w)
+    if jobs:
+        _rx.block_copy(jobs, jobs[0][0].device)
+    return out
+
+
+def narrow_grads(grads, I: int, H: int):
+    """backward_quant_codes_dirs' (dx, dW, dR, dbw, dbr, dh) per direction, in PyTorch's layout
+    and for padded_hidden(H) units, for H units."""
+    Hp = _padded_hidden(H)
+    jobs, out = [], []
+    for (dx, dW, dR, dbw, dbr, dh) in grads:
+        new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dW.device)
+        B = dh.shape[0]
+        n = (dx, new(3 * H, I), new(3 * H, H), new(3 * H), new(3 * H), new(B, H))
+        jobs += [(dW, n[1], 3, (Hp, H), 1, (I, I)), (dR, n[2], 3, (Hp, H), 1, (Hp, H)),
+                 (dbw, n[3], 3, (1, 1), 1, (Hp, H)), (dbr, n[4], 3, (1, 1), 1, (Hp, H)),
+                 (dh, n[5], B, (1, 1), 1, (Hp, H))]
+        out.append(n)
+    _rx.block_copy(jobs, grads[0][1].device)
     return out
 
 

@@ -323,11 +323,78 @@ def _padded_params(params: LstmQuantParams, H: int, Hp: int) -> LstmQuantParams:
         dst.scale[i] = src.scale[i]
         dst.zero_point[i] = src.zero_point[i]
     for k in range(4):
-        d = L.chan_scales(dst, k)
-        d[:] = 1.0
-        sk = L.chan_scales(src, k)
-        for g in range(4):
-            d[g * Hp:g * Hp + H] = sk[g * H:(g + 1) * H]
+        d = L.chan_scales(dst, k).reshape(4, Hp)
+        d[:, :H] = L.chan_scales(src, k).reshape(4, H)
+        d[:, H:] = 1.0
+    return out
+
+
+# Inference and training with saved codes keep the whole-tile form between forward and backward:
+# each direction of a pass widens its operands and narrows its results in one launch
+# (rxmet_block_copy) rather than a fill and copies per block and tensor.
+
+def _resized(jobs_of, device):
+    """Tensors made by one block copy: ``jobs_of`` holds (src or None, outer, (rows_src,
+    rows_dst), (cols_src, cols_dst), shape); None stays None."""
+    jobs, out = [], []
+    for src, outer, rows, cols, shape in jobs_of:
+        if src is None:
+            out.append(None)
+            continue
+        dst = torch.empty(shape, dtype=_F32, device=device)
+        jobs.append((src, dst, outer, rows, 1, cols))
+        out.append(dst)
+    _rx.block_copy(jobs, device)
+    return out
+
+
+def _forward_wide(x, W_ih, W_hh, b_ih, b_hh, h0, c0, params, save_checkpoints, codes):
+    T, B, I = x.shape
+    H = W_hh.shape[1]
+    Hp = _padded_hidden(H)
+    x, W_ih, W_hh = (_dev_f32(n, t) for n, t in (("x", x), ("weight_ih", W_ih), ("weight_hh", W_hh)))
+    bias = params.bias_enabled
+    if bias and (b_ih is None or b_hh is None):
+        raise RuntimeError("quant params enable bias but the module has no bias")
+    vec = lambda n, t: _dev_f32(n, t) if t is not None else None
+    gates, state = ((1, 1), (H, Hp), (4 * Hp,)), ((1, 1), (H, Hp), (B, Hp))
+    W_ih, W_hh, b_ih, b_hh, h0, c0 = _resized((
+        (W_ih, 4, (H, Hp), (I, I), (4 * Hp, I)), (W_hh, 4, (H, Hp), (H, Hp), (4 * Hp, Hp)),
+        (vec("bias_ih", b_ih) if bias else None, 4, *gates),
+        (vec("bias_hh", b_hh) if bias else None, 4, *gates),
+        (vec("h0", h0), B, *state), (vec("c0", c0), B, *state)), x.device)
+    out, hn, cn, saved = forward_quant(x, W_ih, W_hh, b_ih, b_hh, h0, c0,
+                                       _padded_params(params, H, Hp), save_checkpoints, codes)
+    out, hn, cn = _resized(((out, T * B, (1, 1), (Hp, H), (T, B, H)),
+                            (hn, B, (1, 1), (Hp, H), (B, H)),
+                            (cn, B, (1, 1), (Hp, H), (B, H))), x.device)
+    return out, hn, cn, saved
+
+
+def _backward_wide(saved, params, grad_output, grad_h_n, grad_c_n):
+    T, B, I = saved["x_q"].shape
+    H, Hp = params.hidden, saved["h0_q"].shape[1]
+    dev = saved["x_q"].device
+    vec = lambda n, t: _dev_f32(n, t) if t is not None else None
+    state = (B, (1, 1), (H, Hp), (B, Hp))
+    go, ghn, gcn = _resized(((_dev_f32("grad_output", grad_output), T * B, (1, 1), (H, Hp),
+                              (T, B, Hp)), (vec("grad_h_n", grad_h_n), *state),
+                             (vec("grad_c_n", grad_c_n), *state)), dev)
+    dx, dwi, dwh, dbi, dbh, dh0, dc0 = backward_quant(saved, _padded_params(params, H, Hp), go,
+                                                      ghn, gcn)
+    gates, state = (4, (1, 1), (Hp, H), (4 * H,)), (B, (1, 1), (Hp, H), (B, H))
+    return (dx, *_resized(((dwi, 4, (Hp, H), (I, I), (4 * H, I)),
+                           (dwh, 4, (Hp, H), (Hp, H), (4 * H, H)), (dbi, *gates), (dbh, *gates),
+                           (dh0, *state), (dc0, *state)), dev))
+
+
+def narrow_saved(saved: dict, H: int) -> dict:
+    """The saved tensors of a whole-tile forward (codes decoded) for H units."""
+    Hp = saved["h0_q"].shape[1]
+    out = dict(saved)
+    for k, axes in _SAVED_HIDDEN_AXES.items():
+        for axis, groups in axes if out.get(k) is not None else ():
+            out[k] = _unpad(out[k], H, Hp, axis, groups)
     return out
 
 
@@ -372,10 +439,13 @@ def forward_quant(x, W_ih, W_hh, b_ih, b_hh, h0, c0, params: LstmQuantParams,
     ``save_checkpoints`` is set, else None.  With ``codes`` the checkpoints other than hidden
     and the recurrence masks are kept as the blocked codes of rxmet_lstm_forward_quant_codes
     (``codes_blocks``, ``cell_codes``; decode_saved_codes restores them), for backward_quant
-    only."""
+    only; for H not a multiple of 16 every saved tensor then has H rounded up (narrow_saved)."""
     T, B, I = x.shape
     H = W_hh.shape[1]
     if H % _UNIT_TILE:
+        if codes or not save_checkpoints:
+            return _forward_wide(x, W_ih, W_hh, b_ih, b_hh, h0, c0, params, save_checkpoints,
+                                 codes)
         return _forward_padded(x, W_ih, W_hh, b_ih, b_hh, h0, c0, params, save_checkpoints)
     x, W_ih, W_hh = (_dev_f32(n, t) for n, t in (("x", x), ("weight_ih", W_ih), ("weight_hh", W_hh)))
     bias = params.bias_enabled
@@ -412,6 +482,8 @@ def backward_quant(saved: dict, params: LstmQuantParams, grad_output, grad_h_n=N
     H = saved["h0_q"].shape[1]
     if H % _UNIT_TILE:
         return _backward_padded(saved, params, grad_output, grad_h_n, grad_c_n)
+    if H == _padded_hidden(params.hidden) != params.hidden:
+        return _backward_wide(saved, params, grad_output, grad_h_n, grad_c_n)
     C = 4 * H
     dev = saved["x_q"].device
     grad_output = _dev_f32("grad_output", grad_output)

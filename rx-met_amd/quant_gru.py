@@ -464,15 +464,15 @@ class GRUFunction(torch.autograd.Function):
         device = _require_device(input)
         # inference on the FP32 carrier reads the weights as they are too (no reorder kernels),
         # and x in place when its feature stride is 1 (a batch-first caller's transposed view)
-        eval_torch_w = (not is_training and quant_storage_dtype == "float32"
-                        and H % 16 == 0)
+        eval_torch_w = not is_training and quant_storage_dtype == "float32"
         input = ensure_cuda_float32(input, device)
         if not (eval_torch_w and input.stride(2) == 1):
             input = input.contiguous()
         h0_t = (ensure_cuda_float32(h0, device).contiguous() if h0 is not None
                 else torch.empty(0, device=device, dtype=torch.float32))
-        ctx.codes = bool(is_training and quant_storage_dtype == "float32" and H % 16 == 0
+        ctx.codes = bool(is_training and quant_storage_dtype == "float32"
                          and SAVE_STATE_AS_CODES and _codes_fit(quant_params))
+        Hp = gru_ops.padded_hidden(H)
         if ctx.codes or eval_torch_w:
             # weights read in PyTorch's layout by the library; in training the state saved as codes
             W = ensure_cuda_float32(weight_ih, device).contiguous()
@@ -484,7 +484,10 @@ class GRUFunction(torch.autograd.Function):
                 bw = br = _zeros(3 * H, device)
             fwd = (gru_ops.forward_quant_codes_dirs if ctx.codes
                    else gru_ops.forward_quant_float_storage_dirs_x)
-            outs = fwd(bool(is_training), T, B, I, H, [(W, R, bw, br, input, h0_t, quant_params)],
+            dirs = [(W, R, bw, br, input, h0_t, quant_params)]
+            if Hp != H:
+                dirs = gru_ops.widen_dirs(dirs, I, H, B)
+            outs = fwd(bool(is_training), T, B, I, Hp, dirs,
                        [(input.stride(0), input.stride(1), 0, 1)])[0]
         else:
             W, R, bw, br = convert_weights_to_haste_format(weight_ih, weight_hh, bias_ih, bias_hh,
@@ -503,9 +506,11 @@ class GRUFunction(torch.autograd.Function):
         ctx.saved_state = bool(is_training)
         if is_training:
             # (W_q, R_q, bw_q, br_q, x_q, h, v, 11 masks) as the backward consumes them, or
-            # (.., h, v_codes, 6 masks, mask_bits)
+            # (.., h, v_codes, 6 masks, mask_bits), the latter for whole unit tiles
             ctx.save_for_backward(outs[2], outs[3], outs[4], outs[5], outs[6], h_full, outs[1],
                                   *outs[7:])
+        if h_full.shape[-1] != H:
+            h_full = gru_ops.resize_units([h_full], Hp, H)[0]
         return h_full[1:], h_full[-1:]
 
     @staticmethod
@@ -522,10 +527,16 @@ class GRUFunction(torch.autograd.Function):
         masks = saved[7:]
         if ctx.codes:
             # dh read in place from grad_output / grad_h_n (no dh_new buffer)
-            views, _keep = gru_ops.grad_views(grad_output, grad_h_n, T, B, H, False, 1)
-            dx, dW, dR, dbw, dbr, dh = gru_ops.backward_quant_codes_dirs(
-                T, B, I, H, [(W_q, R_q, bw_q, br_q, x_q, None, h, v, ctx.quant_params,
-                              masks)], views=views)[0]
+            Hp, qp = gru_ops.padded_hidden(H), ctx.quant_params
+            if Hp != H:
+                grad_output, grad_h_n = gru_ops.resize_units([grad_output, grad_h_n], H, Hp)
+                qp = gru_ops._padded_params(qp, H, Hp)
+            views, _keep = gru_ops.grad_views(grad_output, grad_h_n, T, B, Hp, False, 1)
+            res = gru_ops.backward_quant_codes_dirs(
+                T, B, I, Hp, [(W_q, R_q, bw_q, br_q, x_q, None, h, v, qp, masks)], views=views)
+            if Hp != H:
+                res = gru_ops.narrow_grads(res, I, H)
+            dx, dW, dR, dbw, dbr, dh = res[0]
             return (dx, dW, dR, None if ctx.bias_none[0] else dbw,
                     None if ctx.bias_none[1] else dbr, None if ctx.h0_is_none else dh,
                     None, None, None, None)
@@ -593,7 +604,13 @@ class GRUBidirectionalFunction(torch.autograd.Function):
                          and _codes_fit(qp_r))
         fwd = (gru_ops.forward_quant_codes_dirs if ctx.codes
                else gru_ops.forward_quant_float_storage_dirs_x)
-        outs = fwd(is_training, T, B, I, H, dirs, [(st, sb, 0, 1), (st, sb, 1, 1)])
+        Hp = gru_ops.padded_hidden(H)
+        if Hp != H:
+            if is_training and not ctx.codes:
+                raise RuntimeError("training with a state that is not saved as codes takes whole "
+                                   "unit tiles here")
+            dirs = gru_ops.widen_dirs(dirs, I, H, B)
+        outs = fwd(is_training, T, B, I, Hp, dirs, [(st, sb, 0, 1), (st, sb, 1, 1)])
         ctx.bias_none = (bi_f is None, bh_f is None)
         ctx.h0_none = (h0_f is None, h0_r is None)
         ctx.quant_params = (qp_f, qp_r)
@@ -603,7 +620,10 @@ class GRUBidirectionalFunction(torch.autograd.Function):
             for o in outs:
                 saved += [o[2], o[3], o[4], o[5], o[6], o[0], o[1], *o[7:]]
             ctx.save_for_backward(*saved)
-        return gru_ops.bidir_assemble(outs[0][0], outs[1][0], ctx.batch_first)
+        output, h_n = gru_ops.bidir_assemble(outs[0][0], outs[1][0], ctx.batch_first)
+        if Hp != H:
+            output, h_n = gru_ops.resize_units([output, h_n], Hp, H, groups=(2, 1))
+        return output, h_n
 
     @staticmethod
     def backward(ctx, g_out, g_hn):
@@ -613,9 +633,14 @@ class GRUBidirectionalFunction(torch.autograd.Function):
         T, B, I, H = ctx.dims
         saved = ctx.saved_tensors
         n = len(saved) // 2
+        Hp, qps = gru_ops.padded_hidden(H), ctx.quant_params
+        if Hp != H:
+            qps = [gru_ops._padded_params(qp, H, Hp) for qp in qps]
         if ctx.codes:
             # each direction reads its dh in place from g_out / g_hn (no split copies)
-            views, _keep = gru_ops.grad_views(g_out, g_hn, T, B, H, ctx.batch_first, 2)
+            if Hp != H:
+                g_out, g_hn = gru_ops.resize_units([g_out, g_hn], H, Hp, groups=(2, 1))
+            views, _keep = gru_ops.grad_views(g_out, g_hn, T, B, Hp, ctx.batch_first, 2)
             dhs = (None, None)
         else:
             views = None
@@ -626,10 +651,12 @@ class GRUBidirectionalFunction(torch.autograd.Function):
         for k, dh_new in enumerate(dhs):
             W_q, R_q, bw_q, br_q, x_q, h, v = saved[k * n:k * n + 7]
             masks = saved[k * n + 7:(k + 1) * n]
-            dirs.append((W_q, R_q, bw_q, br_q, x_q, dh_new, h, v, ctx.quant_params[k], masks))
+            dirs.append((W_q, R_q, bw_q, br_q, x_q, dh_new, h, v, qps[k], masks))
         # weight gradients come back in PyTorch's layout and gate order
-        res = (gru_ops.backward_quant_codes_dirs(T, B, I, H, dirs, views=views) if ctx.codes
+        res = (gru_ops.backward_quant_codes_dirs(T, B, I, Hp, dirs, views=views) if ctx.codes
                else gru_ops.backward_quant_float_storage_dirs_x(T, B, I, H, dirs))
+        if Hp != H:
+            res = gru_ops.narrow_grads(res, I, H)
         grads = []
         for k, (dx, dW, dR, dbw, dbr, dh) in enumerate(res):
             grads.append((dW, dR, None if ctx.bias_none[0] else dbw,
@@ -1259,6 +1286,16 @@ class QuantGRU(nn.Module):
             input.requires_grad or (hx is not None and hx.requires_grad)
             or any(p.requires_grad for p in self.parameters())))
 
+    def _bidirectional_call(self, input, hx) -> bool:
+        """Whether GRUBidirectionalFunction takes this call: it does not for a training pass
+        whose state is saved in the reference's format (SAVE_STATE_AS_CODES) and whose hidden
+        size is not a whole number of unit tiles."""
+        if self.hidden_size % 16 == 0 or not self._save_state(input, hx):
+            return True
+        self._resolve_quant_params()
+        return (SAVE_STATE_AS_CODES and _codes_fit(self.quant_params)
+                and _codes_fit(self.quant_params_reverse))
+
     def _forward_bidirectional(self, input, hx=None):
         """Quantised bidirectional forward on the caller's layout (GRUBidirectionalFunction):
         no transposes, flips or concatenations outside the library."""
@@ -1282,7 +1319,7 @@ class QuantGRU(nn.Module):
         if self.export_mode:
             raise NotImplementedError("ONNX export mode is not provided by the MI355X build")
         if (not self.calibrating and self.bidirectional and self.use_quantization
-                and self.quant_storage_dtype == "float32" and self.hidden_size % 16 == 0):
+                and self.quant_storage_dtype == "float32" and self._bidirectional_call(input, hx)):
             return self._forward_bidirectional(input, hx)
         if self.batch_first:
             input = input.transpose(0, 1)

@@ -342,8 +342,7 @@ class _QuantizedLSTMFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, W_ih, W_hh, b_ih, b_hh, h0, c0, params, save_checkpoints, sink):
-        codes = bool(save_checkpoints and SAVE_STATE_AS_CODES and W_hh.shape[1] % 16 == 0
-                     and lstm_ops.codes_fit(params))
+        codes = bool(save_checkpoints and SAVE_STATE_AS_CODES and lstm_ops.codes_fit(params))
         out, hn, cn, saved = lstm_ops.forward_quant(x, W_ih, W_hh, b_ih, b_hh, h0, c0, params,
                                                     save_checkpoints, codes=codes)
         ctx.has_checkpoints = saved is not None
@@ -363,7 +362,8 @@ class _QuantizedLSTMFunction(torch.autograd.Function):
             raise RuntimeError("quantised backward needs the training q-carrier checkpoints "
                                "(run the forward with grad enabled or in training mode)")
         saved = dict(zip(ctx.names, ctx.saved_tensors))
-        go = grad_out if grad_out is not None else torch.zeros_like(saved["hidden"])
+        go = (grad_out if grad_out is not None else torch.zeros_like(
+            saved["hidden"][..., :ctx.params.hidden]))
         dx, dwi, dwh, dbi, dbh, dh0, dc0 = lstm_ops.backward_quant(saved, ctx.params, go, grad_hn,
                                                                    grad_cn)
         return (dx, dwi, dwh, dbi if ctx.has_bias else None, dbh if ctx.has_bias else None,
@@ -386,6 +386,8 @@ def _qat_state(saved: dict, params=None, batch: int = 0) -> dict:
     codes are decoded into it first."""
     if "codes_blocks" in saved:
         saved = {**saved, **lstm_ops.decode_saved_codes(saved, params, batch)}
+        if saved["h0_q"].shape[1] != params.hidden:
+            saved = lstm_ops.narrow_saved(saved, params.hidden)
     m = lambda k: None if saved.get(k) is None else saved[k].view(torch.bool)
     master = {"input": "x", "weight_ih": "w_ih", "weight_hh": "w_hh", "bias_ih": "b_ih",
               "bias_hh": "b_hh", "h_0": "h0", "c_0": "c0"}

@@ -44,6 +44,16 @@ class QdqMinMaxEnc(ctypes.Structure):
                 ("reserved", ctypes.c_int32)]
 
 
+class BlockJob(ctypes.Structure):
+    """rxmet_block_job (include/rxmet_layout.h): one tensor widened or narrowed."""
+    _fields_ = [("src", c_ptr), ("dst", c_ptr), ("outer", c_i64), ("rows_src", ctypes.c_int32),
+                ("rows_dst", ctypes.c_int32), ("groups", ctypes.c_int32),
+                ("cols_src", ctypes.c_int32), ("cols_dst", ctypes.c_int32),
+                ("reserved", ctypes.c_int32)]
+
+
+BLOCK_JOBS = 16  # RXMET_BLOCK_JOBS
+
 _LAY = ctypes.POINTER(QdqLayout)
 _MME = ctypes.POINTER(QdqMinMaxEnc)
 _NUM = ctypes.POINTER(QdqNumerics)
@@ -88,6 +98,7 @@ _SIGNATURES = {
                                            ctypes.c_float, ctypes.c_float, c_ptr, c_ptr, c_ptr]),
     "rxmet_qdq_encoding_backward": (c_int, [c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64,
                                             ctypes.c_int32, ctypes.c_float, c_ptr, c_ptr, c_ptr]),
+    "rxmet_block_copy": (c_int, [ctypes.c_int32, ctypes.POINTER(BlockJob), c_ptr]),
     "rxmet_prof_enable": (c_int, [ctypes.c_int32]),
     "rxmet_prof_filter": (c_int, [ctypes.c_char_p]),
     "rxmet_prof_reset": (c_int, []),
@@ -179,6 +190,26 @@ def stream_of(device) -> int:
     import torch
 
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def block_copy(jobs, device) -> None:
+    """Widen or narrow tensors in one launch (rxmet_block_copy): ``jobs`` holds (src, dst, outer,
+    (rows_src, rows_dst), groups, (cols_src, cols_dst)) with contiguous fp32 tensors of exactly
+    those sizes on ``device``."""
+    import torch
+
+    arr = (BlockJob * len(jobs))()
+    for k, (src, dst, outer, rows, groups, cols) in enumerate(jobs):
+        for t, r, c in ((src, rows[0], cols[0]), (dst, rows[1], cols[1])):
+            if (t.dtype != torch.float32 or t.device != device or not t.is_contiguous()
+                    or t.numel() != outer * r * groups * c):
+                raise RuntimeError(f"block copy: a tensor of shape {tuple(t.shape)} ({t.dtype}, "
+                                   f"{t.device}) is not [{outer}, {r}, {groups}, {c}] fp32")
+        arr[k] = BlockJob(src.data_ptr(), dst.data_ptr(), outer, *rows, groups, *cols, 0)
+    for k in range(0, len(jobs), BLOCK_JOBS):
+        part = (BlockJob * min(BLOCK_JOBS, len(jobs) - k)).from_buffer(
+            arr, k * ctypes.sizeof(BlockJob))
+        call("rxmet_block_copy", len(part), part, stream_of(device))
 
 
 def prof_enable(on: bool = True) -> None:
