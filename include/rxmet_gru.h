@@ -431,6 +431,25 @@ int rxmet_gru_forward_calibrate(int32_t T, int32_t B, int32_t I, int32_t H, cons
                                 float *stats, void *workspace, void *stream);
 
 /*
+ * rxmet_gru_forward_calibrate for one direction or both directions of a layer (ndir 1 or 2, the
+ * same sizes), the two recurrences in one launch where the GPU holds them side by side.  With
+ * reverse, the direction walks x [T,B,I] from its last step to its first; h [T+1,B,H] and v are
+ * in the direction's own order of steps either way.  With torch_layout, W, R, bw and br are
+ * PyTorch's weight_ih [3H,I], weight_hh [3H,H] and biases with gate order (r, z, n); the
+ * statistics keep the (z, r, n) order.  Each direction needs its own workspace of
+ * rxmet_gru_calibrate_workspace_bytes.
+ */
+typedef struct rxmet_gru_cal_dir {
+  const float *W, *R, *bw, *br, *x, *h0;
+  float *h, *v, *stats;
+  void *workspace;
+  int32_t reverse, torch_layout;
+} rxmet_gru_cal_dir;
+
+int rxmet_gru_forward_calibrate_dirs(int32_t ndir, int32_t T, int32_t B, int32_t I, int32_t H,
+                                     const rxmet_gru_cal_dir *dirs, void *stream);
+
+/*
  * Float GRU forward without quantisation: forward_fp
  * (pytorch/lib/gru_interface_binding.cc:656-697, hasteGRUForward).  Same kernel and
  * summation order as rxmet_gru_forward_calibrate, no statistics.  Writes h [T+1,B,H]

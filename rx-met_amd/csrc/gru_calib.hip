@@ -5,10 +5,10 @@
 //
 // Reference: forwardWithCalibrationCPU (operators/quant-gru/src/gru_forward_cpu.cc:58-151)
 // and its GPU counterpart forwardWithCalibrationGPU (src/gru_interface.cc:930-1024).
-// Main form (H a multiple of 16 up to 1024): the input projection of every step as one fp32
+// Main form (H up to 1024): the input projection of every step as one fp32
 // MFMA GEMM (calib_gemm.h) and the recurrence as a clustered persistent kernel with R resident
 // in VGPRs, the 13 activation ranges observed in registers and folded from per-workgroup
-// partials.  Fallback (other H) and the float forward: one workgroup per sequence keeps h in
+// partials.  Fallback (larger H) and the float forward: one workgroup per sequence keeps h in
 // LDS and walks the T steps with the reference's sequential fp32 summation order (sum over k,
 // then + bias) and sigmoid in double, as the reference's CPU template does; its statistics
 // are reduced with atomic min/max on order-preserving integer images of the floats.  Either
@@ -46,12 +46,19 @@ __device__ __forceinline__ void observe(float v, float &mn, float &mx) {
   }
 }
 
-template <bool STATS>
+// Weights come in one of two layouts: W [I][3H], R [H][3H] with gate order (z, r, n), or
+// (TORCH) PyTorch's weight_ih [3H][I], weight_hh [3H][H] with gate order (r, z, n).
+// Column c of the first layout is row torch_row(c, H) of the second.
+__device__ __forceinline__ int torch_row(int c, int H) {
+  return c < H ? c + H : (c < 2 * H ? c - H : c);
+}
+
+template <bool STATS, bool TORCH>
 __global__ __launch_bounds__(kCalThreads) void calib_forward(
     int T, int B, int I, int H, const float *__restrict__ W, const float *__restrict__ R,
     const float *__restrict__ bw, const float *__restrict__ br, const float *__restrict__ x,
     const float *__restrict__ h0, float *__restrict__ hout, float *__restrict__ v,
-    unsigned *__restrict__ gstat /* 2 x 13 ordered (min, max) */) {
+    unsigned *__restrict__ gstat /* 2 x 13 ordered (min, max) */, int reverse) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int C = 3 * H;
   float *hbuf = reinterpret_cast<float *>(smem);  // [2][H], h_t and h_{t+1}
@@ -79,14 +86,20 @@ __global__ __launch_bounds__(kCalThreads) void calib_forward(
   for (int t = 0; t < T; ++t) {
     const float *hs = hbuf + (t & 1) * H;
     float *hn_s = hbuf + ((t + 1) & 1) * H;
-    const float *xt = x + (static_cast<size_t>(t) * B + b) * I;
+    const float *xt = x + (static_cast<size_t>(reverse ? T - 1 - t : t) * B + b) * I;
     if (STATS)
       for (int k = tid; k < I; k += kCalThreads) observe(xt[k], mn[RXMET_GRU_X], mx[RXMET_GRU_X]);
     for (int c = tid; c < C; c += kCalThreads) {
       float si = 0.0f, sh = 0.0f;
-      for (int k = 0; k < I; ++k) si += xt[k] * W[static_cast<size_t>(k) * C + c];
-      for (int k = 0; k < H; ++k) sh += hs[k] * R[static_cast<size_t>(k) * C + c];
-      const float a = si + bw[c], r = sh + br[c];
+      const int cb = TORCH ? torch_row(c, H) : c;
+      if (TORCH) {
+        for (int k = 0; k < I; ++k) si += xt[k] * W[static_cast<size_t>(cb) * I + k];
+        for (int k = 0; k < H; ++k) sh += hs[k] * R[static_cast<size_t>(cb) * H + k];
+      } else {
+        for (int k = 0; k < I; ++k) si += xt[k] * W[static_cast<size_t>(k) * C + c];
+        for (int k = 0; k < H; ++k) sh += hs[k] * R[static_cast<size_t>(k) * C + c];
+      }
+      const float a = si + bw[cb], r = sh + br[cb];
       wx[c] = a;
       rh[c] = r;
       if (STATS) {
@@ -167,7 +180,7 @@ __global__ void stats_merge(const unsigned *o, float *s) {
 }
 
 // ---------------------------------------------------------------------------------
-// MFMA form (H a multiple of 16, H <= 1024): the input projection of every step as one fp32
+// MFMA form (H <= 1024): the input projection of every step as one fp32
 // MFMA GEMM, then the recurrence as a clustered persistent kernel with R resident in VGPRs.
 // Products and sums are fp32 (v_mfma_f32_16x16x4f32) in another order than the sequential
 // sums above; results agree to rounding (the calibration is held to 1e-5, not bit-exactness).
@@ -253,10 +266,10 @@ __global__ __launch_bounds__(256) void stats_fold(const float *__restrict__ part
 constexpr int kGemmStat = 3;
 static_assert(RXMET_GRU_X < kGemmStat && RXMET_GRU_WX < kGemmStat, "GEMM statistics layout");
 
-// wx[m][c] = sum_k x[m][k] W[k][c] + bw[c] for m < M = T B, c < C = 3H (W [I][3H], K-major),
-// with the X and WX statistics: the LDS-tiled fp32 MFMA block of calib_gemm.h, one partial
+// wx[m][c] = sum_k x[m][k] W[k][c] + bw[c] for m < M = T B, c < C = 3H (in the weights' own
+// column order), with the X and WX statistics: the LDS-tiled fp32 MFMA block of calib_gemm.h, one partial
 // block of statistics per workgroup.
-template <bool STATS>
+template <bool STATS, bool TORCH>
 __global__ __launch_bounds__(256) void calib_input_gemm(int M, int K, int C,
                                                         const float *__restrict__ x,
                                                         const float *__restrict__ W,
@@ -269,7 +282,7 @@ __global__ __launch_bounds__(256) void calib_input_gemm(int M, int K, int C,
     st_mn[i] = FLT_MAX;
     st_mx[i] = -FLT_MAX;
   }
-  calgemm::gemm_block<true>(
+  calgemm::gemm_block<!TORCH>(
       M, C, K, x, W, bw, wx, STATS && blockIdx.x == 0,
       [&](float v) {
         if (STATS) observe(v, st_mn[RXMET_GRU_X], st_mx[RXMET_GRU_X]);
@@ -285,8 +298,10 @@ __global__ __launch_bounds__(256) void calib_input_gemm(int M, int K, int C,
 struct CalClArgs {
   int T, B, H, NC, NWG, ntiles, Bpad, Hpad, G, ncl;
   const float *wx;   // [T, B, 3H] input projection with bw
-  const float *R;    // [H, 3H]
+  const float *R;    // element (k, column c) at R[k rk + c rc]
   const float *br;   // [3H]
+  int rk, rc;
+  int gz, gr;        // first columns of the z and r gates in wx, R and br (n: 2H)
   const float *h0;   // [B, H] or null
   float *hout;       // [T+1, B, H]
   float *v;          // [T, B, 4H] or null
@@ -295,15 +310,69 @@ struct CalClArgs {
   unsigned *counters;
   int *timeout;
   unsigned spin_limit;
+  int reverse;  // step t takes row T - 1 - t of wx (the reverse direction of a layer)
 };
+
+// The directions of one launch: direction k owns clusters [k ncl, (k + 1) ncl).
+struct CalClDirs {
+  CalClArgs d[2];
+  int ndir;
+};
+
+// Where h[b][k] of the exchange buffer lies (floats, within a parity's plane): tiles of 16 rows,
+// chunks of 64 units, and inside those the order of the product's operand (lane group g = k / 16
+// % 4 takes k = 64 c + 16 g .. + 15 of row b % 16, 16 bytes per load), so that each of a wave's
+// four loads of a chunk is one contiguous KB.  In rows of Hpad floats a load touched 64 separate
+// 64-byte lines, and every line four times.
+__device__ __forceinline__ unsigned hx_index(int b, int k, int Hpad) {
+  return static_cast<unsigned>(b / kCT * kCT) * Hpad + (k / 64) * 1024 + (k % 16 / 4) * 256 +
+         (k / 16 % 4) * 64 + (b % kCT) * 4 + k % 4;
+}
 
 // The recurrent product of one member for one tile: wave w takes the consecutive items
 // w IPW .. w IPW + IPW - 1 (item = 3 chunk + gate), so the three gates of a K chunk share one
 // load of its h values; every chunk the wave needs is loaded before the first MFMA.  Partial
 // tiles go to red[item][64].
+// A lane's weights of its wave's items: R(k, unit of the item's gate) for the lane group's k.
+// Rows of PyTorch's weight_hh hold them side by side: 16 bytes per load where they are aligned.
 template <int IPW>
-__device__ __forceinline__ void calib_items(const float (&rfr)[IPW][16], int w, int l, int g,
-                                            int nitems, __amdgpu_buffer_rsrc_t xr, unsigned rowoff,
+__device__ __forceinline__ void load_items(const CalClArgs &a, int w, int g, int unit,
+                                           float (&rfr)[IPW][16]) {
+  const int H = a.H;
+  const bool vec = a.rk == 1 && H % 4 == 0 && (reinterpret_cast<uintptr_t>(a.R) & 15) == 0;
+#pragma unroll
+  for (int it = 0; it < IPW; ++it) {
+    const int item = w * IPW + it, ch = item / 3, gate = item % 3;
+    const int col = (gate == 0 ? a.gz : (gate == 1 ? a.gr : 2 * H)) + unit;
+    const float *p = a.R + static_cast<size_t>(col) * a.rc;
+    const bool in = item < 3 * a.NC && unit < H;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int k = 64 * ch + 16 * g + 4 * q;
+      if (vec) {
+        v4f v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        if (in && k < H) v = *reinterpret_cast<const v4f *>(p + k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rfr[it][4 * q + e] = v[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          rfr[it][4 * q + e] = in && k + e < H ? p[static_cast<size_t>(k + e) * a.rk] : 0.0f;
+      }
+    }
+  }
+}
+
+// Slot of lane l's partial tile: four spare slots after every 16 lanes, so that the finishing
+// threads (hx_index order: four units of sixteen rows per wave) read from all banks.
+constexpr int kRedItem = kWave + 12;
+__device__ __forceinline__ int red_index(int item, int l) {
+  return item * kRedItem + l + l / 16 * 4;
+}
+
+template <int IPW>
+__device__ __forceinline__ void calib_items(const float (&rfr)[IPW][16], int w, int l, int nitems,
+                                            __amdgpu_buffer_rsrc_t xr, unsigned tileoff,
                                             v4f *red) {
   // chunks a run of IPW items spans (IPW items from a multiple of 3 when IPW is one)
   constexpr int NCH = IPW % 3 == 0 ? IPW / 3 : (IPW + 1) / 3 + 1;
@@ -313,10 +382,10 @@ __device__ __forceinline__ void calib_items(const float (&rfr)[IPW][16], int w, 
   for (int c = 0; c < NCH; ++c) {
     const int ch = first + c;
     if (3 * ch < nitems) {
-      const unsigned off = 4u * (rowoff + 64 * ch + 16 * g);
+      const unsigned off = 4u * (tileoff + 1024 * ch) + 16u * l;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int4 v = cluster::load_coherent16(xr, off + 16u * q);
+        const int4 v = cluster::load_coherent16(xr, off + 1024u * q);
         hv[c][4 * q] = __int_as_float(v.x);
         hv[c][4 * q + 1] = __int_as_float(v.y);
         hv[c][4 * q + 2] = __int_as_float(v.z);
@@ -339,7 +408,7 @@ __device__ __forceinline__ void calib_items(const float (&rfr)[IPW][16], int w, 
       for (int cc = 1; cc < NCH; ++cc) hs = c == cc ? hv[cc][s] : hs;
       acc = mfma_f32(hs, rfr[it][s], acc);
     }
-    red[item * kWave + l] = acc;
+    red[red_index(item, l)] = acc;
   }
 }
 
@@ -352,33 +421,29 @@ __device__ __forceinline__ void calib_items(const float (&rfr)[IPW][16], int w, 
 // finished by one thread (the gates, the new h and the statistics), its previous h kept in a
 // register.  NWG >= 4, so the 256 elements have threads of their own.
 template <bool STATS, int IPW, int MAXW = kCMaxW>
-__global__ __launch_bounds__(64 * MAXW) void calib_recurrence_cl(CalClArgs a) {
+__global__ __launch_bounds__(64 * MAXW) void calib_recurrence_cl(CalClDirs dirs) {
   extern __shared__ __align__(16) unsigned char smem[];
-  v4f *red = reinterpret_cast<v4f *>(smem);  // [3 NC][64]
-  const cluster::Place pl = cluster::place(a.G, a.ncl);
+  v4f *red = reinterpret_cast<v4f *>(smem);  // [3 NC][kRedItem]
+  cluster::Place pl = cluster::place(dirs.d[0].G, dirs.ndir * dirs.d[0].ncl);
+  const bool second = pl.cluster >= dirs.d[0].ncl;
+  const CalClArgs a = second ? dirs.d[1] : dirs.d[0];
+  if (second) pl.cluster -= a.ncl;
   unsigned *counter = a.counters + cluster::kCounterStride * pl.cluster;
   const int H = a.H, C = 3 * H, B = a.B, NC = a.NC;
   const int tid = threadIdx.x, w = tid / kWave, l = tid % kWave, r16 = l % 16, g = l / 16;
   const int u0 = 16 * pl.member;
   const int nitems = 3 * NC;
   float rfr[IPW][16];
-#pragma unroll
-  for (int it = 0; it < IPW; ++it) {
-    const int item = w * IPW + it, ch = item / 3, gate = item % 3;
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int k = 64 * ch + 16 * g + s;
-      rfr[it][s] = item < nitems && k < H
-                       ? a.R[static_cast<size_t>(k) * C + gate * H + u0 + r16] : 0.0f;
-    }
-  }
-  // the finishing element of this thread (tid < 256): row 4 (tid % 64 / 16) + tid / 64 and
-  // unit u0 + tid % 16 of the tile, which lane tid % 64 holds as accumulator tid / 64
+  load_items<IPW>(a, w, g, u0 + r16, rfr);
+  // the finishing element of this thread (tid < 256), in the exchange buffer's order: row
+  // tid / 4 % 16 and unit u0 + 4 (tid / 64) + tid % 4, which lane fl holds as accumulator fq
   const bool fin = tid < 256;
-  const int fl = tid % 64, fq = tid / 64;
-  const int frow = 4 * (fl / 16) + fq, fu = u0 + fl % 16;
-  const float bz = fin ? a.br[fu] : 0.0f, brr = fin ? a.br[H + fu] : 0.0f,
-              bn = fin ? a.br[2 * H + fu] : 0.0f;
+  const int frow = tid / 4 % 16, fu = u0 + tid / 64 * 4 + tid % 4;
+  const int fl = frow / 4 * 16 + fu % 16, fq = frow % 4;
+  // units past H (the last member's, H not a multiple of 16) have zero weights and states
+  const bool unit = fin && fu < H;
+  const float bz = unit ? a.br[a.gz + fu] : 0.0f, brr = unit ? a.br[a.gr + fu] : 0.0f,
+              bn = unit ? a.br[2 * H + fu] : 0.0f;
   float mn[kNStat], mx[kNStat];
 #pragma unroll
   for (int i = 0; i < kNStat; ++i) {
@@ -394,20 +459,21 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_cl(CalClArgs a) {
   for (int tile = pl.cluster; tile < a.ntiles && alive; tile += a.ncl) {
     __syncthreads();  // the previous tile's readers of the partial tiles are done
     const int b = tile * kCT + frow;
-    const bool valid = fin && b < B;
+    const bool valid = unit && b < B;
     float hold = 0.0f;
     if (fin) {
       hold = valid && a.h0 ? a.h0[static_cast<size_t>(b) * H + fu] : 0.0f;
-      cluster::store_coherent(hxw + b * a.Hpad + fu, __float_as_uint(hold));
+      cluster::store_coherent(hxw + hx_index(b, fu, a.Hpad), __float_as_uint(hold));
       if (valid) a.hout[static_cast<size_t>(b) * H + fu] = hold;
     }
     // the step's weight_ih_linear values, loaded one step ahead (they do not depend on h)
     float wz = 0.0f, wr = 0.0f, wn = 0.0f;
     auto load_wx = [&](int t) {
       if (valid) {
-        const float *wp = a.wx + (static_cast<size_t>(t) * B + b) * C + fu;
-        wz = wp[0];
-        wr = wp[H];
+        const int tx = a.reverse ? a.T - 1 - t : t;
+      const float *wp = a.wx + (static_cast<size_t>(tx) * B + b) * C + fu;
+        wz = wp[a.gz];
+        wr = wp[a.gr];
         wn = wp[2 * H];
       }
     };
@@ -415,15 +481,14 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_cl(CalClArgs a) {
     alive = cluster::sync(counter, ++epoch * a.G, a.timeout, a.spin_limit);
     for (int t = 0; t < a.T && alive; ++t) {
       const int par = t & 1;
-      const unsigned rowoff = par * plane + static_cast<unsigned>(tile * kCT + r16) * a.Hpad;
-      // A: row tile*16 + r16, h[64 ch + 16 g .. + 15] of each item's chunk
-      calib_items<IPW>(rfr, w, l, g, nitems, xr, rowoff, red);
+      const unsigned tileoff = par * plane + static_cast<unsigned>(tile * kCT) * a.Hpad;
+      calib_items<IPW>(rfr, w, l, nitems, xr, tileoff, red);
       __syncthreads();
       if (fin) {
         float rh[3] = {bz, brr, bn};
         for (int ch = 0; ch < NC; ++ch)
 #pragma unroll
-          for (int gate = 0; gate < 3; ++gate) rh[gate] += red[(ch * 3 + gate) * kWave + fl][fq];
+          for (int gate = 0; gate < 3; ++gate) rh[gate] += red[red_index(ch * 3 + gate, fl)][fq];
         const float zp = wz + rh[0];
         const float rp = wr + rh[1];
         const float z = static_cast<float>(1.0 / (1.0 + exp(-static_cast<double>(zp))));
@@ -435,7 +500,8 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_cl(CalClArgs a) {
         const float newc = (1.0f - z) * n;
         const float hn = oldc + newc;
         hold = hn;
-        cluster::store_coherent(hxw + (par ^ 1) * plane + b * a.Hpad + fu, __float_as_uint(hn));
+        cluster::store_coherent(hxw + (par ^ 1) * plane + hx_index(b, fu, a.Hpad),
+                                __float_as_uint(hn));
         if (STATS && valid) {
           observe(rh[0], mn[RXMET_GRU_RH], mx[RXMET_GRU_RH]);
           observe(rh[1], mn[RXMET_GRU_RH], mx[RXMET_GRU_RH]);
@@ -474,7 +540,7 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_cl(CalClArgs a) {
   if (STATS) {
     __syncthreads();
     block_stats(mn, mx, kNStat,
-                a.part + (static_cast<size_t>(blockIdx.x)) * 2 * kNStat);
+                a.part + static_cast<size_t>(pl.cluster * a.G + pl.member) * 2 * kNStat);
   }
 }
 
@@ -486,11 +552,14 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_cl(CalClArgs a) {
 constexpr int kMtMax = 16;
 
 template <bool STATS, int IPW, int MAXW = kCMaxW>
-__global__ __launch_bounds__(64 * MAXW) void calib_recurrence_mt(CalClArgs a) {
+__global__ __launch_bounds__(64 * MAXW) void calib_recurrence_mt(CalClDirs dirs) {
   extern __shared__ __align__(16) unsigned char smem[];
-  v4f *red = reinterpret_cast<v4f *>(smem);                             // [3 NC][64]
-  float *hl = reinterpret_cast<float *>(red + 3 * a.NC * kWave);        // [kMtMax][256]
-  const cluster::Place pl = cluster::place(a.G, a.ncl);
+  v4f *red = reinterpret_cast<v4f *>(smem);  // [3 NC][kRedItem]
+  cluster::Place pl = cluster::place(dirs.d[0].G, dirs.ndir * dirs.d[0].ncl);
+  const bool second = pl.cluster >= dirs.d[0].ncl;
+  const CalClArgs a = second ? dirs.d[1] : dirs.d[0];
+  if (second) pl.cluster -= a.ncl;
+  float *hl = reinterpret_cast<float *>(red + 3 * a.NC * kRedItem);  // [kMtMax][256]
   unsigned *counter = a.counters + cluster::kCounterStride * pl.cluster;
   const int H = a.H, C = 3 * H, B = a.B, NC = a.NC;
   const int tid = threadIdx.x, w = tid / kWave, l = tid % kWave, r16 = l % 16, g = l / 16;
@@ -498,21 +567,14 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_mt(CalClArgs a) {
   const int nitems = 3 * NC;
   const int nT = (a.ntiles - pl.cluster + a.ncl - 1) / a.ncl;  // <= kMtMax (launcher)
   float rfr[IPW][16];
-#pragma unroll
-  for (int it = 0; it < IPW; ++it) {
-    const int item = w * IPW + it, ch = item / 3, gate = item % 3;
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int k = 64 * ch + 16 * g + s;
-      rfr[it][s] = item < nitems && k < H
-                       ? a.R[static_cast<size_t>(k) * C + gate * H + u0 + r16] : 0.0f;
-    }
-  }
+  load_items<IPW>(a, w, g, u0 + r16, rfr);
   const bool fin = tid < 256;
-  const int fl = tid % 64, fq = tid / 64;
-  const int frow = 4 * (fl / 16) + fq, fu = u0 + fl % 16;
-  const float bz = fin ? a.br[fu] : 0.0f, brr = fin ? a.br[H + fu] : 0.0f,
-              bn = fin ? a.br[2 * H + fu] : 0.0f;
+  const int frow = tid / 4 % 16, fu = u0 + tid / 64 * 4 + tid % 4;
+  const int fl = frow / 4 * 16 + fu % 16, fq = frow % 4;
+  // units past H (the last member's, H not a multiple of 16) have zero weights and states
+  const bool unit = fin && fu < H;
+  const float bz = unit ? a.br[a.gz + fu] : 0.0f, brr = unit ? a.br[a.gr + fu] : 0.0f,
+              bn = unit ? a.br[2 * H + fu] : 0.0f;
   float mn[kNStat], mx[kNStat];
 #pragma unroll
   for (int i = 0; i < kNStat; ++i) {
@@ -527,19 +589,20 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_mt(CalClArgs a) {
   for (int k = 0; k < nT; ++k) {
     const int b = (pl.cluster + k * a.ncl) * kCT + frow;
     if (fin) {
-      const float h0 = b < B && a.h0 ? a.h0[static_cast<size_t>(b) * H + fu] : 0.0f;
-      cluster::store_coherent(hxw + b * a.Hpad + fu, __float_as_uint(h0));
-      if (b < B) a.hout[static_cast<size_t>(b) * H + fu] = h0;
+      const float h0 = unit && b < B && a.h0 ? a.h0[static_cast<size_t>(b) * H + fu] : 0.0f;
+      cluster::store_coherent(hxw + hx_index(b, fu, a.Hpad), __float_as_uint(h0));
+      if (unit && b < B) a.hout[static_cast<size_t>(b) * H + fu] = h0;
       hl[k * 256 + tid] = h0;
     }
   }
   float wz = 0.0f, wr = 0.0f, wn = 0.0f;
   auto load_wx = [&](int t, int k) {
     const int b = (pl.cluster + k * a.ncl) * kCT + frow;
-    if (fin && b < B) {
-      const float *wp = a.wx + (static_cast<size_t>(t) * B + b) * C + fu;
-      wz = wp[0];
-      wr = wp[H];
+    if (unit && b < B) {
+      const int tx = a.reverse ? a.T - 1 - t : t;
+      const float *wp = a.wx + (static_cast<size_t>(tx) * B + b) * C + fu;
+      wz = wp[a.gz];
+      wr = wp[a.gr];
       wn = wp[2 * H];
     }
   };
@@ -551,9 +614,9 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_mt(CalClArgs a) {
     for (int k = 0; k < nT; ++k) {
       const int tile = pl.cluster + k * a.ncl;
       const int b = tile * kCT + frow;
-      const bool valid = fin && b < B;
-      const unsigned rowoff = par * plane + static_cast<unsigned>(tile * kCT + r16) * a.Hpad;
-      calib_items<IPW>(rfr, w, l, g, nitems, xr, rowoff, red);
+      const bool valid = unit && b < B;
+      const unsigned tileoff = par * plane + static_cast<unsigned>(tile * kCT) * a.Hpad;
+      calib_items<IPW>(rfr, w, l, nitems, xr, tileoff, red);
       __syncthreads();
       if (fin) {
         const float cz = wz, cr = wr, cn = wn;
@@ -565,7 +628,7 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_mt(CalClArgs a) {
         float rh[3] = {bz, brr, bn};
         for (int ch = 0; ch < NC; ++ch)
 #pragma unroll
-          for (int gate = 0; gate < 3; ++gate) rh[gate] += red[(ch * 3 + gate) * kWave + fl][fq];
+          for (int gate = 0; gate < 3; ++gate) rh[gate] += red[red_index(ch * 3 + gate, fl)][fq];
         const float hold = hl[k * 256 + tid];
         const float zp = cz + rh[0];
         const float rp = cr + rh[1];
@@ -578,7 +641,8 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_mt(CalClArgs a) {
         const float newc = (1.0f - z) * n;
         const float hn = oldc + newc;
         hl[k * 256 + tid] = hn;
-        cluster::store_coherent(hxw + (par ^ 1) * plane + b * a.Hpad + fu, __float_as_uint(hn));
+        cluster::store_coherent(hxw + (par ^ 1) * plane + hx_index(b, fu, a.Hpad),
+                                __float_as_uint(hn));
         if (STATS && valid) {
           observe(rh[0], mn[RXMET_GRU_RH], mx[RXMET_GRU_RH]);
           observe(rh[1], mn[RXMET_GRU_RH], mx[RXMET_GRU_RH]);
@@ -613,7 +677,7 @@ __global__ __launch_bounds__(64 * MAXW) void calib_recurrence_mt(CalClArgs a) {
   }
   if (STATS) {
     __syncthreads();
-    block_stats(mn, mx, kNStat, a.part + static_cast<size_t>(blockIdx.x) * 2 * kNStat);
+    block_stats(mn, mx, kNStat, a.part + static_cast<size_t>(pl.cluster * a.G + pl.member) * 2 * kNStat);
   }
 }
 
@@ -632,7 +696,7 @@ struct CalWorkspace {
     Hpad = (H + 63) / 64 * 64;
     const int64_t M = static_cast<int64_t>(T) * B;
     const int64_t gemm_blocks = (3 * static_cast<int64_t>(H) + 63) / 64 * ((M + 63) / 64);
-    const int64_t rec_blocks = static_cast<int64_t>(ntiles) * (H / 16 > 0 ? H / 16 : 1);
+    const int64_t rec_blocks = static_cast<int64_t>(ntiles) * ((H + 15) / 16);
     nparts = 2 * kNStat * (gemm_blocks > rec_blocks ? gemm_blocks : rec_blocks);
     size_t o = 0;
     ord = o; o += al(sizeof(unsigned) * 2 * kNStat);
@@ -646,56 +710,73 @@ struct CalWorkspace {
   }
 };
 
-// The MFMA form when it applies (H a multiple of 16 up to 1024, the clusters resident);
+// The MFMA form when it applies (H up to 1024, the clusters resident);
 // returns 1 when launched, 0 when the caller must use the per-sequence kernel.
+//
+// The waves of a member: for more than two chunks of K each takes whole chunks, three gates
+// together (IPW 3 and up), so a member reads its tile's h once.  One (chunk, gate) item per wave
+// read it three times, in rows rather than in the operand's order (hx_index): T 200, B 128, I 80,
+// H 256, one direction 729 us, now 560 us (2.8 us per step, of which the fp32 MFMAs take 0.64 and
+// the exchange through the coherence point about 1.4; the rest is the gates' serial chain).  Up
+// to two chunks, items of their own keep all four SIMDs of a CU busy.
+//
+// Both directions of a layer share one launch when that takes fewer tile passes than one launch
+// after the other: a step is mostly latency, which the other direction's step hides (the same
+// layer, both directions: 2 x 729 us before, 563 us in one launch).
+//
+// Sizes that are no multiple of 16 leave units of the last member without weights; before, they
+// took one workgroup per sequence with R read from the L2 at every step (T 200, B 128, I 80,
+// H 250, both directions: a calibration pass of 39975 us, now 1240 us).
 template <bool STATS>
-static int calibrate_mfma(int T, int B, int I, int H, const float *W, const float *R,
-                          const float *bw, const float *br, const float *x, const float *h0,
-                          float *h, float *v, void *workspace, hipStream_t stream) {
-  if (H % 16 != 0 || H > 1024 || std::getenv("RXMET_NO_CLUSTER") != nullptr) return 0;
+static int calibrate_mfma(int ndir, int T, int B, int I, int H, const rxmet_gru_cal_dir *dirs,
+                          hipStream_t stream) {
+  if (H > 1024 || std::getenv("RXMET_NO_CLUSTER") != nullptr) return 0;
   const CalWorkspace ws(T, B, I, H);
   if (2.0 * ws.Bpad * ws.Hpad * 4 >= 2147483648.0) return 0;  // 32-bit exchange offsets
   CalClArgs a{};
   a.T = T; a.B = B; a.H = H;
   a.NC = (H + 63) / 64;
-  // up to 320 units: 4..16 waves of one item (1024 threads, 128 VGPRs); above, 8 waves of
-  // 3..6 items (512 threads, 256 VGPRs: two or three items per wave at 1024 threads spilled)
-  const bool wide = 3 * a.NC > kCMaxW;
-  a.NWG = wide ? 8 : std::max(4, 3 * a.NC);
-  const int ipw = (3 * a.NC + a.NWG - 1) / a.NWG;  // 1, or 3..6 when wide
+  const bool chunks = a.NC > 2;
+  a.NWG = chunks ? std::min(8, std::max(4, a.NC)) : std::max(4, 3 * a.NC);
+  const int ipw = chunks ? std::max(3, (3 * a.NC + a.NWG - 1) / a.NWG) : 1;  // 1, or 3..6
   a.ntiles = ws.ntiles; a.Bpad = ws.Bpad; a.Hpad = ws.Hpad;
-  a.G = H / 16;
+  a.G = (H + 15) / 16;
   using K = const void *;
   const K cl_fns[7] = {nullptr,
-                       reinterpret_cast<K>(&calib_recurrence_cl<STATS, 1>),
+                       reinterpret_cast<K>(&calib_recurrence_cl<STATS, 1, 8>),
                        nullptr,
                        reinterpret_cast<K>(&calib_recurrence_cl<STATS, 3, 8>),
                        reinterpret_cast<K>(&calib_recurrence_cl<STATS, 4, 8>),
                        reinterpret_cast<K>(&calib_recurrence_cl<STATS, 5, 8>),
                        reinterpret_cast<K>(&calib_recurrence_cl<STATS, 6, 8>)};
   const K mt_fns[7] = {nullptr,
-                       reinterpret_cast<K>(&calib_recurrence_mt<STATS, 1>),
+                       reinterpret_cast<K>(&calib_recurrence_mt<STATS, 1, 8>),
                        nullptr,
                        reinterpret_cast<K>(&calib_recurrence_mt<STATS, 3, 8>),
                        reinterpret_cast<K>(&calib_recurrence_mt<STATS, 4, 8>),
                        reinterpret_cast<K>(&calib_recurrence_mt<STATS, 5, 8>),
                        reinterpret_cast<K>(&calib_recurrence_mt<STATS, 6, 8>)};
   const void *fn = cl_fns[ipw];
-  size_t lds = sizeof(v4f) * kWave * 3 * static_cast<size_t>(a.NC);
+  size_t lds = sizeof(v4f) * kRedItem * 3 * static_cast<size_t>(a.NC);
   RXMET_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds)));
   int device = 0, ncu = 0, per_cu = 0;
   RXMET_CHECK_HIP(hipGetDevice(&device));
   RXMET_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
   RXMET_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kWave * a.NWG, lds));
-  int ncl = per_cu * ncu / a.G;
-  if (ncl < 1) return 0;
-  if (ncl > a.ntiles) ncl = a.ntiles;
-  if (ncl >= 8) ncl -= ncl % 8;
-  a.ncl = ncl;
+  const int avail = per_cu * ncu / a.G;
+  if (avail < 1) return 0;
+  auto clusters = [&](int most) {
+    int n = std::min(most, a.ntiles);
+    return n >= 8 ? n - n % 8 : n;
+  };
+  auto passes = [&](int ncl) { return (a.ntiles + ncl - 1) / ncl; };
+  const bool joint = ndir == 2 && avail >= 2 && passes(clusters(avail / 2)) <= kMtMax &&
+                     passes(clusters(avail / 2)) < 2 * passes(clusters(avail));
+  a.ncl = clusters(joint ? avail / 2 : avail);
   // clusters owning several tiles run them all in each step (one barrier per step), when
   // the multi-tile kernel's occupancy allows the same cluster count
-  if (a.ntiles > ncl && (a.ntiles + ncl - 1) / ncl <= kMtMax &&
+  if (passes(a.ncl) > 1 && passes(a.ncl) <= kMtMax &&
       std::getenv("RXMET_CALIB_TILEWISE") == nullptr) {
     const void *mt = mt_fns[ipw];
     const size_t lds_mt = lds + sizeof(float) * kMtMax * 256;
@@ -709,59 +790,75 @@ static int calibrate_mfma(int T, int B, int I, int H, const float *W, const floa
       lds = lds_mt;
     }
   }
-  char *wsb = static_cast<char *>(workspace);
-  unsigned *ord = reinterpret_cast<unsigned *>(wsb + ws.ord);
-  float *wx = reinterpret_cast<float *>(wsb + ws.wx);
-  float *part = reinterpret_cast<float *>(wsb + ws.part);
-  a.hx = reinterpret_cast<float *>(wsb + ws.hx);
-  a.counters = reinterpret_cast<unsigned *>(wsb + ws.sync);
-  a.timeout = reinterpret_cast<int *>(a.counters + cluster::kCounterStride * ncl);
   a.spin_limit = cluster::spin_limit();
   const int C = 3 * H;
   const int M = T * B;
-  {
-    rxmet::prof::Scope ps__("gru_calibrate_input_gemm", stream);
-    const dim3 grid(static_cast<unsigned>((C + calgemm::kBN - 1) / calgemm::kBN),
-                    static_cast<unsigned>((M + calgemm::kBM - 1) / calgemm::kBM));
-    hipLaunchKernelGGL(calib_input_gemm<STATS>, grid, dim3(256), 0, stream, M, I, C, x, W, bw,
-                       wx, part);
+  CalClDirs cd{};
+  for (int k = 0; k < ndir; ++k) {
+    const rxmet_gru_cal_dir &d = dirs[k];
+    char *wsb = static_cast<char *>(d.workspace);
+    unsigned *ord = reinterpret_cast<unsigned *>(wsb + ws.ord);
+    float *wx = reinterpret_cast<float *>(wsb + ws.wx);
+    float *part = reinterpret_cast<float *>(wsb + ws.part);
+    a.hx = reinterpret_cast<float *>(wsb + ws.hx);
+    a.counters = reinterpret_cast<unsigned *>(wsb + ws.sync);
+    a.timeout = reinterpret_cast<int *>(a.counters + cluster::kCounterStride * a.ncl);
+    {
+      rxmet::prof::Scope ps__("gru_calibrate_input_gemm", stream);
+      const dim3 grid(static_cast<unsigned>((C + calgemm::kBN - 1) / calgemm::kBN),
+                      static_cast<unsigned>((M + calgemm::kBM - 1) / calgemm::kBM));
+      hipLaunchKernelGGL((d.torch_layout ? calib_input_gemm<STATS, true>
+                                         : calib_input_gemm<STATS, false>),
+                         grid, dim3(256), 0, stream, M, I, C, d.x, d.W, d.bw, wx, part);
+      RXMET_CHECK_LAUNCH();
+      if (STATS) {
+        hipLaunchKernelGGL(stats_fold<kGemmStat>, dim3(1), dim3(256), 0, stream, part,
+                           static_cast<int>(grid.x * grid.y), 0, ord);
+        RXMET_CHECK_LAUNCH();
+      }
+    }
+    // the exchange buffer's padding columns must read as zero
+    hipLaunchKernelGGL(cluster::zero_words, dim3(cluster::zero_blocks(2 * ws.Bpad * ws.Hpad)),
+                       dim3(256), 0, stream, reinterpret_cast<unsigned *>(a.hx),
+                       2 * ws.Bpad * ws.Hpad);
     RXMET_CHECK_LAUNCH();
-    if (STATS) {
-      hipLaunchKernelGGL(stats_fold<kGemmStat>, dim3(1), dim3(256), 0, stream, part,
-                         static_cast<int>(grid.x * grid.y), 0, ord);
-      RXMET_CHECK_LAUNCH();
-    }
-  }
-  // the exchange buffer's padding columns must read as zero
-  hipLaunchKernelGGL(cluster::zero_words, dim3(cluster::zero_blocks(2 * ws.Bpad * ws.Hpad)),
-                     dim3(256), 0, stream, reinterpret_cast<unsigned *>(a.hx),
-                     2 * ws.Bpad * ws.Hpad);
-  RXMET_CHECK_LAUNCH();
-  hipLaunchKernelGGL(cluster::zero_words, dim3(1), dim3(256), 0, stream, a.counters,
-                     cluster::kCounterStride * ncl + 1);
-  RXMET_CHECK_LAUNCH();
-  a.wx = wx; a.R = R; a.br = br; a.h0 = h0; a.hout = h; a.v = v; a.part = part;
-  void *args[] = {&a};
-  {
+    hipLaunchKernelGGL(cluster::zero_words, dim3(1), dim3(256), 0, stream, a.counters,
+                       cluster::kCounterStride * a.ncl + 1);
+    RXMET_CHECK_LAUNCH();
+    a.wx = wx; a.R = d.R; a.br = d.br; a.h0 = d.h0; a.hout = d.h; a.v = d.v; a.part = part;
+    a.reverse = d.reverse;
+    a.rk = d.torch_layout ? 1 : C;
+    a.rc = d.torch_layout ? H : 1;
+    a.gz = d.torch_layout ? H : 0;
+    a.gr = d.torch_layout ? 0 : H;
+    cd.d[joint ? k : 0] = a;
+    cd.ndir = joint ? 2 : 1;
+    if (joint && k == 0) continue;
     rxmet::prof::Scope ps__("gru_calibrate_forward", stream);
-    RXMET_CHECK_HIP(cluster::launch(fn, dim3(ncl * a.G), dim3(kWave * a.NWG), args,
+    void *args[] = {&cd};
+    RXMET_CHECK_HIP(cluster::launch(fn, dim3(cd.ndir * a.ncl * a.G), dim3(kWave * a.NWG), args,
                                     static_cast<unsigned>(lds), stream));
-    if (STATS) {
-      hipLaunchKernelGGL(stats_fold<kNStat>, dim3(1), dim3(256), 0, stream, part, ncl * a.G, 0,
-                         ord);
+    for (int j = joint ? 0 : k; j <= k; ++j) {
+      const CalClArgs &e = cd.d[joint ? j : 0];
+      if (STATS) {
+        hipLaunchKernelGGL(stats_fold<kNStat>, dim3(1), dim3(256), 0, stream, e.part,
+                           e.ncl * e.G, 0,
+                           reinterpret_cast<unsigned *>(static_cast<char *>(dirs[j].workspace) +
+                                                        ws.ord));
+        RXMET_CHECK_LAUNCH();
+      }
+      // a wait that timed out: the outputs become NaN (the statistics skip non-finite values)
+      cluster::PoisonList pl{};
+      pl.p[pl.count] = e.hout;
+      pl.n[pl.count++] = static_cast<int64_t>(T + 1) * B * H;
+      if (e.v) {
+        pl.p[pl.count] = e.v;
+        pl.n[pl.count++] = static_cast<int64_t>(T) * B * 4 * H;
+      }
+      hipLaunchKernelGGL(cluster::poison_list, dim3(256), dim3(256), 0, stream, e.timeout, pl);
       RXMET_CHECK_LAUNCH();
     }
   }
-  // a wait that timed out: the outputs become NaN (the statistics skip non-finite values)
-  cluster::PoisonList pl{};
-  pl.p[pl.count] = h;
-  pl.n[pl.count++] = static_cast<int64_t>(T + 1) * B * H;
-  if (v) {
-    pl.p[pl.count] = v;
-    pl.n[pl.count++] = static_cast<int64_t>(T) * B * 4 * H;
-  }
-  hipLaunchKernelGGL(cluster::poison_list, dim3(256), dim3(256), 0, stream, a.timeout, pl);
-  RXMET_CHECK_LAUNCH();
   return 1;
 }
 
@@ -813,6 +910,32 @@ __global__ __launch_bounds__(256) void calib_params_part(int I, int H, const flo
   p[3 * C + c] = hr;
 }
 
+// The same for PyTorch's layout, where a channel is one row of W and of R: one wave per channel.
+__global__ __launch_bounds__(256) void calib_params_rows(int I, int H, const float *W,
+                                                         const float *R, const float *bw,
+                                                         const float *br,
+                                                         float *chan /* 4 x (min[C], max[C]) */) {
+  const int C = 3 * H, lane = threadIdx.x % kWave;
+  const int c = blockIdx.x * 4 + threadIdx.x / kWave;
+  if (c >= C) return;
+  const int row = torch_row(c, H);
+  auto range = [&](const float *p, int n, int k) {
+    float lo = FLT_MAX, hi = -FLT_MAX;
+    for (int i = lane; i < n; i += kWave) observe(p[i], lo, hi);
+    lo = wave_min(lo);
+    hi = wave_max(hi);
+    if (lane != 0) return;
+    if (lo > hi) lo = hi = 0.0f;
+    float *mn = chan + static_cast<size_t>(k) * 2 * C, *mx = mn + C;
+    mn[c] = lo < mn[c] ? lo : mn[c];
+    mx[c] = hi > mx[c] ? hi : mx[c];
+  };
+  range(W + static_cast<size_t>(row) * I, I, 0);
+  range(R + static_cast<size_t>(row) * H, H, 1);
+  range(bw + row, 1, 2);
+  range(br + row, 1, 3);
+}
+
 __global__ __launch_bounds__(256) void calib_params_fold(int H, int S, const float *part,
                                                          const float *bw, const float *br,
                                                          float *chan /* 4 x (min[C], max[C]) */) {
@@ -859,38 +982,67 @@ int64_t rxmet_gru_calibrate_workspace_bytes(int32_t T, int32_t B, int32_t I, int
 int rxmet_gru_forward_calibrate(int32_t T, int32_t B, int32_t I, int32_t H, const float *W,
                                 const float *R, const float *bw, const float *br,
                                 const float *x, const float *h0, float *h, float *v,
-                                float *stats, void *workspace, void *stream_) {
+                                float *stats, void *workspace, void *stream) {
+  const rxmet_gru_cal_dir d = {W, R, bw, br, x, h0, h, v, stats, workspace, 0, 0};
+  return rxmet_gru_forward_calibrate_dirs(1, T, B, I, H, &d, stream);
+}
+
+int rxmet_gru_forward_calibrate_dirs(int32_t ndir, int32_t T, int32_t B, int32_t I, int32_t H,
+                                     const rxmet_gru_cal_dir *dirs, void *stream_) {
   clear_error();
+  RXMET_CHECK_ARG((ndir == 1 || ndir == 2) && dirs != nullptr, "one or two directions");
   RXMET_CHECK_ARG(T >= 1 && B >= 1 && I >= 1 && H >= 1, "dimensions must be positive");
   RXMET_CHECK_ARG(H <= 4096, "hidden_size above 4096 is not supported by the calibration pass");
-  RXMET_CHECK_ARG(W && R && bw && br && x && h && stats && workspace, "required pointer is null");
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
-  unsigned *ord = static_cast<unsigned *>(workspace);  // the workspace's first region
-  hipLaunchKernelGGL(stats_init, dim3(1), dim3(64), 0, stream, ord);
-  RXMET_CHECK_LAUNCH();
-  const int mf = calibrate_mfma<true>(T, B, I, H, W, R, bw, br, x, h0, h, v, workspace, stream);
-  if (mf < 0) return mf;
-  if (mf == 0) {
-    const size_t lds = sizeof(float) * 8 * static_cast<size_t>(H);
-    if (lds > 64 * 1024)
-      RXMET_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&calib_forward<true>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          static_cast<int>(lds)));
-    rxmet::prof::Scope ps__("gru_calibrate_forward", stream);
-    hipLaunchKernelGGL(calib_forward<true>, dim3(B), dim3(kCalThreads), lds, stream, T, B, I, H, W, R, bw,
-                       br, x, h0, h, v, ord);
+  for (int k = 0; k < ndir; ++k) {
+    const rxmet_gru_cal_dir &d = dirs[k];
+    RXMET_CHECK_ARG(d.W && d.R && d.bw && d.br && d.x && d.h && d.stats && d.workspace,
+                    "required pointer is null");
+    RXMET_CHECK_ARG((d.reverse == 0 || d.reverse == 1) &&
+                        (d.torch_layout == 0 || d.torch_layout == 1),
+                    "reverse and torch_layout must be 0 or 1");
   }
-  RXMET_CHECK_LAUNCH();
-  hipLaunchKernelGGL(stats_merge, dim3(1), dim3(64), 0, stream, ord, stats);
-  RXMET_CHECK_LAUNCH();
-  const CalWorkspace cw(T, B, I, H);
-  float *prm = reinterpret_cast<float *>(static_cast<char *>(workspace) + cw.prm);
-  hipLaunchKernelGGL(calib_params_part, dim3((3 * H + 63) / 64, cw.prm_slabs), dim3(256), 0,
-                     stream, I, H, W, R, prm);
-  RXMET_CHECK_LAUNCH();
-  hipLaunchKernelGGL(calib_params_fold, dim3((3 * H + 255) / 256), dim3(256), 0, stream, H,
-                     cw.prm_slabs, prm, bw, br, stats + 2 * kNStat);
-  RXMET_CHECK_LAUNCH();
+  RXMET_CHECK_ARG(ndir == 1 || dirs[0].workspace != dirs[1].workspace,
+                  "each direction needs a workspace of its own");
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  for (int k = 0; k < ndir; ++k) {  // the workspace's first region
+    hipLaunchKernelGGL(stats_init, dim3(1), dim3(64), 0, stream,
+                       static_cast<unsigned *>(dirs[k].workspace));
+    RXMET_CHECK_LAUNCH();
+  }
+  const int mf = calibrate_mfma<true>(ndir, T, B, I, H, dirs, stream);
+  if (mf < 0) return mf;
+  for (int k = 0; k < ndir; ++k) {
+    const rxmet_gru_cal_dir &d = dirs[k];
+    unsigned *ord = static_cast<unsigned *>(d.workspace);
+    if (mf == 0) {
+      const size_t lds = sizeof(float) * 8 * static_cast<size_t>(H);
+      const auto fn = d.torch_layout ? calib_forward<true, true> : calib_forward<true, false>;
+      if (lds > 64 * 1024)
+        RXMET_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            static_cast<int>(lds)));
+      rxmet::prof::Scope ps__("gru_calibrate_forward", stream);
+      hipLaunchKernelGGL(fn, dim3(B), dim3(kCalThreads), lds, stream, T, B, I, H,
+                         d.W, d.R, d.bw, d.br, d.x, d.h0, d.h, d.v, ord, d.reverse);
+    }
+    RXMET_CHECK_LAUNCH();
+    hipLaunchKernelGGL(stats_merge, dim3(1), dim3(64), 0, stream, ord, d.stats);
+    RXMET_CHECK_LAUNCH();
+    if (d.torch_layout) {
+      hipLaunchKernelGGL(calib_params_rows, dim3((3 * H + 3) / 4), dim3(256), 0, stream, I, H, d.W,
+                         d.R, d.bw, d.br, d.stats + 2 * kNStat);
+      RXMET_CHECK_LAUNCH();
+      continue;
+    }
+    const CalWorkspace cw(T, B, I, H);
+    float *prm = reinterpret_cast<float *>(static_cast<char *>(d.workspace) + cw.prm);
+    hipLaunchKernelGGL(calib_params_part, dim3((3 * H + 63) / 64, cw.prm_slabs), dim3(256), 0,
+                       stream, I, H, d.W, d.R, prm);
+    RXMET_CHECK_LAUNCH();
+    hipLaunchKernelGGL(calib_params_fold, dim3((3 * H + 255) / 256), dim3(256), 0, stream, H,
+                       cw.prm_slabs, prm, d.bw, d.br, d.stats + 2 * kNStat);
+    RXMET_CHECK_LAUNCH();
+  }
   return 0;
 }
 
@@ -905,11 +1057,11 @@ int rxmet_gru_forward_fp(int32_t is_training, int32_t T, int32_t B, int32_t I, i
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   const size_t lds = sizeof(float) * 8 * static_cast<size_t>(H);
   if (lds > 64 * 1024)
-    RXMET_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&calib_forward<false>),
+    RXMET_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&calib_forward<false, false>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize,
                                         static_cast<int>(lds)));
-  hipLaunchKernelGGL(calib_forward<false>, dim3(B), dim3(kCalThreads), lds, stream, T, B, I, H, W,
-                     R, bw, br, x, h0, h, is_training ? v : nullptr, nullptr);
+  hipLaunchKernelGGL((calib_forward<false, false>), dim3(B), dim3(kCalThreads), lds, stream, T, B, I, H, W,
+                     R, bw, br, x, h0, h, is_training ? v : nullptr, nullptr, 0);
   RXMET_CHECK_LAUNCH();
   return 0;
 }

@@ -353,30 +353,51 @@ def forward_calibrate(is_training, time_steps, batch_size, input_size, hidden_si
                       hist_collectors=None):
     """Float GRU forward + MinMax statistics merged into ``quant_ranges``
     (forwardWithCalibrationGPU, src/gru_interface.cc:930-1024).  Returns (h, v)."""
+    return forward_calibrate_dirs(is_training, time_steps, batch_size, input_size, hidden_size,
+                                  [(W, R, bw, br, x, h0, quant_ranges, False)], calib_method)[0]
+
+
+def forward_calibrate_dirs(is_training, time_steps, batch_size, input_size, hidden_size, dirs,
+                           calib_method="minmax", torch_layout=False):
+    """forward_calibrate of one direction or of both directions of a layer
+    (rxmet_gru_forward_calibrate_dirs): ``dirs`` holds (W, R, bw, br, x, h0, quant_ranges,
+    reverse) per direction; a reverse direction walks x [T, B, I] backwards and returns (h, v) in
+    its own order of steps.  ``torch_layout``: W, R, bw, br as PyTorch's weight_ih [3H, I],
+    weight_hh [3H, H] and biases, gate order (r, z, n)."""
     if calib_method != "minmax":
         raise NotImplementedError("only MinMax calibration is implemented on MI355X")
-    for n, t in (("W", W), ("R", R), ("bw", bw), ("br", br), ("x", x)):
-        _check_f32_cuda(n, t)
-    dev = x.device
     T, B, I, H = time_steps, batch_size, input_size, hidden_size
-    h = torch.empty((T + 1, B, H), dtype=torch.float32, device=dev)
-    # gate values are only materialised when asked for (is_training); the ranges never need them
-    v = torch.empty((T, B, 4 * H) if is_training else (0,), dtype=torch.float32, device=dev)
-    if quant_ranges is None:
-        raise RuntimeError("forward_calibrate needs quant_ranges (MinMax statistics)")
-    if quant_ranges.hidden_ != H:
-        raise RuntimeError("quant_ranges hidden size does not match hidden_size")
-    if tuple(x.shape) != (T, B, I) or tuple(W.shape) != (I, 3 * H) or tuple(R.shape) != (H, 3 * H):
-        raise RuntimeError("x/W/R shapes do not match (time_steps, batch_size, input_size, "
-                           "hidden_size)")
-    if quant_ranges.stats.device != dev:
-        quant_ranges.stats = quant_ranges.stats.to(dev)
-    h0p = h0.data_ptr() if (h0 is not None and h0.numel() > 0) else None
-    ws = _ws(_rx.load().rxmet_gru_calibrate_workspace_bytes(T, B, I, H), dev)
-    _rx.call("rxmet_gru_forward_calibrate", T, B, I, H, W.data_ptr(), R.data_ptr(), bw.data_ptr(),
-             br.data_ptr(), x.data_ptr(), h0p, h.data_ptr(), v.data_ptr() if is_training else None,
-             quant_ranges.stats.data_ptr(), ws.data_ptr(), _stream(dev))
-    return h, v
+    arr = (A.CalDir * len(dirs))()
+    outs, keep = [], []
+    for k, (W, R, bw, br, x, h0, quant_ranges, reverse) in enumerate(dirs):
+        for n, t in (("W", W), ("R", R), ("bw", bw), ("br", br), ("x", x)):
+            _check_f32_cuda(n, t)
+        dev = x.device
+        h = torch.empty((T + 1, B, H), dtype=torch.float32, device=dev)
+        # gate values are only materialised when asked for (is_training); the ranges never need
+        # them
+        v = torch.empty((T, B, 4 * H) if is_training else (0,), dtype=torch.float32, device=dev)
+        if quant_ranges is None:
+            raise RuntimeError("forward_calibrate needs quant_ranges (MinMax statistics)")
+        if quant_ranges.hidden_ != H:
+            raise RuntimeError("quant_ranges hidden size does not match hidden_size")
+        shapes = ((3 * H, I), (3 * H, H)) if torch_layout else ((I, 3 * H), (H, 3 * H))
+        if tuple(x.shape) != (T, B, I) or (tuple(W.shape), tuple(R.shape)) != shapes:
+            raise RuntimeError("x/W/R shapes do not match (time_steps, batch_size, input_size, "
+                               "hidden_size)")
+        if quant_ranges.stats.device != dev:
+            quant_ranges.stats = quant_ranges.stats.to(dev)
+        h0p = h0.data_ptr() if (h0 is not None and h0.numel() > 0) else None
+        ws = _ws(_rx.load().rxmet_gru_calibrate_workspace_bytes(T, B, I, H), dev)
+        arr[k] = A.CalDir(W.data_ptr(), R.data_ptr(), bw.data_ptr(), br.data_ptr(), x.data_ptr(),
+                          h0p, h.data_ptr(), v.data_ptr() if is_training else None,
+                          quant_ranges.stats.data_ptr(), ws.data_ptr(), int(bool(reverse)),
+                          int(bool(torch_layout)))
+        outs.append((h, v))
+        keep.append(ws)
+    _rx.call("rxmet_gru_forward_calibrate_dirs", len(dirs), T, B, I, H, arr,
+             _stream(dirs[0][4].device))
+    return outs
 
 
 def forward_fp(is_training, time_steps, batch_size, input_size, hidden_size, W, R, bw, br, x,

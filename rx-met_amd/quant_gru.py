@@ -1161,6 +1161,15 @@ class QuantGRU(nn.Module):
             getattr(self, "bias_ih_l0" + sfx) if self.bias else None,
             getattr(self, "bias_hh_l0" + sfx) if self.bias else None, self.hidden_size, device)
 
+    def _torch_weights(self, reverse: bool, device):
+        """(weight_ih, weight_hh, bias_ih, bias_hh) as they are, missing biases as zeros."""
+        sfx = "_reverse" if reverse else ""
+        names = ("weight_ih_l0", "weight_hh_l0") + (("bias_ih_l0", "bias_hh_l0") if self.bias
+                                                    else ())
+        w = [ensure_cuda_float32(getattr(self, n + sfx).detach(), device).contiguous()
+             for n in names]
+        return (*w, *([_zeros(3 * self.hidden_size, device)] * 2 if not self.bias else ()))
+
     def _parse_initial_state(self, hx, batch_size: int):
         """hx [D, B, H] -> (h0_forward, h0_reverse) (quant_gru.py:1372-1400)."""
         if hx is None:
@@ -1188,32 +1197,28 @@ class QuantGRU(nn.Module):
         empty = torch.empty(0, device=device)
         if self.quant_ranges is None:
             self.quant_ranges = gru_ops.GRUQuantizationRanges(H, device=device)
-        W, R, bw, br = self._direction_weights(False, device)
+        if self.bidirectional and self.quant_ranges_reverse is None:
+            self.quant_ranges_reverse = gru_ops.GRUQuantizationRanges(H, device=device)
+        dirs = []
+        for reverse, h0, ranges in ((False, h0f, self.quant_ranges),
+                                    (True, h0r, self.quant_ranges_reverse if self.bidirectional
+                                     else None))[:self.num_directions]:
+            dirs.append((*self._torch_weights(reverse, device), input,
+                         ensure_cuda_float32(h0, device).contiguous() if h0 is not None else empty,
+                         ranges, reverse))
         with torch.no_grad():
             # the gate values (v) are not needed for the ranges: not materialised
-            h, _ = gru_ops.forward_calibrate(
-                is_training=False, time_steps=T, batch_size=B, input_size=I, hidden_size=H,
-                W=W, R=R, bw=bw, br=br, x=input,
-                h0=ensure_cuda_float32(h0f, device).contiguous() if h0f is not None else empty,
-                calib_method=self.calibration_method, bitwidth_config=self._bitwidth_config,
-                quant_ranges=self.quant_ranges)
-        out_f, hn_f = h[1:], h[-1:]
-        out_r = hn_r = None
-        if self.bidirectional:
-            if self.quant_ranges_reverse is None:
-                self.quant_ranges_reverse = gru_ops.GRUQuantizationRanges(H, device=device)
-            W, R, bw, br = self._direction_weights(True, device)
-            with torch.no_grad():
-                h_r, _ = gru_ops.forward_calibrate(
-                    is_training=False, time_steps=T, batch_size=B, input_size=I, hidden_size=H,
-                    W=W, R=R, bw=bw, br=br, x=input.flip(0).contiguous(),
-                    h0=ensure_cuda_float32(h0r, device).contiguous() if h0r is not None else empty,
-                    calib_method=self.calibration_method, bitwidth_config=self._bitwidth_config,
-                    quant_ranges=self.quant_ranges_reverse)
-            out_r, hn_r = h_r[1:].flip(0), h_r[-1:]
+            outs = gru_ops.forward_calibrate_dirs(False, T, B, I, H, dirs,
+                                                  self.calibration_method, torch_layout=True)
         if (not self._quant_params_locked) or self.quant_params is None:
             self._quant_params_dirty = True
-        return self._combine_bidirectional_outputs(out_f, hn_f, out_r, hn_r)
+        h = outs[0][0]
+        if self.bidirectional and H % 4 == 0:  # flips and concatenations in one launch
+            return gru_ops.bidir_assemble(h, outs[1][0], False)
+        out_r = hn_r = None
+        if self.bidirectional:
+            out_r, hn_r = outs[1][0][1:].flip(0), outs[1][0][-1:]
+        return self._combine_bidirectional_outputs(h[1:], h[-1:], out_r, hn_r)
 
     def _resolve_quant_params(self):
         """Dirty / lock handling before a quantised forward (quant_gru.py:2218-2242)."""

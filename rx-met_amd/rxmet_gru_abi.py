@@ -105,6 +105,13 @@ class GradView(ctypes.Structure):
                 ("col0", ctypes.c_int32), ("reverse", ctypes.c_int32), ("g_hn", _p)]
 
 
+class CalDir(ctypes.Structure):
+    """rxmet_gru_cal_dir: one direction of a calibration pass."""
+    _fields_ = [(n, _p) for n in ("W", "R", "bw", "br", "x", "h0", "h", "v", "stats",
+                                  "workspace")] + [("reverse", ctypes.c_int32),
+                                                   ("torch_layout", ctypes.c_int32)]
+
+
 _SIGS = {
     "rxmet_gru_make_params": (ctypes.c_int, [ctypes.POINTER(GruRanges), ctypes.POINTER(GruConfig),
                                              ctypes.POINTER(GruQParams)]),
@@ -120,6 +127,7 @@ _SIGS = {
     "rxmet_gru_forward_quant_dirs": (ctypes.c_int, [_i32] * 6 + [ctypes.POINTER(FwdDir), _p]),
     "rxmet_gru_backward_quant_dirs": (ctypes.c_int, [_i32] * 5 + [ctypes.POINTER(BwdDir), _p]),
     "rxmet_gru_forward_calibrate": (ctypes.c_int, [_i32, _i32, _i32, _i32] + [_p] * 9 + [_p, _p]),
+    "rxmet_gru_forward_calibrate_dirs": (ctypes.c_int, [_i32] * 5 + [ctypes.POINTER(CalDir), _p]),
     "rxmet_gru_forward_fp": (ctypes.c_int, [_i32] * 5 + [_p] * 8 + [_p]),
     "rxmet_gru_forward_quant_dirs_x": (ctypes.c_int, [_i32] * 6 + [ctypes.POINTER(FwdDir), _p, _p]),
     "rxmet_gru_backward_quant_dirs_x": (ctypes.c_int, [_i32] * 5 + [ctypes.POINTER(BwdDir), _i32, _p]),
