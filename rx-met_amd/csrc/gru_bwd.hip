@@ -24,8 +24,8 @@
 //                    planes against the resident int8 R_q, recombined in fp64; error <= 2^-22
 //                    of the row maximum per term).  Both fuse the STE pointwise (all mask
 //                    families), write dp/dq for the GEMMs and keep fp64 bias partials;
-//                    For H > 256 the stepped path (bwd_step_point + a K-split dh GEMM per
-//                    step) replaces both;
+//                    For H > 256 the stepped path (gru_bwd_step.h: one launch per step)
+//                    replaces both;
 //   3. bias fold   : per-workgroup fp64 partials summed in a fixed order (deterministic);
 //   4. dx, dW, dR  : bf16-MFMA GEMMs with the gradients split exactly into three bf16 terms
 //                    (wgrad_gemm.h; dW and dR split over the long T*B reduction and summed in
@@ -326,7 +326,6 @@ __global__ __launch_bounds__(512) void bwd_recurrence(BwdArgs a) {
 constexpr int kBwMaxKS2 = 12;  // 3H <= 768
 constexpr int kBwMaxKB = (kBwMaxKS2 + 1) / 2;  // 32-channel MFMA blocks per wave
 constexpr int kMaxHStepped = 1024;
-constexpr int kStepMaxSplit = 8;  // K splits of the stepped dh GEMM
 
 struct BwdClArgs {
   int ncl, G, UT, ntiles, Bpad, KP, ndir;  // KP = 3H padded to a multiple of 64
@@ -965,85 +964,13 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
   }
 }
 
-// ---------------------------------------------------------------------------------
-// stepped backward (H > 256): per step one pointwise launch and one dh GEMM launch
-// ---------------------------------------------------------------------------------
-// Step t: every (sequence, unit) takes dh_c = dhl + gsum of step t + 1 (zero at t = T - 1),
-// stores dp, dq and dhl = z dh_t, and adds its bias terms to the partial sums of its 16-row
-// chunk (bias_partial[chunk][2][3H], each slot owned by one thread, steps in order); the dh
-// GEMM gsum = (dq_t scale_R) R_q^T then runs on the split-bf16 MFMA product (wgrad::nt).
-__global__ __launch_bounds__(256) void bwd_step_point(BwdArgs a, int t, int S,
-                                                      const float *__restrict__ gsum,
-                                                      float *__restrict__ dhl) {
-  // block: 64 units x 4 row groups; a 16-row chunk per block (row group y takes rows y + 4 i)
-  __shared__ double red[3][6][64];
-  const int H = a.H, C = 3 * H, B = a.B;
-  const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;
-  const int j = blockIdx.x * 64 + tx, chunk = blockIdx.y;
-  const bool on = j < H;
-  const int jj = on ? j : 0;
-  const BwdMasks mk = {mask_ref(a.h_m, a.v), mask_ref(a.gout_m, a.v), mask_ref(a.gin_m, a.v),
-                       mask_ref(a.hh_m, a.v), mask_ref(a.ih_m, a.v)};
-  double sb[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  const uint32_t BH = static_cast<uint32_t>(B) * H;
-  const size_t split = static_cast<size_t>(B) * H;
-#pragma unroll
-  for (int i = 0; i < kBTile / 4; ++i) {
-    const int b = chunk * kBTile + ty + 4 * i;
-    if (!on || b >= B) continue;
-    const uint32_t o = static_cast<uint32_t>(b) * H + jj;
-    float dhc = 0.0f;
-    if (t != a.T - 1) {
-      float gs = gsum[o];
-      for (int z = 1; z < S; ++z) gs += gsum[z * split + o];
-      dhc = dhl[o] + gs;
-    }
-    float cur[kBwRaw];
-    bwd_load_step(a, mk, t, b, jj, cur);
-    float dpv[3], dqv[3];
-    dhl[o] = bwd_point(cur, dhc, dpv, dqv);
-    const uint32_t m = 3u * static_cast<uint32_t>(t) * BH + 3u * static_cast<uint32_t>(b) * H + jj;
-#pragma unroll
-    for (int g = 0; g < 3; ++g) {
-      a.dp[m + g * H] = dpv[g];
-      a.dq[m + g * H] = dqv[g];
-      sb[g] += static_cast<double>(dpv[g]);
-      sb[3 + g] += static_cast<double>(dqv[g]);
-    }
-  }
-  if (ty > 0)
-#pragma unroll
-    for (int e = 0; e < 6; ++e) red[ty - 1][e][tx] = sb[e];
-  __syncthreads();
-  if (ty == 0 && on) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int e = 0; e < 6; ++e) sb[e] += red[k][e][tx];
-    double *p = a.bias_partial + static_cast<size_t>(chunk) * 2 * C;
-    const bool first = t == a.T - 1;
-#pragma unroll
-    for (int g = 0; g < 3; ++g) {
-      const double mw = a.bw_m ? static_cast<double>(a.bw_m[g * H + j]) : 1.0;
-      const double mr = a.br_m ? static_cast<double>(a.br_m[g * H + j]) : 1.0;
-      p[g * H + j] = (first ? 0.0 : p[g * H + j]) + sb[g] * mw;
-      p[C + g * H + j] = (first ? 0.0 : p[C + g * H + j]) + sb[3 + g] * mr;
-    }
-  }
-}
+}  // namespace gru
+}  // namespace rxmet
 
-// dh0 = (dhl + gsum of step 0) * h0 mask (gsum: S K-split parts summed in order).
-__global__ __launch_bounds__(256) void bwd_step_dh0(int64_t n, int S, const float *__restrict__ dhl,
-                                                    const float *__restrict__ gsum,
-                                                    const uint8_t *__restrict__ h0_m,
-                                                    float *__restrict__ dh0) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float gs = gsum[i];
-  for (int z = 1; z < S; ++z) gs += gsum[z * n + i];
-  const float v = dhl[i] + gs;
-  dh0[i] = h0_m ? v * static_cast<float>(h0_m[i]) : v;
-}
+#include "gru_bwd_step.h"
+
+namespace rxmet {
+namespace gru {
 
 __global__ __launch_bounds__(256) void zero_floats(int64_t n, float *p) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
@@ -1104,7 +1031,7 @@ size_t bwd_lds_bytes(int KS2) {
 }
 
 struct BwdWorkspace {
-  size_t dp, dq, xt, ht, wb, qsc, rfrag, rowsum, effr, effw, bias, part, xch, rt, sync, rb, gsum,
+  size_t dp, dq, xt, ht, wb, qsc, rfrag, rowsum, effr, effw, bias, part, xch, rt, sync, rb, dqp,
       dhl, total;
   int Mp, S_w[2], kper_w[2], S_r[2], kper_r[2];  // K splits by number of B planes
   int Cp;                                         // 3H rounded up to a multiple of 32
@@ -1145,10 +1072,10 @@ struct BwdWorkspace {
     xch = o; o += al(sizeof(float) * 2 * Bpad * KS2 * 64);
     rt = o; o += al(sizeof(uint4) * 2 * ((H + 15) / 16) * 4 * ((KS2 + 1) / 2) * 64);
     sync = o; o += al(sizeof(unsigned) * cluster::kCounterStride * (2 * nwg + 2));  // clusters of both directions
-    // stepped recurrence: R codes as bf16 planes [H][Cp], the dh GEMM output, dhl
+    // stepped recurrence: R codes as bf16 fragments (two planes), the terms of dq of two steps, dhl
     Cp = static_cast<int>((C + 31) / 32 * 32);
-    rb = o; o += al(sizeof(__bf16) * 2 * H * static_cast<size_t>(Cp));
-    gsum = o; o += al(sizeof(float) * kStepMaxSplit * static_cast<size_t>(B) * H);
+    rb = o; o += al(sizeof(__bf16) * 2 * step_rplane(H));
+    dqp = o; o += al(sizeof(__bf16) * 2 * step_terms(B, H));
     dhl = o; o += al(sizeof(float) * static_cast<size_t>(B) * H);
     total = o;
   }
@@ -1401,43 +1328,63 @@ static int backward_recurrence_clustered(BwdPlan *plans, int ndir, int T, int B,
   return 1;
 }
 
-// The stepped recurrence of one direction (any H): 2 T launches.
-static int backward_recurrence_stepped(BwdPlan &plan, int T, int B, int I, int H,
+// 64 x 64 tiles when they give half of the CUs a workgroup.  Training steps (T 50, I 256) with
+// tiles of 64 | of 32: B 512, H 1024 (128 tiles of 64) 4445 | 4589 us; with 64 of them, B 256,
+// H 1024 3182 | 2476, B 512, H 512 2496 | 1926, B 256, H 512, two directions 2740 | 2166.
+static bool step_big(int ndir, int B, int H, int ncu) {
+  return static_cast<int64_t>(ndir) * ((B + 63) / 64) * ((H + 63) / 64) >= ncu / 2;
+}
+
+// The stepped recurrence of every direction: T + 1 launches (gru_bwd_step.h).
+static int backward_recurrence_stepped(BwdPlan *plans, int ndir, int T, int B, int I, int H,
                                        hipStream_t stream) {
-  const int C = 3 * H;
   const BwdWorkspace ws(T, B, I, H);
-  const rxmet_gru_bwd_dir &d = *plan.d;
-  const Bounds br = bounds_of(d.params->chan_bits[RXMET_GRU_R], d.params->chan_unsigned[RXMET_GRU_R]);
-  const int npr = wgrad::planes_for(br.lo, br.hi, 0.0);
-  __bf16 *rb = reinterpret_cast<__bf16 *>(plan.wsb + ws.rb);
-  float *gsum = reinterpret_cast<float *>(plan.wsb + ws.gsum);
-  float *dhl = reinterpret_cast<float *>(plan.wsb + ws.dhl);
-  // R_q [H][3H] as is: rows are the units (N), the channels c are K
-  if (int rc = wgrad::codes_t(d.R_q, C, nullptr, C, H, 1, C, 0.0f, 1.0f, npr, rb, ws.Cp,
-                              static_cast<int64_t>(H) * ws.Cp, stream))
-    return rc;
-  rxmet::prof::Scope ps__("gru_bwd_recurrence", stream);
-  const dim3 grid((H + 63) / 64, (B + kBTile - 1) / kBTile);
-  wgrad::NtArgs na;
-  na.lda = C;
-  na.kscale = plan.ba.eff_r;
-  na.Bt = rb; na.ldb = ws.Cp; na.bplane = static_cast<int64_t>(H) * ws.Cp;
-  na.M = B; na.N = H; na.K = C; na.out = gsum; na.ldo = H;
-  // K splits so that the dh GEMM fills the GPU (the parts are summed in order by the next
-  // step's pointwise)
-  wgrad::nt_plan(B, H, C, kStepMaxSplit, &na.ksplit, &na.kper);
-  na.out_split = static_cast<int64_t>(B) * H;
-  const int S = na.ksplit;
-  for (int t = T - 1; t >= 0; --t) {
-    hipLaunchKernelGGL(bwd_step_point, grid, dim3(256), 0, stream, plan.ba, t, S, gsum, dhl);
-    RXMET_CHECK_LAUNCH();
-    na.A = plan.ba.dq + static_cast<size_t>(t) * B * C;
-    if (int rc = wgrad::nt(na, npr, stream)) return rc;
+  int device = 0, ncu = 0;
+  RXMET_CHECK_HIP(hipGetDevice(&device));
+  RXMET_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
+  StepArgs sa[2];
+  StepShape sh{};
+  sh.ndir = ndir;
+  sh.Hk = (H + 31) / 32 * 32;
+  sh.KC = 3 * sh.Hk / 32;
+  sh.MT = (B + 63) / 64 * 4;
+  const bool big = step_big(ndir, B, H, ncu), codes = plans[0].ba.vc != nullptr;
+  sh.KR = step_kr(sh.KC);
+  sh.rbplane = step_rplane(H);
+  int npb = 1;
+  for (int k = 0; k < ndir; ++k) {
+    const rxmet_gru_qparams &qp = *plans[k].d->params;
+    const Bounds br = bounds_of(qp.chan_bits[RXMET_GRU_R], qp.chan_unsigned[RXMET_GRU_R]);
+    npb = std::max(npb, wgrad::planes_for(br.lo, br.hi, 0.0));
   }
-  const int64_t n = static_cast<int64_t>(B) * H;
-  hipLaunchKernelGGL(bwd_step_dh0, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream,
-                     n, S, dhl, gsum, plan.ba.h0_m, plan.ba.dh0);
-  RXMET_CHECK_LAUNCH();
+  for (int k = 0; k < ndir; ++k) {
+    sa[k].a = plans[k].ba;
+    sa[k].rb = reinterpret_cast<const __bf16 *>(plans[k].wsb + ws.rb);
+    sa[k].dqp = reinterpret_cast<__bf16 *>(plans[k].wsb + ws.dqp);
+    sa[k].dhl = reinterpret_cast<float *>(plans[k].wsb + ws.dhl);
+    hipLaunchKernelGGL((npb == 1 ? pack_rt_step<1> : pack_rt_step<2>), dim3(H / 16 * sh.KR), dim3(64),
+                       0, stream, H, sh.Hk, sh.KR, plans[k].d->R_q,
+                       reinterpret_cast<__bf16 *>(plans[k].wsb + ws.rb), sh.rbplane);
+    RXMET_CHECK_LAUNCH();
+  }
+  if (ndir == 1) sa[1] = sa[0];
+  rxmet::prof::Scope ps__("gru_bwd_recurrence", stream);
+  const int bt = big ? 64 : 32;
+  sh.tm = (B + bt - 1) / bt;
+  sh.tn = (H + bt - 1) / bt;
+  using Fn = void (*)(StepArgs, StepArgs, StepShape);
+  const Fn fns[2][2][2] = {{{&bwd_step<32, 1, false>, &bwd_step<32, 1, true>},
+                            {&bwd_step<32, 2, false>, &bwd_step<32, 2, true>}},
+                           {{&bwd_step<64, 1, false>, &bwd_step<64, 1, true>},
+                            {&bwd_step<64, 2, false>, &bwd_step<64, 2, true>}}};
+  const Fn fn = fns[big][npb - 1][codes];
+  const unsigned grid = (static_cast<unsigned>(ndir * sh.tm * sh.tn) + 7) / 8 * 8;
+  for (int t = T - 1; t >= -1; --t) {
+    sh.t = t;
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(512), 0, stream, sa[0], sa[1], sh);
+    RXMET_CHECK_LAUNCH();
+  }
+  for (int k = 0; k < ndir; ++k) plans[k].nbias = sh.tm;
   return 0;
 }
 
@@ -1540,7 +1487,7 @@ static int backward_dirs(int ndir, int T, int B, int I, int H, const rxmet_gru_b
       return rc;
   for (int k = 0; k < ndir; ++k) plans[k].torch_layout = torch_layout;
   // H > 256 (more R values than the clustered and per-tile kernels keep in registers), or
-  // RXMET_BWD_STEPPED set: one pointwise and one GEMM launch per step
+  // RXMET_BWD_STEPPED set: one launch per step
   const bool stepped = H > 256 || std::getenv("RXMET_BWD_STEPPED") != nullptr;
   int *timeout_flag = nullptr;
   int rc = stepped ? 0 : backward_recurrence_resident(plans, ndir, T, B, I, H, stream);
@@ -1552,11 +1499,12 @@ static int backward_dirs(int ndir, int T, int B, int I, int H, const rxmet_gru_b
   for (int k = 0; k < ndir; ++k)
     wide_r = wide_r || dirs[k].params->chan_bits[RXMET_GRU_R] > 8 ||
              dirs[k].params->chan_unsigned[RXMET_GRU_R] != 0;
-  if (rc == 0)
+  if (rc == 0 && (stepped || wide_r || codes)) {
+    if (int r = backward_recurrence_stepped(plans, ndir, T, B, I, H, stream)) return r;
+  } else if (rc == 0) {
     for (int k = 0; k < ndir; ++k)
-      if (int r = (stepped || wide_r || codes) ? backward_recurrence_stepped(plans[k], T, B, I, H, stream)
-                                      : backward_recurrence_tiles(plans[k], B, H, stream))
-        return r;
+      if (int r = backward_recurrence_tiles(plans[k], B, H, stream)) return r;
+  }
   for (int k = 0; k < ndir; ++k)
     if (int r = backward_epilogue(T, B, I, H, plans[k], stream)) return r;
   if (timeout_flag != nullptr) {
