@@ -938,6 +938,7 @@ __global__ __launch_bounds__(256) void step_point(RecArgs a, StepParams p, int t
 constexpr int kClMaxKPerWave = 4;  // K-steps per wave: H <= 1024
 constexpr int kHsMax = 4;          // 16-byte h chunks staged per thread and step
 constexpr int kStageMinH = 512;    // H from which the h tile is staged in LDS
+constexpr size_t kMaxLds = 160 * 1024;
 
 struct ClArgs {
   int ncl, G, UT, ntiles, Bpad, ndir;  // clusters walk (direction, batch tile) pairs
@@ -969,12 +970,18 @@ __device__ __forceinline__ unsigned hx_offset(int b, int j, int KS) {
   return ((static_cast<unsigned>(b / kTileB) * KS + j / 64) * kTileB + b % kTileB) * 64 + j % 64;
 }
 
-// One (direction, batch tile) pair of the clustered recurrence, run by one member.
-template <int NPL, bool STAGE>
-__device__ __forceinline__ void recurrence_cl_pair(const RecArgs &a, const StepParams &p,
-                                                   const ClArgs &cl, int tile, int member,
-                                                   unsigned *counter, unsigned &epoch,
-                                                   bool &alive) {
+// One direction's batch tiles tile, tile + tstep, .. (nT of them) of the clustered recurrence, run
+// by one member.  MT = false: one tile.  MT: several, all of them in every step, so that the
+// members meet once per step rather than once per tile and step, and the next tile's h codes and
+// input linear are on their way while a tile is computed; a tile's previous h waits in LDS.
+// Measured (T 50, B 1024, H 1024, 16-bit h: eight tiles per cluster): 2065 us one tile after the
+// other, 1882 us; bound by the chain of one tile (two meetings of the waves in LDS, the piecewise
+// gates of one element per thread), which leaves the matrix cores idle for 90% of it.
+template <int NPL, bool STAGE, bool MT>
+__device__ __forceinline__ void recurrence_cl_tiles(const RecArgs &a, const StepParams &p,
+                                                    const ClArgs &cl, int tile0, int tstep, int nT,
+                                                    int member, unsigned *counter,
+                                                    unsigned &epoch, bool &alive) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int H = a.H, C = 3 * H, B = a.B, KS = a.KS;
   float *lut_f = reinterpret_cast<float *>(smem);               // 3 * 16 * 3 (thr, qb, c)
@@ -989,6 +996,8 @@ __device__ __forceinline__ void recurrence_cl_pair(const RecArgs &a, const StepP
   int8_t *hs = reinterpret_cast<int8_t *>(sb + 16 * 13 * UW);
   // gate tables, [3][kGateTabMax] (16-byte aligned: H is a multiple of 16)
   int *gtab = reinterpret_cast<int *>(hs + NPL * kTileB * (H + 16));
+  // MT: previous h per tile and thread (MT has no gate tables in the staged form)
+  float *hl = reinterpret_cast<float *>(gtab + (cl.gate_tab ? 3 * kGateTabMax : 0));
   const int tid = threadIdx.x, w = tid / 64, l = tid % 64;
   const int utl = w / 4, kq = w % 4;
   const int ut = member * cl.UT + utl;
@@ -1031,215 +1040,254 @@ __device__ __forceinline__ void recurrence_cl_pair(const RecArgs &a, const StepP
   const auto xr = cluster::buffer_rsrc(a.hx, 2u * NPL * plane_stride);
   v4i *myred = red + (static_cast<size_t>(utl) * 4 + kq) * 3 * NPL * 64;
 
-  {
-    const int b0 = tile * kTileB, b = b0 + nr;
-    const bool valid = b < B;
-    float hold = valid ? a.h0codes[static_cast<size_t>(b) * H + j] : p.zp_h;
+  int4 hv[STAGE ? kHsMax : 1];  // staged: this thread's chunks of a tile's h codes
+  v4i hx_fr[STAGE ? 1 : kClMaxKPerWave][NPL];  // unstaged: the wave's fragments of them
+  // issue the loads of a tile's h codes of the step whose planes start at byte hin
+  auto load_h = [&](int tile, unsigned hin) {
+    if constexpr (STAGE) {
+      // the tile's h codes are read from the exchange buffer once per workgroup (16-byte
+      // coherent loads, all issued before any is stored) into LDS, where the unit tiles
+      // share them (at H >= 512; at smaller H the extra barrier costs more than it saves)
+      // 16-byte chunk e -> plane p, K-step s, row r, chunk c of the step: the tile's blocks
+      // in order, 1 KB per 64 threads; chunks past H (a partial last step) are not stored
+      const int n = NPL * KS * 64, nt = blockDim.x;
+      const unsigned tb = hin + static_cast<unsigned>(tile) * KS * 1024;
+#pragma unroll
+      for (int i = 0; i < kHsMax; ++i) {
+        const int e0 = tid + nt * i, e = e0 < n ? e0 : 0;
+        const int q = e / (KS * 64), s = (e / 64) % KS;
+        hv[i] = cluster::load_coherent16(xr, tb + q * plane_stride + s * 1024 + 16 * (e % 64));
+      }
+    } else {
+      // lane l: row l % 16, units 16 (l / 16) .. + 15 of K-step kq + 4 i
+      const unsigned hrow = hin + static_cast<unsigned>(tile) * KS * 1024 + 64 * (l % 16) + 16 * (l / 16);
+#pragma unroll
+      for (int i = 0; i < kClMaxKPerWave; ++i)
+#pragma unroll
+        for (int q = 0; q < NPL; ++q)
+          if (kq + 4 * i < KS) {
+            const int4 v = cluster::load_coherent16(xr, hrow + q * plane_stride + 1024 * (kq + 4 * i));
+            hx_fr[i][q] = v4i{v.x, v.y, v.z, v.w};
+          }
+    }
+  };
+  float gi_next[3];
+  auto load_gih = [&](int tile, int t) {
+    const int b = tile * kTileB + nr;
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+      gi_next[g] = b < B ? a.gih[(static_cast<size_t>(t) * B + b) * C + g * H + j] : 0.0f;
+  };
+  // one step of one tile up to its published and staged outputs; `ahead` issues the next loads
+  // once the tile's own are used
+  PointOut o;
+  auto compute = [&](int tile, int par, float &hold, auto ahead) {
+    const int b = tile * kTileB + nr;
+    int8_t *hout = a.hx + (par ^ 1) * NPL * plane_stride;
+    const float gih[3] = {gi_next[0], gi_next[1], gi_next[2]};
+    // partial recurrent sums over this wave's K-steps
+    v4i acc[3][NPL];
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+#pragma unroll
+      for (int q = 0; q < NPL; ++q) acc[g][q] = v4i{0, 0, 0, 0};
+    v4i hfr[kClMaxKPerWave][NPL];
+    if constexpr (STAGE) {
+      const int rs = H + 16, n = NPL * KS * 64, nt = blockDim.x;
+#pragma unroll
+      for (int i = 0; i < kHsMax; ++i) {
+        const int e = tid + nt * i;
+        const int q = e / (KS * 64), s = (e / 64) % KS, r = (e / 4) % kTileB, c = 4 * s + e % 4;
+        if (e < n && 16 * c < H)
+          *reinterpret_cast<int4 *>(hs + (q * kTileB + r) * rs + 16 * c) = hv[i];
+      }
+      __syncthreads();
+      ahead();
+      const int8_t *hrow = hs + (l % 16) * rs + 16 * (l / 16);
+#pragma unroll
+      for (int i = 0; i < kClMaxKPerWave; ++i)
+#pragma unroll
+        for (int q = 0; q < NPL; ++q)
+          if (kq + 4 * i < KS)
+            hfr[i][q] = *reinterpret_cast<const v4i *>(hrow + q * kTileB * rs + 64 * (kq + 4 * i));
+    } else {
+#pragma unroll
+      for (int i = 0; i < kClMaxKPerWave; ++i)
+#pragma unroll
+        for (int q = 0; q < NPL; ++q) hfr[i][q] = hx_fr[i][q];
+    }
+#pragma unroll
+    for (int i = 0; i < kClMaxKPerWave; ++i)
+      if (kq + 4 * i < KS) {
+#pragma unroll
+        for (int g = 0; g < 3; ++g)
+#pragma unroll
+          for (int q = 0; q < NPL; ++q) acc[g][q] = mfma_i8(hfr[i][q], rfr[i][g], acc[g][q]);
+      }
+    if constexpr (!STAGE) ahead();
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+#pragma unroll
+      for (int q = 0; q < NPL; ++q) myred[(g * NPL + q) * 64 + l] = acc[g][q];
+    __syncthreads();
+    int sum[3][NPL];
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+#pragma unroll
+      for (int q = 0; q < NPL; ++q) {
+        int v = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int *src = reinterpret_cast<const int *>(
+              red + ((static_cast<size_t>(utl) * 4 + k) * 3 * NPL + g * NPL + q) * 64 + l);
+          v += src[kq];
+        }
+        sum[g][q] = v;
+      }
+    // pointwise update of (row b, unit j)
+    float gh3[3];
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+      gh3[g] = recombine_rh<NPL>(a.wide_acc, sum[g][0], sum[g][NPL - 1], plane_off, a.h_offset,
+                                 cst[g][6]);
+    o = gru_point(gih, gh3, cst, p, lut_f, lut_n, hold, tab);
+    const float h2 = o.h;
+    hold = h2;
     {
-      const int hcv = static_cast<int>(hold - a.h_offset);
-      unsigned char *dst = reinterpret_cast<unsigned char *>(a.hx) + hx_offset(b, j, KS);
+      const int hcv = static_cast<int>(h2 - a.h_offset);
+      unsigned char *dst = reinterpret_cast<unsigned char *>(hout) + hx_offset(b, j, KS);
 #pragma unroll
       for (int q = 0; q < NPL; ++q)
         cluster::store_bytes_coherent(dst + q * plane_stride,
                                       NPL == 1 ? hcv : (q == 0 ? (hcv & 255) - 128 : hcv >> 8));
     }
-    float gi_next[3];
-    auto load_gih = [&](int t) {
+    if (a.wide_out) {
+      float *f = sf + nr * 5 * UW + jj;
+      f[0] = (h2 - p.zp_h) * p.eff_h;
+      if (a.training && a.vc) {
+        // codes in their blocked layout (codes_row), over the mask bytes: the member's UT
+        // v-code blocks, then its UT mask-bit blocks
+        uint16_t *c16 = reinterpret_cast<uint16_t *>(sb) + (utl * 16 + nr) * 64 + l % 16;
+        c16[0] = static_cast<uint16_t>(code_u16(o.z, p.zout.lo));
+        c16[16] = static_cast<uint16_t>(code_u16(o.r, p.rout.lo));
+        c16[32] = static_cast<uint16_t>(code_u16(o.n, p.nout.lo));
+        c16[48] = static_cast<uint16_t>(code_u16(o.rh_n, p.rh.lo));
+        reinterpret_cast<uint16_t *>(sb)[1024 * cl.UT + (utl * 16 + nr) * 16 + l % 16] =
+            static_cast<uint16_t>(code_mask_bits(o));
+      } else if (a.training) {
+        f[UW] = (o.z - p.zp_zout) * p.eff_zout;
+        f[2 * UW] = (o.r - p.zp_rout) * p.eff_rout;
+        f[3 * UW] = (o.n - p.zp_nout) * p.eff_nout;
+        f[4 * UW] = (o.rh_n - p.zp_rh) * p.eff_rh;
+        uint8_t *m8 = sb + nr * 13 * UW + jj;
 #pragma unroll
-      for (int g = 0; g < 3; ++g)
-        gi_next[g] = valid ? a.gih[(static_cast<size_t>(t) * B + b) * C + g * H + j] : 0.0f;
-    };
-    load_gih(0);
-    alive = cluster::sync(counter, ++epoch * cl.G, cl.timeout, cl.spin_limit);
+        for (int g = 0; g < 3; ++g) {
+          m8[g * UW] = o.k_ih[g];
+          m8[(3 + g) * UW] = o.k_hh[g];
+          m8[(6 + g) * UW] = o.k_gi[g];
+          m8[(9 + g) * UW] = o.k_go[g];
+        }
+        m8[12 * UW] = o.k_h;
+      }
+    }
+  };
+  // the staged outputs of one step of one tile to memory
+  auto flush = [&](int t, int tile) {
+    const int b0 = tile * kTileB, b = b0 + nr;
+    if (a.wide_out) {
+      // 16-byte rows of the staged outputs, spread over the whole workgroup (each array
+      // in a loop of its own: a pointer chosen per lane would put the arguments in scratch)
+      const size_t stepH = static_cast<size_t>(t) * B * H;
+      const int nthr = blockDim.x, fq = UW / 4;
+      for (int c = tid; c < 16 * fq; c += nthr) {
+        const int row = c / fq, q = c % fq, bb = b0 + row;
+        if (bb < B)
+          *reinterpret_cast<float4 *>(a.hout + stepH + static_cast<size_t>(B + bb) * H +
+                                      member * UW + 4 * q) =
+              *reinterpret_cast<const float4 *>(sf + row * 5 * UW + 4 * q);
+      }
+      if (a.training && a.vc) {
+        // one contiguous run of UT blocks per array (the batch tile's padding rows too)
+        const uint4 *c16 = reinterpret_cast<const uint4 *>(sb);
+        const size_t blk = (static_cast<size_t>(t) * cl.ntiles + tile) * (H / 16) +
+                           static_cast<size_t>(member) * cl.UT;
+        uint4 *dv = reinterpret_cast<uint4 *>(a.vc + blk * 1024);
+        uint4 *dm = reinterpret_cast<uint4 *>(a.mb + blk * 256);
+        const int nv = 128 * cl.UT, nm = 32 * cl.UT;  // 16-byte chunks
+        for (int c = (tid + nthr - (16 * fq) % nthr) % nthr; c < nv; c += nthr) dv[c] = c16[c];
+        for (int c = (tid + nthr - (16 * fq + nv) % nthr) % nthr; c < nm; c += nthr)
+          dm[c] = c16[nv + c];
+      } else if (a.training) {
+        for (int c = (tid + nthr - (16 * fq) % nthr) % nthr; c < 64 * fq; c += nthr) {
+          const int row = c / (4 * fq), fld = (c / fq) % 4, q = c % fq, bb = b0 + row;
+          if (bb < B)
+            *reinterpret_cast<float4 *>(a.v + 4 * (stepH + static_cast<size_t>(bb) * H) +
+                                        fld * H + member * UW + 4 * q) =
+                *reinterpret_cast<const float4 *>(sf + (row * 5 + 1 + fld) * UW + 4 * q);
+        }
+        const int bq = UW / 16;
+        flush_masks(a.ih_m, 0, 3, sb, UW, bq, b0, B, H, member, stepH, (tid + 0 * 48 * bq) % nthr, nthr);
+        flush_masks(a.hh_m, 3, 3, sb, UW, bq, b0, B, H, member, stepH, (tid + nthr - (48 * bq) % nthr) % nthr, nthr);
+        flush_masks(a.gin_m, 6, 3, sb, UW, bq, b0, B, H, member, stepH, (tid + nthr - (96 * bq) % nthr) % nthr, nthr);
+        flush_masks(a.gout_m, 9, 3, sb, UW, bq, b0, B, H, member, stepH, (tid + nthr - (144 * bq) % nthr) % nthr, nthr);
+        flush_masks(a.h_m, 12, 1, sb, UW, bq, b0, B, H, member, stepH, (tid + nthr - (192 * bq) % nthr) % nthr, nthr);
+      }
+    } else if (b < B) {
+      store_point(a, p, t, b, j, o);
+    }
+  };
 
-    for (int t = 0; t < a.T && alive; ++t) {
-      const int par = t & 1;
-      const unsigned hin = par * NPL * plane_stride;  // byte offset of the step's planes
-      int8_t *hout = a.hx + (par ^ 1) * NPL * plane_stride;
-      float gih[3] = {gi_next[0], gi_next[1], gi_next[2]};
-      // partial recurrent sums over this wave's K-steps
-      v4i acc[3][NPL];
+  // the initial state of every tile
+  float hold = 0.0f;
+  for (int k = 0; k < nT; ++k) {
+    const int b = (tile0 + k * tstep) * kTileB + nr;
+    hold = b < B ? a.h0codes[static_cast<size_t>(b) * H + j] : p.zp_h;
+    const int hcv = static_cast<int>(hold - a.h_offset);
+    unsigned char *dst = reinterpret_cast<unsigned char *>(a.hx) + hx_offset(b, j, KS);
 #pragma unroll
-      for (int g = 0; g < 3; ++g)
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) acc[g][q] = v4i{0, 0, 0, 0};
-      if constexpr (STAGE) {
-        // the tile's h codes are read from the exchange buffer once per workgroup (16-byte
-        // coherent loads, all issued before any is stored) into LDS, where the unit tiles
-        // share them (at H >= 512; at smaller H the extra barrier costs more than it saves)
-        // 16-byte chunk e -> plane p, K-step s, row r, chunk c of the step: the tile's blocks
-        // in order, 1 KB per 64 threads; chunks past H (a partial last step) are not stored
-        const int rs = H + 16, n = NPL * KS * 64, nt = blockDim.x;
-        const unsigned tb = hin + static_cast<unsigned>(tile) * KS * 1024;
-        int4 hv[kHsMax];
-#pragma unroll
-        for (int i = 0; i < kHsMax; ++i) {
-          const int e0 = tid + nt * i, e = e0 < n ? e0 : 0;
-          const int p = e / (KS * 64), s = (e / 64) % KS;
-          hv[i] = cluster::load_coherent16(xr, tb + p * plane_stride + s * 1024 + 16 * (e % 64));
-        }
-#pragma unroll
-        for (int i = 0; i < kHsMax; ++i) {
-          const int e = tid + nt * i;
-          const int p = e / (KS * 64), s = (e / 64) % KS, r = (e / 4) % kTileB, c = 4 * s + e % 4;
-          if (e < n && 16 * c < H)
-            *reinterpret_cast<int4 *>(hs + (p * kTileB + r) * rs + 16 * c) = hv[i];
-        }
-        __syncthreads();
-        const int8_t *hrow = hs + (l % 16) * rs + 16 * (l / 16);
-        v4i hfr[kClMaxKPerWave][NPL];
-#pragma unroll
-        for (int i = 0; i < kClMaxKPerWave; ++i)
-#pragma unroll
-          for (int q = 0; q < NPL; ++q)
-            if (kq + 4 * i < KS)
-              hfr[i][q] = *reinterpret_cast<const v4i *>(hrow + q * kTileB * rs + 64 * (kq + 4 * i));
-#pragma unroll
-        for (int i = 0; i < kClMaxKPerWave; ++i)
-          if (kq + 4 * i < KS) {
-#pragma unroll
-            for (int g = 0; g < 3; ++g)
-#pragma unroll
-              for (int q = 0; q < NPL; ++q) acc[g][q] = mfma_i8(hfr[i][q], rfr[i][g], acc[g][q]);
+    for (int q = 0; q < NPL; ++q)
+      cluster::store_bytes_coherent(dst + q * plane_stride,
+                                    NPL == 1 ? hcv : (q == 0 ? (hcv & 255) - 128 : hcv >> 8));
+    if (MT) hl[k * blockDim.x + tid] = hold;
+  }
+  load_gih(tile0, 0);
+  alive = cluster::sync(counter, ++epoch * cl.G, cl.timeout, cl.spin_limit);
+  for (int t = 0; t < a.T && alive; ++t) {
+    const int par = t & 1;
+    const unsigned hin = par * NPL * plane_stride;  // byte offset of the step's planes
+    load_h(tile0, hin);
+    if constexpr (MT) {
+      for (int k = 0; k < nT; ++k) {
+        const int tile = tile0 + k * tstep;
+        hold = hl[k * blockDim.x + tid];
+        compute(tile, par, hold, [&]() {
+          if (k + 1 < nT) {
+            load_h(tile + tstep, hin);
+            load_gih(tile + tstep, t);
+          } else if (t + 1 < a.T) {
+            load_gih(tile0, t + 1);
           }
-      } else {
-        // lane l: row l % 16, units 16 (l / 16) .. + 15 of K-step kq + 4 i
-        const unsigned hrow = hin + static_cast<unsigned>(tile) * KS * 1024 + 64 * (l % 16) + 16 * (l / 16);
-        v4i hfr[kClMaxKPerWave][NPL];
-#pragma unroll
-        for (int i = 0; i < kClMaxKPerWave; ++i)
-#pragma unroll
-          for (int q = 0; q < NPL; ++q)
-            if (kq + 4 * i < KS) {
-              const int4 v = cluster::load_coherent16(xr, hrow + q * plane_stride + 1024 * (kq + 4 * i));
-              hfr[i][q] = v4i{v.x, v.y, v.z, v.w};
-            }
-#pragma unroll
-        for (int i = 0; i < kClMaxKPerWave; ++i)
-          if (kq + 4 * i < KS) {
-#pragma unroll
-            for (int g = 0; g < 3; ++g)
-#pragma unroll
-              for (int q = 0; q < NPL; ++q) acc[g][q] = mfma_i8(hfr[i][q], rfr[i][g], acc[g][q]);
-          }
+        });
+        hl[k * blockDim.x + tid] = hold;
+        __syncthreads();  // the staged outputs are whole; the partial sums are read
+        flush(t, tile);  // the next tile stages its own after at least one more barrier
       }
-#pragma unroll
-      for (int g = 0; g < 3; ++g)
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) myred[(g * NPL + q) * 64 + l] = acc[g][q];
-      __syncthreads();
-      int sum[3][NPL];
-#pragma unroll
-      for (int g = 0; g < 3; ++g)
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) {
-          int v = 0;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int *src = reinterpret_cast<const int *>(
-                red + ((static_cast<size_t>(utl) * 4 + k) * 3 * NPL + g * NPL + q) * 64 + l);
-            v += src[kq];
-          }
-          sum[g][q] = v;
-        }
-      // pointwise update of (row b, unit j)
-      float gh3[3];
-#pragma unroll
-      for (int g = 0; g < 3; ++g)
-        gh3[g] = recombine_rh<NPL>(a.wide_acc, sum[g][0], sum[g][NPL - 1], plane_off, a.h_offset,
-                                   cst[g][6]);
-      const PointOut o = gru_point(gih, gh3, cst, p, lut_f, lut_n, hold, tab);
-      const float h2 = o.h;
-      hold = h2;
-      {
-        const int hcv = static_cast<int>(h2 - a.h_offset);
-        unsigned char *dst = reinterpret_cast<unsigned char *>(hout) + hx_offset(b, j, KS);
-#pragma unroll
-        for (int q = 0; q < NPL; ++q)
-          cluster::store_bytes_coherent(dst + q * plane_stride,
-                                        NPL == 1 ? hcv : (q == 0 ? (hcv & 255) - 128 : hcv >> 8));
-      }
-      if (a.wide_out) {
-        float *f = sf + nr * 5 * UW + jj;
-        f[0] = (h2 - p.zp_h) * p.eff_h;
-        if (a.training && a.vc) {
-          // codes in their blocked layout (codes_row), over the mask bytes: the member's UT
-          // v-code blocks, then its UT mask-bit blocks
-          uint16_t *c16 = reinterpret_cast<uint16_t *>(sb) + (utl * 16 + nr) * 64 + l % 16;
-          c16[0] = static_cast<uint16_t>(code_u16(o.z, p.zout.lo));
-          c16[16] = static_cast<uint16_t>(code_u16(o.r, p.rout.lo));
-          c16[32] = static_cast<uint16_t>(code_u16(o.n, p.nout.lo));
-          c16[48] = static_cast<uint16_t>(code_u16(o.rh_n, p.rh.lo));
-          reinterpret_cast<uint16_t *>(sb)[1024 * cl.UT + (utl * 16 + nr) * 16 + l % 16] =
-              static_cast<uint16_t>(code_mask_bits(o));
-        } else if (a.training) {
-          f[UW] = (o.z - p.zp_zout) * p.eff_zout;
-          f[2 * UW] = (o.r - p.zp_rout) * p.eff_rout;
-          f[3 * UW] = (o.n - p.zp_nout) * p.eff_nout;
-          f[4 * UW] = (o.rh_n - p.zp_rh) * p.eff_rh;
-          uint8_t *m8 = sb + nr * 13 * UW + jj;
-#pragma unroll
-          for (int g = 0; g < 3; ++g) {
-            m8[g * UW] = o.k_ih[g];
-            m8[(3 + g) * UW] = o.k_hh[g];
-            m8[(6 + g) * UW] = o.k_gi[g];
-            m8[(9 + g) * UW] = o.k_go[g];
-          }
-          m8[12 * UW] = o.k_h;
-        }
-      }
+      cluster::arrive(counter);
+      ++epoch;
+    } else {
+      compute(tile0, par, hold, []() {});
       // the other members only read the h codes: arrive now, store the outputs while waiting
       // (the arrival's workgroup barrier also publishes the staged outputs)
       cluster::arrive(counter);
       ++epoch;
-      if (a.wide_out) {
-        // 16-byte rows of the staged outputs, spread over the whole workgroup (each array
-        // in a loop of its own: a pointer chosen per lane would put the arguments in scratch)
-        const size_t stepH = static_cast<size_t>(t) * B * H;
-        const int nthr = blockDim.x, fq = UW / 4;
-        for (int c = tid; c < 16 * fq; c += nthr) {
-          const int row = c / fq, q = c % fq, bb = b0 + row;
-          if (bb < B)
-            *reinterpret_cast<float4 *>(a.hout + stepH + static_cast<size_t>(B + bb) * H +
-                                        member * UW + 4 * q) =
-                *reinterpret_cast<const float4 *>(sf + row * 5 * UW + 4 * q);
-        }
-        if (a.training && a.vc) {
-          // one contiguous run of UT blocks per array (the batch tile's padding rows too)
-          const uint4 *c16 = reinterpret_cast<const uint4 *>(sb);
-          const size_t blk = (static_cast<size_t>(t) * cl.ntiles + tile) * (H / 16) +
-                             static_cast<size_t>(member) * cl.UT;
-          uint4 *dv = reinterpret_cast<uint4 *>(a.vc + blk * 1024);
-          uint4 *dm = reinterpret_cast<uint4 *>(a.mb + blk * 256);
-          const int nv = 128 * cl.UT, nm = 32 * cl.UT;  // 16-byte chunks
-          for (int c = (tid + nthr - (16 * fq) % nthr) % nthr; c < nv; c += nthr) dv[c] = c16[c];
-          for (int c = (tid + nthr - (16 * fq + nv) % nthr) % nthr; c < nm; c += nthr)
-            dm[c] = c16[nv + c];
-        } else if (a.training) {
-          for (int c = (tid + nthr - (16 * fq) % nthr) % nthr; c < 64 * fq; c += nthr) {
-            const int row = c / (4 * fq), fld = (c / fq) % 4, q = c % fq, bb = b0 + row;
-            if (bb < B)
-              *reinterpret_cast<float4 *>(a.v + 4 * (stepH + static_cast<size_t>(bb) * H) +
-                                          fld * H + member * UW + 4 * q) =
-                  *reinterpret_cast<const float4 *>(sf + (row * 5 + 1 + fld) * UW + 4 * q);
-          }
-          const int bq = UW / 16;
-          flush_masks(a.ih_m, 0, 3, sb, UW, bq, b0, B, H, member, stepH, (tid + 0 * 48 * bq) % nthr, nthr);
-          flush_masks(a.hh_m, 3, 3, sb, UW, bq, b0, B, H, member, stepH, (tid + nthr - (48 * bq) % nthr) % nthr, nthr);
-          flush_masks(a.gin_m, 6, 3, sb, UW, bq, b0, B, H, member, stepH, (tid + nthr - (96 * bq) % nthr) % nthr, nthr);
-          flush_masks(a.gout_m, 9, 3, sb, UW, bq, b0, B, H, member, stepH, (tid + nthr - (144 * bq) % nthr) % nthr, nthr);
-          flush_masks(a.h_m, 12, 1, sb, UW, bq, b0, B, H, member, stepH, (tid + nthr - (192 * bq) % nthr) % nthr, nthr);
-        }
-      } else if (valid) {
-        store_point(a, p, t, b, j, o);
-      }
-      if (t + 1 < a.T) load_gih(t + 1);
-      alive = cluster::wait(counter, epoch * cl.G, cl.timeout, cl.spin_limit);
+      flush(t, tile0);
+      if (t + 1 < a.T) load_gih(tile0, t + 1);
     }
+    alive = cluster::wait(counter, epoch * cl.G, cl.timeout, cl.spin_limit);
   }
 }
 
-template <int NPL, bool STAGE>
+template <int NPL, bool STAGE, bool MT>
 __global__ __launch_bounds__(512) void recurrence_cl(RecArgs a0, RecArgs a1,
                                                      const StepParams *__restrict__ ps,
                                                      ClArgs cl) {
@@ -1247,13 +1295,21 @@ __global__ __launch_bounds__(512) void recurrence_cl(RecArgs a0, RecArgs a1,
   unsigned *counter = cl.counters + cluster::kCounterStride * pl.cluster;
   unsigned epoch = 0;
   bool alive = true;
+  if constexpr (MT) {
+    // each direction's tiles over its share of the clusters
+    const int per = cl.ncl / cl.ndir, d = pl.cluster / per, c = pl.cluster % per;
+    recurrence_cl_tiles<NPL, STAGE, true>(d == 0 ? a0 : a1, ps[d], cl, c, per,
+                                          (cl.ntiles - c + per - 1) / per, pl.member, counter,
+                                          epoch, alive);
+    return;
+  }
   for (int pair = pl.cluster; pair < cl.ndir * cl.ntiles && alive; pair += cl.ncl) {
     const int d = pair / cl.ntiles, tile = pair % cl.ntiles;
     // the previous pair's readers of the LUT and the partial-sum buffer are done
     __syncthreads();
     // one copy of the step code for both directions (d is uniform across the workgroup)
-    recurrence_cl_pair<NPL, STAGE>(d == 0 ? a0 : a1, ps[d], cl, tile, pl.member, counter, epoch,
-                                   alive);
+    recurrence_cl_tiles<NPL, STAGE, false>(d == 0 ? a0 : a1, ps[d], cl, tile, 0, 1, pl.member,
+                                           counter, epoch, alive);
   }
 }
 
@@ -1624,11 +1680,17 @@ static int forward_recurrence_clustered(FwdPlan *plans, int ndir, int T, int B, 
       if (!(g.hi - g.lo < static_cast<float>(kGateTabMax))) cl.gate_tab = 0;
   }
   const bool tab = cl.gate_tab != 0;
-  const void *fn = npl == 1 ? (stage ? reinterpret_cast<const void *>(&recurrence_cl<1, true>)
-                                     : reinterpret_cast<const void *>(&recurrence_cl<1, false>))
-                            : (stage ? reinterpret_cast<const void *>(&recurrence_cl<2, true>)
-                                     : reinterpret_cast<const void *>(&recurrence_cl<2, false>));
-  const size_t lds_cl = recurrence_cl_lds_bytes(chosen, npl, H, tab);
+  using K = const void *;
+  const K fns[2][2][2] = {{{reinterpret_cast<K>(&recurrence_cl<1, false, false>),
+                            reinterpret_cast<K>(&recurrence_cl<1, false, true>)},
+                           {reinterpret_cast<K>(&recurrence_cl<1, true, false>),
+                            reinterpret_cast<K>(&recurrence_cl<1, true, true>)}},
+                          {{reinterpret_cast<K>(&recurrence_cl<2, false, false>),
+                            reinterpret_cast<K>(&recurrence_cl<2, false, true>)},
+                           {reinterpret_cast<K>(&recurrence_cl<2, true, false>),
+                            reinterpret_cast<K>(&recurrence_cl<2, true, true>)}}};
+  const void *fn = fns[npl - 1][stage][0];
+  size_t lds_cl = recurrence_cl_lds_bytes(chosen, npl, H, tab);
   RXMET_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds_cl)));
   int per_cu = 0;
@@ -1637,6 +1699,23 @@ static int forward_recurrence_clustered(FwdPlan *plans, int ndir, int T, int B, 
   if (ncl < 1) return 0;
   if (ncl > pairs) ncl = pairs;
   if (ncl >= 8) ncl -= ncl % 8;
+  // clusters that own several tiles run them all in each step, when the clusters divide evenly
+  // over the directions and the tiles' previous h fit in LDS beside the rest
+  if (pairs > ncl && ncl % ndir == 0) {
+    const int per = ncl / ndir, nT = (cl.ntiles + per - 1) / per;
+    const size_t lds_mt = lds_cl + sizeof(float) * static_cast<size_t>(nT) * 256 * chosen;
+    if (lds_mt <= kMaxLds) {
+      const void *mt = fns[npl - 1][stage][1];
+      int per_cu_mt = 0;
+      RXMET_CHECK_HIP(hipFuncSetAttribute(mt, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          static_cast<int>(lds_mt)));
+      RXMET_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_mt, mt, 256 * chosen, lds_mt));
+      if (per_cu_mt * ncu / cl.G >= ncl) {
+        fn = mt;
+        lds_cl = lds_mt;
+      }
+    }
+  }
   cl.UT = chosen;
   cl.stage_h = stage ? 1 : 0;
   cl.ncl = ncl;
