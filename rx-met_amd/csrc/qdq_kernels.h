@@ -767,6 +767,8 @@ struct ColGeo {
 // runs: block b handles chunks sp, sp + splits, ... (`passes` of them, sp = b % splits) of
 // run b / splits, so that the blocks in flight read adjacent memory; one partial per block,
 // or (kFold, direct) the block's encoding gradients.
+// vec: a chunk moves whole vectors between the first and the last 16-byte boundary inside it, and
+// the up to E - 1 elements before and after them one by one (launch_decomp's rule).
 template <class W>
 __global__ __launch_bounds__(kThreads) void k_runs(W w, Geo geo, int64_t splits, int passes,
                                                    int vec,
@@ -784,7 +786,13 @@ __global__ __launch_bounds__(kThreads) void k_runs(W w, Geo geo, int64_t splits,
     if (beg >= geo.inner) break;
     const int64_t end = min(geo.inner, beg + kChunk);
     if (vec) {
-      w.vec_block(e, (rb + beg) / W::E, static_cast<int>((end - beg) / W::E), acc);
+      const int64_t a = rb + beg, z = rb + end;
+      const int64_t va = (a + W::E - 1) / W::E, vz = z / W::E;
+      w.vec_block(e, va, static_cast<int>(vz - va), acc);  // none when a chunk's end has vz < va
+      const int64_t h = min(va * W::E, z), t = max(vz * W::E, h);
+      const int nh = static_cast<int>(h - a), nt = static_cast<int>(z - t);
+      if (static_cast<int>(threadIdx.x) < nh) w.elem(e, a + threadIdx.x, acc);
+      if (static_cast<int>(threadIdx.x) < nt) w.elem(e, t + threadIdx.x, acc);
     } else {
       const int n = static_cast<int>(end - beg);
       for (int i = threadIdx.x; i < n; i += kThreads) w.elem(e, rb + beg + i, acc);
@@ -909,9 +917,15 @@ static int launch_decomp(const Plan &pl, const W &w, bool aligned, void *partial
   using Acc = typename W::Acc;
   Acc *part = static_cast<Acc *>(partial);
   const bool vec = aligned && pl.inner % W::E == 0;
+  // 16-bit elements go as vectors in runs of any length: one by one, 2 bytes an access, a wavefront
+  // moves a line per access and the passes are bound by their number ([3001, 4099] bf16 as one run,
+  // backward 34.9 us and forward 19.8, as vectors 22.4 and 14.6; in runs of a row 32.4 and 21.7,
+  // 24.3 and 16.4).  4-byte elements fill two lines: rows of 4099 fp32 take 29.3 us one by one and
+  // 31.6 as vectors that no row starts on a boundary of.
+  const bool edges = aligned && (vec || W::E >= 8);
   if (pl.kind == KIND_RUNS) {
     hipLaunchKernelGGL(k_runs<W>, dim3(static_cast<unsigned>(pl.runs * pl.splits)),
-                       dim3(kThreads), 0, s, w, pl.geo, pl.splits, pl.passes, int(vec), part);
+                       dim3(kThreads), 0, s, w, pl.geo, pl.splits, pl.passes, int(edges), part);
   } else if (pl.kind == KIND_SEGS) {
     const int64_t nv = vec ? pl.inner / W::E : pl.inner;
     int shift = 0;

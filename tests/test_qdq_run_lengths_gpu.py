@@ -1,0 +1,57 @@
+"""Long runs whose length is no multiple of a 16-byte vector: whole vectors between the boundaries
+inside a chunk, single elements around them.  The same tensors one element off alignment go element
+by element, so outputs and input gradients are equal bit for bit, and the encoding gradients (fp64
+sums in another order, rounded to fp32 once) within one unit in the last place."""
+import sys
+from pathlib import Path
+
+import pytest
+import torch
+
+sys.path.insert(0, str(Path(__file__).resolve().parents[1] / "rx-met_amd"))
+import mi355x_qdq as Q  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def cuda():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    return torch.device("cuda:0")
+
+
+def _off(t):
+    """The same values, starting one element past an aligned address."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    buf[1:] = t.flatten()
+    return buf[1:].view(t.shape)
+
+
+# runs below one vector, at a chunk's edge (4096 fp32, 8192 16-bit, 2048 fp64 elements) and across
+# several, every misalignment of a row's start, and two chunks per workgroup (over 2048 chunks)
+@pytest.mark.parametrize("shape,enc", [
+    ((1,), ()), ((7,), ()), ((9,), ()), ((4095,), ()), ((4097,), ()), ((8191,), ()), ((8193,), ()),
+    ((9, 1025), (9, 1)), ((17, 4099), (17, 1)), ((9, 8185), (9, 1)), ((1030, 8197), (1030, 1)),
+    ((4099, 4101), ())])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+def test_vectors_and_edges_equal_single_elements(cuda, shape, enc, dtype):
+    gen = torch.Generator(device=cuda).manual_seed(len(shape) * 7919 + shape[-1])
+    x = torch.randn(shape, generator=gen, device=cuda).to(dtype)
+    g = torch.randn(shape, generator=gen, device=cuda).to(dtype)
+    res = []
+    for form in (lambda t: t, _off):
+        xf = form(x.detach()).requires_grad_()
+        s = torch.full(enc, 0.013, device=cuda).requires_grad_()
+        o = torch.full(enc, 3.0, device=cuda).requires_grad_()
+        y = Q.quantize_dequantize(xf, s, o, -128, 127)
+        y.backward(form(g))
+        lo, hi = Q.minmax(xf.detach(), enc)
+        res.append((y.detach(), xf.grad, s.grad, o.grad, lo, hi))
+    a, b = res
+    for k in (0, 1, 4, 5):
+        assert torch.equal(a[k], b[k]), k
+    for k in (2, 3):
+        # one unit where the value stands, and the sums' own error (2^-52 of the terms' magnitudes)
+        terms = (g.double().abs() * 128).sum() * 2.0 ** -40
+        assert bool(((a[k] - b[k]).abs().double() <= a[k].abs().double() * 2.0 ** -23 + terms).all())
