@@ -55,3 +55,30 @@ def test_vectors_and_edges_equal_single_elements(cuda, shape, enc, dtype):
         # one unit where the value stands, and the sums' own error (2^-52 of the terms' magnitudes)
         terms = (g.double().abs() * 128).sum() * 2.0 ** -40
         assert bool(((a[k] - b[k]).abs().double() <= a[k].abs().double() * 2.0 ** -23 + terms).all())
+
+
+# One check for the quotients of a vector: zeros of either sign, values outside the range of the
+# residual steps, infinities and NaN, one in a vector or all of it, and scales outside theirs.
+@pytest.mark.parametrize("scale", [0.013, 2.0 ** -61, 2.0 ** 61, 2.0 ** -60, 2.0 ** 60, 1e-39, 0.0])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_quotients_of_a_vector_equal_single_ones(cuda, scale, dtype):
+    gen = torch.Generator(device=cuda).manual_seed(11)
+    special = torch.tensor([0.0, -0.0, 2.0 ** -40, -2.0 ** -41, 2.0 ** 40, -2.0 ** 41, 1e-45, 3e38,
+                            float("inf"), -float("inf"), float("nan"), 6.5e4], device=cuda)
+    x = torch.randn(64, 8, 8, generator=gen, device=cuda)
+    x[1:49, :, 3] = special.repeat_interleave(4)[:, None]       # one of a vector
+    x[49:61] = special[:, None, None]                           # all of it
+    x = x.flatten().to(dtype)
+    g = torch.randn(x.shape, generator=gen, device=cuda).to(dtype)
+    res = []
+    for form in (lambda t: t, _off):
+        xf = form(x.detach()).requires_grad_()
+        s = torch.tensor(scale, device=cuda).requires_grad_()
+        o = torch.tensor(0.0, device=cuda).requires_grad_()
+        y = Q.quantize_dequantize(xf, s, o, -128, 127)
+        y.backward(form(g))
+        q = Q.quantize(form(x.detach()), s.detach(), o.detach(), -128, 127) if dtype == torch.float32 else y
+        res.append([t.detach().view(torch.int32 if t.dtype == torch.float32 else torch.int16)
+                    for t in (y, xf.grad, q)])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
