@@ -978,11 +978,10 @@ __global__ __launch_bounds__(256) void zero_floats(int64_t n, float *p) {
     p[i] = 0.0f;
 }
 
-
 // Bias gradients: the partials of the nwg workgroups (or 16-row chunks) summed in a fixed order,
 // 16 interleaved chains per channel: 128 partials of the resident recurrence take 5.5 us (one
-// chain over the clustered form's 16 took 7.6).  swap_h > 0: written in the (r, z, n) gate order (the first two blocks of swap_h
-// swapped).
+// chain over the clustered form's 16 took 7.6).  swap_h > 0: written in the (r, z, n) gate order
+// (the first two blocks of swap_h swapped).
 __global__ __launch_bounds__(256) void fold_bias(int nwg, int C, const double *__restrict__ part,
                                                  float *__restrict__ dbw, float *__restrict__ dbr,
                                                  int swap_h) {
