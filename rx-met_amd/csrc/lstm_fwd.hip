@@ -1294,6 +1294,13 @@ static int lstm_res_launch(const RecArgs &ra, const StepParams &sp, int npl, int
   }
   const int64_t nc = static_cast<int64_t>(sp.c.hi) - sp.c.lo + 1;
   if (nc > kGlobalLutMaxCodes) return 0;
+  int device = 0, ncu = 0, dev_lds = 0;
+  RXMET_CHECK_HIP(hipGetDevice(&device));
+  RXMET_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
+  RXMET_CHECK_HIP(hipDeviceGetAttribute(&dev_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+  const bool clustered = H > 256;
+  const int ns = clustered ? kLresTile : ((B + 1) / 2 <= ncu ? 2 : 4);
+  const int ks = H > 256 ? 8 : (H > 128 ? 4 : (H > 64 ? 2 : 1)), upw = ks == 4 ? 2 : 1;
   LresParams p{};
   int tab = kTabLds;
   ActLut lut{};
@@ -1312,9 +1319,13 @@ static int lstm_res_launch(const RecArgs &ra, const StepParams &sp, int npl, int
     lut.tanh_n = static_cast<int>(nc);
     lut.total += lut.tanh_n;
   } else {
-    // 16-bit entries (output code and mask) when the output grid leaves room for the mask bit
-    tab = !lds_gates ? kTabGlobal
-          : sp.tanh_c.hi - sp.tanh_c.lo < (1 << 15) ? kTabLds16 : kTabGlobalTanh;
+    // 16-bit entries (output code and mask) when the output grid leaves room for the mask bit and
+    // the LDS for the table (a 16-bit cell grid's 128 KB beside the h rows and the gate tables: two
+    // planes of h above H = 256 leave 3966 gate entries, of the 4096 that may be asked for)
+    const bool fits16 = sp.tanh_c.hi - sp.tanh_c.lo < (1 << 15) &&
+                        lres_lds_bytes(npl, ks, ns, lut.total, static_cast<int>(nc)) +
+                                kLresStaticLds <= static_cast<size_t>(dev_lds);
+    tab = !lds_gates ? kTabGlobal : (fits16 ? kTabLds16 : kTabGlobalTanh);
     lut.gtanh_off = lut.gtotal;
     lut.gtanh_n = static_cast<int>(nc);
     lut.gtotal += lut.gtanh_n;
@@ -1355,11 +1366,6 @@ static int lstm_res_launch(const RecArgs &ra, const StepParams &sp, int npl, int
   p.hid_mult = sp.hidden.mult;
   p.hid_shift = sp.hidden.shift;
 
-  int device = 0, ncu = 0;
-  RXMET_CHECK_HIP(hipGetDevice(&device));
-  RXMET_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
-  const bool clustered = H > 256;
-  const int ns = clustered ? kLresTile : ((B + 1) / 2 <= ncu ? 2 : 4);
   const int mode = ra.hidden == nullptr ? kLresInfer : (ra.ckb ? kLresCodes : kLresFloat);
   const void *fn = npl == 1 ? (mode == kLresInfer   ? lres_kernel<1, kLresInfer>(H, ns, tab)
                                : mode == kLresCodes ? lres_kernel<1, kLresCodes>(H, ns, tab)
@@ -1367,7 +1373,6 @@ static int lstm_res_launch(const RecArgs &ra, const StepParams &sp, int npl, int
                             : (mode == kLresInfer   ? lres_kernel<2, kLresInfer>(H, ns, tab)
                                : mode == kLresCodes ? lres_kernel<2, kLresCodes>(H, ns, tab)
                                                     : lres_kernel<2, kLresFloat>(H, ns, tab));
-  const int ks = H > 256 ? 8 : (H > 128 ? 4 : (H > 64 ? 2 : 1)), upw = ks == 4 ? 2 : 1;
   const size_t lds = lres_lds_bytes(npl, ks, ns, p.lds_gates, tab == kTabLds16 ? p.tanh_n : 0);
   RXMET_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds)));

@@ -15,7 +15,7 @@
 //
 // Activations are table lookups (one entry per input code): gate tables in LDS, or in global
 // memory where four grids do not fit; the cell's tanh as 16-bit entries in LDS for a 16-bit cell
-// grid (128 KB, which the weights no longer need), else in global memory.
+// grid (128 KB, which the weights no longer need) where they fit, else in global memory.
 //
 // Measured (recurrence alone; before: clusters of 64-unit members on 16 sequences with W_hh in LDS):
 // H = 256, B = 64, T = 50, 8 bits, inference: 294 -> 55 us; H = 512, B = 512, T = 100, 16-bit cell,
@@ -67,6 +67,9 @@ __device__ __forceinline__ float lres_clamp(float s, float lo, float hi, unsigne
   if (s < lo || s > hi) m |= bit;
   return fminf(fmaxf(s, lo), hi);
 }
+
+// LDS beside the dynamic part: the meeting's flags of cluster.h (two words), rounded up.
+constexpr size_t kLresStaticLds = 64;
 
 constexpr size_t lres_lds_bytes(int npl, int ks, int ns, int lds_gates, int tanh16) {
   return static_cast<size_t>(2) * ns * npl * (64 * ks + 16) + 4 * static_cast<size_t>(lds_gates) +

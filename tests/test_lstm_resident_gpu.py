@@ -10,7 +10,8 @@ import torch
 
 import lstm_ops
 import lstm_oracle as LO
-from test_lstm_gpu import _case, _dev, _gpu_forward, _wrap
+import rxmet_lstm_abi as L
+from test_lstm_gpu import _case, _config, _dev, _gpu_forward, _weights, _wrap
 
 pytestmark = pytest.mark.gpu
 
@@ -47,6 +48,30 @@ def test_resident_forward_matches_oracle(cuda, case):
     dec = lstm_ops.decode_saved_codes(cod[3], prm, B)
     for n in lstm_ops.CODED_FIELDS:
         np.testing.assert_array_equal(saved[n].cpu().numpy(), dec[n].cpu().numpy(), err_msg=n)
+
+
+@pytest.mark.parametrize("case", [(3, 9, 4, 272), (3, 11, 4, 512)])
+@pytest.mark.parametrize("gate_bits", [9, 10])
+def test_tables_that_do_not_fit_beside_two_h_planes(cuda, case, gate_bits):
+    """Two planes of h above H = 256, a 16-bit cell grid and 4096 gate-input codes together (four
+    10-bit grids) ask for 164352 bytes of LDS with the 16-bit tanh table, more than a workgroup
+    has (163840): the table stays in global memory.  Four 9-bit grids leave room for it."""
+    T, B, I, H = case
+    print(f"[lstm resident tables] {case} {gate_bits}", flush=True)
+    c = _config("c4")
+    for n in ("input", "forget", "cell", "output"):
+        c.op[L.OP[f"{n}_gate_input"]].bits = gate_bits
+    c.op[L.OP["output"]].bits = 10
+    Wi, Wh, bi, bh = _weights(I, H, 21)
+    g = np.random.default_rng(22)
+    x = (g.random((T, B, I)) * 2 - 1).astype(np.float32)
+    p = LO.finalize(LO.calibrate(Wi, Wh, bi, bh, x, None, None, mode=LO.ACT_CR), c, H, True)
+    args = (Wi, Wh, bi, bh, x, None, None)
+    exp = LO.forward_quant(*args[:5], p, None, None, mode=LO.ACT_LIBM_EXACT)
+    for training in (True, False):
+        out, hn, cn, _ = _gpu_forward(cuda, args, p, training)
+        for n, t in (("output", out), ("h_n", hn), ("c_n", cn)):
+            np.testing.assert_array_equal(t.cpu().numpy(), exp[n], err_msg=n)
 
 
 def test_cluster_timeout_poisons_the_outputs(cuda, monkeypatch):
