@@ -809,9 +809,12 @@ struct ColGeo {
 // runs: block b handles chunks sp, sp + splits, ... (`passes` of them, sp = b % splits) of
 // run b / splits, so that the blocks in flight read adjacent memory; one partial per block,
 // or (kFold, direct) the block's encoding gradients.
-// vec: a chunk moves whole vectors between the first and the last 16-byte boundary inside it, and
-// the up to E - 1 elements before and after them one by one (launch_decomp's rule).
-template <class W>
+// EDGES: a chunk moves whole vectors between the first and the last 16-byte boundary inside it, and
+// the up to E - 1 elements before and after them one by one (launch_decomp's rule); else vec: runs of
+// whole vectors.  A kernel of its own: where the edges are always empty their 64-bit boundaries and
+// two element-wise branches cost both streaming passes (a one-shot quantizer node of [2048, 5000] fp16:
+// 18.3 -> 17.9 us).
+template <class W, bool EDGES>
 __global__ __launch_bounds__(kThreads) void k_runs(W w, Geo geo, int64_t splits, int passes,
                                                    int vec,
                                                    typename W::Acc *__restrict__ partial) {
@@ -827,7 +830,7 @@ __global__ __launch_bounds__(kThreads) void k_runs(W w, Geo geo, int64_t splits,
     const int64_t beg = first + q * step;
     if (beg >= geo.inner) break;
     const int64_t end = min(geo.inner, beg + kChunk);
-    if (vec) {
+    if constexpr (EDGES) {
       const int64_t a = rb + beg, z = rb + end;
       const int64_t va = (a + W::E - 1) / W::E, vz = z / W::E;
       w.vec_block(e, va, static_cast<int>(vz - va), acc);  // none when a chunk's end has vz < va
@@ -835,6 +838,8 @@ __global__ __launch_bounds__(kThreads) void k_runs(W w, Geo geo, int64_t splits,
       const int nh = static_cast<int>(h - a), nt = static_cast<int>(z - t);
       if (static_cast<int>(threadIdx.x) < nh) w.elem(e, a + threadIdx.x, acc);
       if (static_cast<int>(threadIdx.x) < nt) w.elem(e, t + threadIdx.x, acc);
+    } else if (vec) {
+      w.vec_block(e, (rb + beg) / W::E, static_cast<int>((end - beg) / W::E), acc);
     } else {
       const int n = static_cast<int>(end - beg);
       for (int i = threadIdx.x; i < n; i += kThreads) w.elem(e, rb + beg + i, acc);
@@ -964,10 +969,13 @@ static int launch_decomp(const Plan &pl, const W &w, bool aligned, void *partial
   // backward 34.9 us and forward 19.8, as vectors 22.4 and 14.6; in runs of a row 32.4 and 21.7,
   // 24.3 and 16.4).  4-byte elements fill two lines: rows of 4099 fp32 take 29.3 us one by one and
   // 31.6 as vectors that no row starts on a boundary of.
-  const bool edges = aligned && (vec || W::E >= 8);
   if (pl.kind == KIND_RUNS) {
-    hipLaunchKernelGGL(k_runs<W>, dim3(static_cast<unsigned>(pl.runs * pl.splits)),
-                       dim3(kThreads), 0, s, w, pl.geo, pl.splits, pl.passes, int(edges), part);
+    auto fn = &k_runs<W, false>;
+    if constexpr (W::E >= 8) {
+      if (aligned && !vec) fn = &k_runs<W, true>;
+    }
+    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(pl.runs * pl.splits)), dim3(kThreads), 0, s, w,
+                       pl.geo, pl.splits, pl.passes, int(vec), part);
   } else if (pl.kind == KIND_SEGS) {
     const int64_t nv = vec ? pl.inner / W::E : pl.inner;
     int shift = 0;
