@@ -11,8 +11,8 @@
 //   1. prologue    : x, h_prev and W codes as bf16 operand planes for the weight-gradient
 //                    GEMMs (h codes recovered exactly from the dequantised h);
 //   2. recurrence  : up to H = 256 with 8-bit R one workgroup per two or four sequences with
-//                    all of R_q in its VGPRs (bwd_recurrence_res: dq as 31-bit fixed point
-//                    in four byte digits, dh += R_q dq on int8 MFMA); else both
+//                    all of R_q in its VGPRs (bwd_recurrence_res: dq as its exact three bf16
+//                    terms, dh += R_q dq on bf16 MFMA); else both
 //                    directions walk t = T-1..0 in one clustered launch
 //                    (bwd_recurrence_cl: a batch tile's hidden units split over a cluster of
 //                    workgroups, dq * scale_R exchanged through global memory each step and
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(64) void pack_rt_frags(int H, int KS2, const float 
     wd[q] = pack4_i8(by[0], by[1], by[2], by[3]);
   }
   frag[static_cast<size_t>(idx) * 64 + lane] = v4i{wd[0], wd[1], wd[2], wd[3]};
-  if (rowsum != nullptr && s == 0 && lane < 16 && k < H) {
+  if (s == 0 && lane < 16 && k < H) {
     int sum = 0;
     for (int c = 0; c < C; ++c) sum += static_cast<int>(Rq[static_cast<size_t>(k) * C + c]);
     rowsum[k] = static_cast<float>(sum);
@@ -661,29 +661,43 @@ __global__ __launch_bounds__(256 * UT) void bwd_recurrence_cl(BwdArgs a0, BwdArg
 // ---------------------------------------------------------------------------------
 // 2a. resident backward recurrence (H <= 256, R_q of signed 8 bits)
 // ---------------------------------------------------------------------------------
-// One workgroup owns NS sequences and all H units and holds all of R_q in its VGPRs as int8 MFMA
-// operands, as the resident forward does; a step exchanges nothing with other workgroups.  Per
-// step a lane finishes the STE pointwise of one (sequence, unit), the gate gradients scaled by
-// R's channel scales become 31-bit fixed point on one exponent per sequence (the step's largest
-// magnitude, met through LDS), split into four signed byte digits, and dh += R_q dq runs on
-// v_mfma_i32_16x16x64_i8 with row 4 s + q = digit q of sequence s: the four digit sums of a
-// (sequence, unit) arrive in one lane's accumulator.  Each term is off by at most 2^-30 of the
-// sequence's largest, the digit sums are exact and their combination is within two units in the
-// last place of fp32 (the three bf16 terms of the clustered form are exact, but accumulate over 3H
-// products in fp32): the error of a whole step's gradients against 64 bits is no larger (training
-// steps at H = 100 and 256: 2.9e-7 and 4.8e-7 here, 2.9e-7 and 4.9e-7 clustered; the later fp32
-// weight products dominate).
+// One workgroup owns NS sequences and all H units and holds all of R_q as bf16 MFMA operands in its
+// VGPRs (the last KL of the K chunks in LDS, where 256 VGPRs a wave are not enough); a step exchanges
+// nothing with other workgroups.  Per step a lane finishes the STE pointwise of one (sequence, unit)
+// and splits the gate gradients, scaled by R's channel scales, into their exact three bf16 terms, as
+// the clustered form does; dh += R_q dq runs on v_mfma_f32_16x16x32_bf16 with row 4 s + q = term q
+// of sequence s, so the three sums of a (sequence, unit), fp32 over all 3H channels, arrive in one
+// lane's accumulator and are added smallest first.  Every gradient keeps its 24 bits whatever the
+// others of its sequence are (31-bit fixed point on one exponent per sequence, on int8 MFMA, takes 360
+// us in place of the 422 below, and loses the units that see only gradients far below the largest).
 //
-// A digit must sit next to its neighbours' along K: a lane holds the four digits of one channel,
-// four lanes of a quad hold four consecutive channels, and two DPP exchanges transpose the 4 x 4
-// bytes so that each lane writes one aligned word of one digit row.
+// The rows have two buffers, so that a step meets at one workgroup barrier.
 //
 // Measured (both directions of B = 256, T = 200, H = 256, saved codes): 1021 us clustered ->
-// 345 us.  Bound: the chain of one step (two LDS exchanges, 24 MFMA per wave, about 200 VALU).
+// 422 us.  Bound: the chain of one step (one LDS exchange, 48 MFMA per wave whose row operands
+// are 24 KB per wave from LDS, about 150 VALU).
 constexpr int kResMaxH = 256;
 
-constexpr size_t bwd_res_lds(int ks2, int ns) {
-  return 256 + static_cast<size_t>(4) * ns * (64 * ks2 + 16);
+constexpr int bwd_res_row(int kb) { return 64 * kb + 16; }  // bytes
+constexpr size_t bwd_res_lds(int kb, int ns, int kl, int waves, int upw) {
+  return static_cast<size_t>(6) * ns * bwd_res_row(kb) + static_cast<size_t>(1024) * kl * waves * upw;
+}
+
+// R_q [H][3H] -> per (unit tile ut, 32-channel block kb, lane l) the bf16 B fragment R_q[j][k + e],
+// e = 0..7, with j = 16 ut + l % 16 and k = 32 kb + 8 (l / 16), zero beyond 3H (codes of at most
+// 8 bits are bf16 values).
+__global__ __launch_bounds__(64) void pack_rt_res(int H, int KB, const float *__restrict__ Rq,
+                                                  uint4 *__restrict__ rt) {
+  const int l = threadIdx.x, idx = blockIdx.x, kb = idx % KB, ut = idx / KB;
+  const int j = 16 * ut + l % 16, k0 = 32 * kb + 8 * (l / 16);
+  unsigned w[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int k = k0 + 2 * e;  // 3H is even
+    const float *p = Rq + static_cast<size_t>(j) * 3 * H + k;
+    w[e] = k < 3 * H ? pack_bf16x2(v2f{p[0], p[1]}) : 0u;
+  }
+  rt[static_cast<size_t>(idx) * 64 + l] = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
 // One element's step inputs as they are in memory.
@@ -730,31 +744,34 @@ __device__ __forceinline__ float bwd_point_raw(const BwdRaw<CODES> &r, const Bwd
   return z * dht;
 }
 
-template <int KS2, int UPW, int NS, bool CODES>
-__global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1, int nblk) {
+// KB: 32-channel blocks of 3H (a.KB of them used), the last KL of them in LDS.
+template <int KB, int UPW, int NS, int KL, bool CODES>
+__global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1, int nblk, int nkb) {
   constexpr bool kMerge = UPW == 2 && NS == 2;  // two tiles' sums share one pass of the lanes
   constexpr int NP = UPW == 2 && !kMerge ? 2 : 1;
-  constexpr int ROW = 64 * KS2 + 16;
-  extern __shared__ __align__(16) unsigned char smem[];
-  unsigned *smax = reinterpret_cast<unsigned *>(smem);  // [NS][8]: a wave's largest per sequence
-  int8_t *pl = reinterpret_cast<int8_t *>(smem + 256);  // [4 NS][ROW] digit rows
+  constexpr bool kDeep = NP == 1;  // inputs loaded two steps ahead; one where registers are short
+  constexpr int ROW = bwd_res_row(KB), BUF = 3 * NS * ROW, KV = KB - KL;
+  extern __shared__ __align__(16) unsigned char smem[];  // [2][3 NS][ROW] term rows, weights
   const int dir = blockIdx.x / nblk, blk = blockIdx.x % nblk;
   const BwdArgs &a = dir == 0 ? a0 : a1;
   const int H = a.H, C = 3 * H, B = a.B, T = a.T, UT = H / 16;
   const int tid = threadIdx.x, w = tid / 64, l = tid % 64, grp = l / 16, e = l % 16;
+  uint4 *wl = reinterpret_cast<uint4 *>(smem + 2 * BUF) + w * (UPW * KL * 64) + l;
 
-  for (int i = tid; i < NS * ROW; i += blockDim.x) reinterpret_cast<int *>(pl)[i] = 0;
-  if (tid < NS * 8) smax[tid] = 0u;
+  for (int i = tid; i < 2 * BUF / 4; i += blockDim.x) reinterpret_cast<int *>(smem)[i] = 0;
 
-  v4i rfr[UPW][KS2];
+  auto weight = [&](int u, int k) {
+    const int ut = UPW * w + u;
+    return ut < UT && k < nkb ? a.rt[(static_cast<size_t>(ut) * nkb + k) * 64 + l] : make_uint4(0, 0, 0, 0);
+  };
+  v8bf rfr[UPW][KV];
 #pragma unroll
-  for (int u = 0; u < UPW; ++u)
+  for (int u = 0; u < UPW; ++u) {
 #pragma unroll
-    for (int s = 0; s < KS2; ++s) {
-      const int ut = UPW * w + u;
-      rfr[u][s] = ut < UT && s < a.KS2 ? a.rfrag[(static_cast<size_t>(ut) * a.KS2 + s) * 64 + l]
-                                       : v4i{0, 0, 0, 0};
-    }
+    for (int s = 0; s < KV; ++s) rfr[u][s] = __builtin_bit_cast(v8bf, weight(u, s));
+#pragma unroll
+    for (int s = 0; s < KL; ++s) wl[(u * KL + s) * 64] = weight(u, KV + s);
+  }
 
   // the elements this lane finishes: pass k, (sequence b, unit j)
   const int seq = kMerge ? grp % 2 : grp;
@@ -763,7 +780,7 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
   double sbw[NP][3], sbr[NP][3];
   unsigned od[NP], ol[NP], oc[NP], om[NP];  // dp / dq stores; h, v codes (or v), mask loads
   const float *gp[NP];
-  int8_t *pw[NP];
+  unsigned char *pw[NP];
   bool own[NP], ok[NP];
   const float *gbase = a.gv_on ? (a.gv ? a.gv : a.h) : a.dh_new + static_cast<size_t>(B) * H;
   const int64_t gst = a.gv_on ? (a.gv ? a.gv_t : 0) : static_cast<int64_t>(B) * H;
@@ -792,11 +809,11 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
       effr[k][g] = a.eff_r[g * H + jc];
       sbw[k][g] = sbr[k][g] = 0.0;
     }
-    // this lane writes digit row 4 seq + e % 4, channels of the quad's four units
-    pw[k] = pl + (own[k] ? (4 * seq + e % 4) * ROW + 16 * ut + (e & ~3) : 0);
+    pw[k] = smem + (own[k] ? 3 * seq * ROW + 2 * j : 0);
   }
-  // A operand: row l % 16 = 4 s + q (rows without a sequence repeat one that exists)
-  const int8_t *ar = pl + (e % (4 * NS)) * ROW + 16 * grp;
+  // A operand: row l % 16 = 4 s + q, term q of sequence s (rows without one repeat the first; their
+  // sums are not read)
+  const unsigned char *ar = smem + (e / 4 < NS && e % 4 < 3 ? 3 * (e / 4) + e % 4 : 0) * ROW + 16 * grp;
 
   const unsigned step_c = 4u * static_cast<unsigned>(B) * C, step_h = 4u * static_cast<unsigned>(B) * H;
   const unsigned step_blk = static_cast<unsigned>((B + 15) / 16) * H;  // x 128 B of v codes, x 32 B
@@ -848,9 +865,8 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
   const unsigned ones = CODES ? 0u : (a.ih_m ? 0u : 1u) | (a.hh_m ? 0u : 2u) | (a.gin_m ? 0u : 4u) |
                                          (a.gout_m ? 0u : 8u) | (a.h_m ? 0u : 16u);
 
-  auto step = [&](int t, BwdRaw<CODES> (&r)[NP]) {
-    float dpv[NP][3], dqv[NP][3], dhl[NP], sv[NP][3];
-    unsigned mx = 0u;
+  auto step = [&](int t, int par, BwdRaw<CODES> (&r)[NP]) {
+    float dpv[NP][3], dqv[NP][3], dhl[NP];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
       if (nog) r[k].g = 0.0f;
@@ -864,20 +880,23 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
       for (int g = 0; g < 3; ++g) {
         sbw[k][g] += static_cast<double>(dpv[k][g]);
         sbr[k][g] += static_cast<double>(dqv[k][g]);
-        sv[k][g] = dqv[k][g] * effr[k][g];
-        // magnitudes as integers: a NaN is the largest
-        const unsigned m = __builtin_bit_cast(unsigned, sv[k][g]) & 0x7fffffffu;
-        if (own[k]) mx = max(mx, m);
+      }
+      // term q of the element's gates g to [3 seq + q][g H + j]
+      unsigned zr[3], n0[3];
+      split3x2(v2f{dqv[k][0] * effr[k][0], dqv[k][1] * effr[k][1]}, zr[0], zr[1], zr[2]);
+      split3x2(v2f{dqv[k][2] * effr[k][2], 0.0f}, n0[0], n0[1], n0[2]);
+      if (own[k]) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          unsigned char *d = pw[k] + par * BUF + q * ROW;
+          *reinterpret_cast<uint16_t *>(d) = static_cast<uint16_t>(zr[q]);
+          *reinterpret_cast<uint16_t *>(d + 2 * H) = static_cast<uint16_t>(zr[q] >> 16);
+          *reinterpret_cast<uint16_t *>(d + 4 * H) = static_cast<uint16_t>(n0[q]);
+        }
       }
     }
-    mx = row16_max(mx);
-    if constexpr (kMerge) {
-      const auto sw = __builtin_amdgcn_permlane32_swap(mx, mx, false, false);
-      mx = max(sw[0], sw[1]);
-    }
-    if (e == 0 && (kMerge ? grp < 2 : grp < NS)) smax[seq * 8 + w] = mx;
     lds_barrier();
-    load(t - 2, r);
+    load(t - (kDeep ? 2 : 1), r);
     {
       const size_t tt = static_cast<size_t>(t);
       const auto rp = cluster::buffer_rsrc(a.dp + tt * B * C, step_c);
@@ -890,49 +909,35 @@ __global__ __launch_bounds__(512) void bwd_recurrence_res(BwdArgs a0, BwdArgs a1
           buf_f32(rq, dqv[k][g], od[k] + 4u * g * H);
         }
     }
-    const uint4 m0 = *reinterpret_cast<const uint4 *>(smax + (seq < NS ? seq : 0) * 8);
-    const uint4 m1 = *reinterpret_cast<const uint4 *>(smax + (seq < NS ? seq : 0) * 8 + 4);
-    const unsigned top = max(max(max(m0.x, m0.y), max(m0.z, m0.w)), max(max(m1.x, m1.y), max(m1.z, m1.w)));
-    const int ex2 = fixed_exp(top);
-    const bool bad = fixed_bad(top);
+    v4f acc[UPW];
 #pragma unroll
-    for (int k = 0; k < NP; ++k)
+    for (int u = 0; u < UPW; ++u) acc[u] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int g = 0; g < 3; ++g) {
-        const unsigned tr = quad_transpose8(bad ? 0u : fixed_digits(sv[k][g], ex2), e);
-        if (own[k]) *reinterpret_cast<unsigned *>(pw[k] + g * H) = tr;
-      }
-    lds_barrier();
-    v4i acc[UPW];
+    for (int s = 0; s < KB; ++s) {
+      const v8bf af = *reinterpret_cast<const v8bf *>(ar + par * BUF + 64 * s);
 #pragma unroll
-    for (int u = 0; u < UPW; ++u) acc[u] = v4i{0, 0, 0, 0};
-#pragma unroll
-    for (int s = 0; s < KS2; ++s) {
-      const v4i af = *reinterpret_cast<const v4i *>(ar + 64 * s);
-#pragma unroll
-      for (int u = 0; u < UPW; ++u) acc[u] = mfma_i8(af, rfr[u][s], acc[u]);
+      for (int u = 0; u < UPW; ++u)
+        acc[u] = mfma_bf16(af, s < KV ? rfr[u][s < KV ? s : 0]
+                                      : __builtin_bit_cast(v8bf, wl[(u * KL + s - KV) * 64]), acc[u]);
     }
+    float sum[UPW];
 #pragma unroll
-    for (int k = 0; k < NP; ++k) {
-      int sum[4];
+    for (int u = 0; u < UPW; ++u) sum[u] = (acc[u][2] + acc[u][1]) + acc[u][0];
+    if constexpr (kMerge)
+      sum[0] = __builtin_bit_cast(
+          float, __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, sum[0]),
+                                                  __builtin_bit_cast(unsigned, sum[1]), false, false)[0]);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        sum[q] = acc[k][q];
-        if constexpr (kMerge)
-          sum[q] = __builtin_amdgcn_permlane32_swap(acc[0][q], acc[UPW - 1][q], false, false)[0];
-      }
-      const float add = bad ? NAN : fixed_sum(sum[0], sum[1], sum[2], sum[3], ex2);
-      dhc[k] = dhl[k] + add;
-    }
+    for (int k = 0; k < NP; ++k) dhc[k] = dhl[k] + sum[k];
   };
   BwdRaw<CODES> ra[NP], rb[NP];
   load(T - 1, ra);
-  load(T - 2, rb);
+  if constexpr (kDeep) load(T - 2, rb);
   lds_barrier();  // the zeroed rows are in LDS
   for (int t = T - 1;;) {
-    step(t, ra);
+    step(t, 0, ra);
     if (--t < 0) break;
-    step(t, rb);
+    step(t, 1, kDeep ? rb : ra);
     if (--t < 0) break;
   }
 
@@ -1201,12 +1206,19 @@ static int backward_prologue(int T, int B, int I, int H, const rxmet_gru_bwd_dir
   return 0;
 }
 
+// The kernel for nkb blocks, and its KB, KL and unit tiles per wave.
+struct BwdResKernel {
+  const void *fn;
+  int kb, kl, upw;
+};
 template <int NS, bool CODES>
-static const void *bwd_res_kernel(int ks2) {
-  if (ks2 <= 3) return reinterpret_cast<const void *>(&bwd_recurrence_res<3, 1, NS, CODES>);
-  if (ks2 <= 6) return reinterpret_cast<const void *>(&bwd_recurrence_res<6, 1, NS, CODES>);
-  // four sequences in the float format would need more than the 256 VGPRs of a wave
-  return reinterpret_cast<const void *>(&bwd_recurrence_res<12, 2, (CODES ? NS : 2), CODES>);
+static BwdResKernel bwd_res_kernel(int nkb) {
+  if (nkb <= 6) return {reinterpret_cast<const void *>(&bwd_recurrence_res<6, 1, NS, 0, CODES>), 6, 0, 1};
+  if (nkb <= 12) return {reinterpret_cast<const void *>(&bwd_recurrence_res<12, 1, NS, 0, CODES>), 12, 0, 1};
+  // the fewest blocks in LDS that leave no register spilled; four sequences in the float format would
+  // need more still
+  constexpr int kNs = CODES ? NS : 2, kKl = !CODES ? 5 : (NS == 4 ? 6 : 2);
+  return {reinterpret_cast<const void *>(&bwd_recurrence_res<24, 2, kNs, kKl, CODES>), 24, kKl, 2};
 }
 
 // Resident recurrence of every direction in one ordinary launch; returns 1 when launched, 0 when
@@ -1215,7 +1227,6 @@ static const void *bwd_res_kernel(int ks2) {
 // clustered form.
 static int backward_recurrence_resident(BwdPlan *plans, int ndir, int T, int B, int I, int H,
                                         hipStream_t stream) {
-  const int KS2 = (3 * H + 63) / 64;
   if (H > kResMaxH || std::getenv("RXMET_NO_CLUSTER") != nullptr ||
       cluster::spin_limit() != cluster::kSpinLimit)
     return 0;
@@ -1229,23 +1240,25 @@ static int backward_recurrence_resident(BwdPlan *plans, int ndir, int T, int B, 
   RXMET_CHECK_HIP(hipGetDevice(&device));
   RXMET_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
   const bool codes = plans[0].ba.vc != nullptr;
-  const int ns = static_cast<int64_t>(ndir) * ((B + 1) / 2) <= ncu || (!codes && KS2 > 6) ? 2 : 4;
+  int nkb = (3 * H + 31) / 32;
+  const int ns = static_cast<int64_t>(ndir) * ((B + 1) / 2) <= ncu || (!codes && nkb > 12) ? 2 : 4;
   int nblk = (B + ns - 1) / ns;
   for (int k = 0; k < ndir; ++k) {
     plans[k].nbias = nblk;
-    hipLaunchKernelGGL(pack_rt_frags, dim3((H / 16) * KS2), dim3(64), 0, stream, H, KS2,
-                       plans[k].d->R_q, const_cast<v4i *>(plans[k].ba.rfrag),
-                       static_cast<float *>(nullptr));
+    hipLaunchKernelGGL(pack_rt_res, dim3((H / 16) * nkb), dim3(64), 0, stream, H, nkb, plans[k].d->R_q,
+                       const_cast<uint4 *>(plans[k].ba.rt));
     RXMET_CHECK_LAUNCH();
   }
-  const void *fn = ns == 2 ? (codes ? bwd_res_kernel<2, true>(KS2) : bwd_res_kernel<2, false>(KS2))
-                           : (codes ? bwd_res_kernel<4, true>(KS2) : bwd_res_kernel<4, false>(KS2));
-  const int ks = KS2 <= 3 ? 3 : (KS2 <= 6 ? 6 : 12), upw = ks == 12 ? 2 : 1;
-  const int waves = (H / 16 + upw - 1) / upw;
-  void *args[] = {&plans[0].ba, &plans[ndir > 1 ? 1 : 0].ba, &nblk};
+  const BwdResKernel kn =
+      ns == 2 ? (codes ? bwd_res_kernel<2, true>(nkb) : bwd_res_kernel<2, false>(nkb))
+              : (codes ? bwd_res_kernel<4, true>(nkb) : bwd_res_kernel<4, false>(nkb));
+  const int waves = (H / 16 + kn.upw - 1) / kn.upw;
+  const size_t lds = bwd_res_lds(kn.kb, ns, kn.kl, waves, kn.upw);
+  RXMET_CHECK_HIP(hipFuncSetAttribute(kn.fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      static_cast<int>(lds)));
+  void *args[] = {&plans[0].ba, &plans[ndir > 1 ? 1 : 0].ba, &nblk, &nkb};
   rxmet::prof::Scope ps__("gru_bwd_recurrence", stream);
-  RXMET_CHECK_HIP(hipLaunchKernel(fn, dim3(ndir * nblk), dim3(64 * waves), args,
-                                  bwd_res_lds(ks, ns), stream));
+  RXMET_CHECK_HIP(hipLaunchKernel(kn.fn, dim3(ndir * nblk), dim3(64 * waves), args, lds, stream));
   return 1;
 }
 

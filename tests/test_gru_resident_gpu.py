@@ -89,6 +89,40 @@ def test_resident_backward_matches_oracle_and_clustered(cuda, case, monkeypatch)
             assert np.linalg.norm(q.cpu().numpy() - e) <= 1e-5 * scale, (d, n)
 
 
+@pytest.mark.parametrize("case", [(6, 3, 5, 64, "8b-sym"), (6, 5, 4, 128, "c3"), (6, 4, 5, 256, "c3"),
+                                  (3, 515, 4, 256, "8b-sym")])
+@pytest.mark.parametrize("small", [1e-5, 1e-9, 1e-20])
+def test_resident_backward_keeps_small_gradients(cuda, case, small):
+    """Two blocks of units that R does not couple, the output gradients of the second `small` times
+    the first's: its dh0, its channels of dR and its bias gradients are as close to the 64-bit sums as
+    the first's, relative to their own norm (32-bit sums over 3 H and T B terms: a few 1e-7)."""
+    T, B, I, H, cfg = case
+    print(f"[gru resident bwd small] {case} {small}", flush=True)
+    W, R, bw, br, x, h0, qp = _case(T, B, I, H, cfg, 51, True)
+    half = np.arange(H) >= H // 2
+    mixed = np.arange(H) % 3 == 0  # every K chunk holds units of both blocks
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    for second in (half, mixed):
+        cols = np.tile(second, 3)
+        R2 = np.where(second[:, None] == cols[None, :], R, np.float32(0))
+        dh = (np.random.default_rng(6).standard_normal((T + 1, B, H)) * 1e-2).astype(np.float32)
+        dh[..., second] *= np.float32(small)
+        fwd = GO.forward_quant(W, R2, bw, br, x, qp, h0=h0, training=True)
+        exp = GO.backward_quant(fwd, dh, qp)
+        args = [(t(W), t(R2), t(bw), t(br), t(x), t(h0), gru_ops.GRUQuantParams.from_struct(qp))]
+        o = gru_ops.forward_quant_codes_dirs(True, T, B, I, H, args)[0]
+        got = gru_ops.backward_quant_codes_dirs(
+            T, B, I, H, [(o[2], o[3], o[4], o[5], o[6], t(dh), o[0], o[1], args[0][6], o[7:])],
+            torch_layout=False)[0]
+        torch.cuda.synchronize()
+        got = dict(zip(("dx", "dW", "dR", "dbw", "dbr", "dh0"), (a.cpu().numpy() for a in got)))
+        for block, c in ((second, cols), (~second, ~cols)):
+            for n, sel in (("dh0", block), ("dR", c), ("dW", c), ("dbr", c)):
+                e, a = (np.asarray(v[n], np.float64)[..., sel] for v in (exp, got))
+                err = np.linalg.norm(a - e) / (np.linalg.norm(e) + 1e-300)
+                assert err <= 1e-5, (n, int(block.sum()), err)
+
+
 def test_resident_backward_keeps_nan_in_its_sequence(cuda):
     """A NaN and an infinity in two sequences' output gradients reach every unit's dh0 and the
     weight gradients, and leave the other sequences' dx and dh0 as they are without them."""
