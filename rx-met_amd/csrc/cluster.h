@@ -120,7 +120,8 @@ __device__ __forceinline__ bool wait(unsigned *counter, unsigned arrivals, int *
   return ok != 0;
 }
 
-__device__ __forceinline__ void store_coherent(unsigned *p, unsigned v) {
+template <typename U>
+__device__ __forceinline__ void store_coherent(U *p, U v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

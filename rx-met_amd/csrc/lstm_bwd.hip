@@ -952,7 +952,7 @@ struct BwdWorkspace {
     const size_t Bpad = (static_cast<size_t>(B) + kBB - 1) / kBB * kBB, G = H / kBcUnits + 1;
     wfrag_cl = o; o += al(sizeof(v4i) * std::max(64 * (H / 16) * KS2, bres_frags(H)));
     csum = o; o += al(sizeof(float) * KS2 * H);
-    xp = o; o += al(std::max(2 * 3 * Bpad * C, sizeof(float) * bres_exchange(B, H)));
+    xp = o; o += al(std::max(2 * 3 * Bpad * C, sizeof(double) * bres_exchange(B, H)));
     xe = o; o += al(sizeof(int) * 2 * Bpad * G);
     sync = o; o += al(sizeof(unsigned) * cluster::kCounterStride * (Bpad / kBresTile + 1));
     // stepped recurrence: K-split parts of dh, the cell gradient, W_hh codes as bf16 planes
@@ -1133,7 +1133,7 @@ static int lstm_backward_impl(int32_t T, int32_t B, int32_t I, int32_t H,
                   a16(sv.cell_tanh_m) && a16(sv.hidden_m);
   if (!stepped && ck_aligned) {
     const int rc = lstm_bwd_res_launch(ba, sp, sv.w_hh_q, reinterpret_cast<v4i *>(wsb + ws.wfrag_cl),
-                                       reinterpret_cast<float *>(wsb + ws.xp),
+                                       reinterpret_cast<double *>(wsb + ws.xp),
                                        reinterpret_cast<unsigned *>(wsb + ws.sync), stream,
                                        &timeout_flag);
     if (rc < 0) return rc;

@@ -5,17 +5,21 @@
 // operands: a step exchanges nothing with other workgroups.  Up to H = 512 a cluster of up to four
 // workgroups shares eight sequences; member m owns 128 units, that is 512 of the 4H channels, and
 // holds W_hh of those channels for every unit.  It multiplies its own gate gradients only, and the
-// members exchange partial dh (16 KB per member and step) instead of gate gradients (64 KB).
+// members exchange partial dh (32 KB per member and step) instead of gate gradients (64 KB).
 //
 // The gate gradients scaled by W's channel scales become 31-bit fixed point on one exponent per
-// (sequence, workgroup), in four signed byte digits; row 4 s + q of v_mfma_i32_16x16x64_i8 is digit
-// q of sequence s, so the four digit sums of a (sequence, unit) arrive in one lane: each term is off
-// by at most 2^-30 of the workgroup's largest, the digit sums are exact, their combination within
-// two units in the last place of fp32, and a cluster adds its members' partials in member order.
-// Gradients of a whole training step against 64 bits: 5.0e-7 (22-bit fixed point before: 5.1e-7).
+// (sequence, group of 64 units), in four signed byte digits; row 4 s + q of
+// v_mfma_i32_16x16x64_i8 is digit q of sequence s, so the four digit sums of a (sequence, unit) over
+// a group's 256 channels arrive in one lane.  Each term is off by at most 2^-30 of its group's
+// largest; the rest is exact up to the order of a few sums in double: the digit sums and their
+// combination per group, the groups' and the members' (which meet as doubles), rounded once to fp32.
+// The clustered form's groups are the same, with 22 bits.  (One exponent per workgroup, sums met and
+// combined in fp32: 731 us in place of the 803 below, and a group whose gradients are far below
+// another's loses its bits.)
+// Gradients of a whole training step against 64 bits: 5.0e-7 (clustered form: 5.1e-7).
 //
-// Measured (recurrence of B = 512, T = 100, H = 512, saved codes): 949 -> 727 us against clusters of
-// 64-unit members on 16 sequences.  What bounds it there: two elements per lane (about 470 VALU per
+// Measured (recurrence of B = 512, T = 100, H = 512, saved codes): 949 -> 803 us against clusters of
+// 64-unit members on 16 sequences.  What bounds it there: two elements per lane (some 500 VALU per
 // step), 64 MFMA per wave and the exchange.
 #pragma once
 
@@ -32,15 +36,15 @@ struct BresParams {
   float c_s, c_z, t_s, t_z;
   const v4i *frag;     // lstm_pack_bres
   int G, ncl, ntiles;  // cluster
-  float *xp;           // [2][ntiles][G dst][G src][8][128] partial dh
+  double *xp;          // [2][ntiles][G dst][G src][8][128] partial dh
   unsigned *counters;
   int *timeout;
   unsigned spin_limit;
 };
 
-// W_hh codes [4H][H] -> frag[((m UT + jt) KS + s) 64 + lane]: channels k = 64 s + 16 (lane / 16) ..
-// + 15 of member m's, gate k / U and unit m U + k % U, against unit 16 jt + lane % 16 (zero beyond
-// the member's channels and H).
+// W_hh codes [4H][H] -> frag[((m UT + jt) KS + s) 64 + lane]: channels 64 s + 16 (lane / 16) .. + 15 of
+// member m's, in groups of 64 units and by gate inside a group (K step s: gate s % 4 of units m U +
+// 64 (s / 4) .. + 63), against unit 16 jt + lane % 16 (zero beyond H).
 __global__ __launch_bounds__(64) void lstm_pack_bres(int H, int U, int KS, const float *__restrict__ wq,
                                                      v4i *__restrict__ frag) {
   const int lane = threadIdx.x, idx = blockIdx.x, UT = H / 16;
@@ -52,8 +56,8 @@ __global__ __launch_bounds__(64) void lstm_pack_bres(int H, int U, int KS, const
     int by[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int k = 64 * s + 16 * (lane / 16) + 4 * q + e, g = k / U, u = m * U + k % U;
-      by[e] = g < 4 && u < H ? static_cast<int>(wq[static_cast<size_t>(g * H + u) * H + j]) : 0;
+      const int g = s % 4, u = m * U + 64 * (s / 4) + 16 * (lane / 16) + 4 * q + e;
+      by[e] = u < H ? static_cast<int>(wq[static_cast<size_t>(g * H + u) * H + j]) : 0;
     }
     wd[q] = pack4_i8(by[0], by[1], by[2], by[3]);
   }
@@ -84,9 +88,11 @@ __global__ __launch_bounds__(512) void lstm_bwd_recurrence_res(BwdArgs a, BresPa
   constexpr int RB = kCluster ? 2 : 1;   // blocks of 16 digit rows
   constexpr bool kDeep = NP == 1;        // inputs loaded two steps ahead
   constexpr int ROW = 64 * KS + 16;
+  constexpr int NG = KS / 4;                               // groups of 64 units
+  constexpr int WPG = UPW == 2 && !kCluster ? 2 : 4;       // waves whose elements make a group
   extern __shared__ __align__(16) unsigned char smem[];
   unsigned *smax = reinterpret_cast<unsigned *>(smem);  // [NS][8]: a wave's largest per sequence
-  unsigned *stop = smax + 64;                           // [8]: a sequence's largest
+  unsigned *stop = smax + 64;                           // [8][2]: a cluster's largest per group
   int8_t *pl = reinterpret_cast<int8_t *>(smem + 512);  // [4 NS][ROW] digit rows
   const int H = a.H, C = 4 * H, B = a.B, T = a.T, UT = H / 16;
   const int U = kCluster ? kBresMember : H;             // units of the workgroup
@@ -99,7 +105,7 @@ __global__ __launch_bounds__(512) void lstm_bwd_recurrence_res(BwdArgs a, BresPa
   for (int i = tid; i < 128; i += blockDim.x) smax[i] = 0u;
   // operands: the units whose dh this wave sums (all of the layer's in a cluster)
   v4i wf[UPW][KS];
-  const int ksn = (4 * U + 63) / 64;
+  const int ksn = 4 * ((U + 63) / 64);
 #pragma unroll
   for (int u = 0; u < UPW; ++u)
 #pragma unroll
@@ -154,7 +160,7 @@ __global__ __launch_bounds__(512) void lstm_bwd_recurrence_res(BwdArgs a, BresPa
       for (int g = 0; g < 4; ++g) sw[k][g] = a.s_whh[g * H + jc];
       dh[k] = a.grad_hn && ok[k] ? a.grad_hn[row] : 0.0f;
       dc[k] = a.grad_cn && ok[k] ? a.grad_cn[row] : 0.0f;
-      pw[k] = pl + (own[k] ? (4 * seq + e % 4) * ROW + 16 * utl + (e & ~3) : 0);
+      pw[k] = pl + (own[k] ? (4 * seq + e % 4) * ROW + 256 * (utl / 4) + 16 * (utl % 4) + (e & ~3) : 0);
     }
     auto load = [&](int t, BresRaw<CODES> (&r)[NP]) {
       const size_t tt = static_cast<size_t>(t > 0 ? t : 0);
@@ -267,7 +273,7 @@ __global__ __launch_bounds__(512) void lstm_bwd_recurrence_res(BwdArgs a, BresPa
         dc[k] = mdc * go[1];
         mx[k] = own[k] ? m : 0u;
       }
-      // the largest magnitude of each sequence: its lanes, then the waves through LDS
+      // the largest magnitude of each sequence's groups: a wave's lanes, then the waves through LDS
       if constexpr (kCluster) {
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
@@ -300,31 +306,39 @@ __global__ __launch_bounds__(512) void lstm_bwd_recurrence_res(BwdArgs a, BresPa
         load(t - (kDeep ? 2 : 1), r);
         store();
       }
-      auto top_of = [&](int s) {
-        const uint4 x = *reinterpret_cast<const uint4 *>(smax + s * 8);
-        const uint4 y = *reinterpret_cast<const uint4 *>(smax + s * 8 + 4);
-        return max(max(max(x.x, x.y), max(x.z, x.w)), max(max(y.x, y.y), max(y.z, y.w)));
+      auto top_of = [&](int s, int g) {  // of sequence s, group g
+        const unsigned *m = smax + s * 8 + WPG * g;
+        const uint2 x = *reinterpret_cast<const uint2 *>(m);
+        unsigned v = max(x.x, x.y);
+        if constexpr (WPG == 4) {
+          const uint2 y = *reinterpret_cast<const uint2 *>(m + 2);
+          v = max(v, max(y.x, y.y));
+        }
+        return v;
       };
-      unsigned top[NP];
+      unsigned top[kCluster ? NP : NG];  // of the lane's elements' group; else of all groups
+#pragma unroll
+      for (int k = 0; k < (kCluster ? NP : NG); ++k)
+        top[k] = kCluster ? top_of(sq[k % NP], w / WPG) : top_of(sq[0] < NS ? sq[0] : 0, k);
 #pragma unroll
       for (int k = 0; k < NP; ++k) {
-        top[k] = k > 0 && !kCluster ? top[0] : top_of(sq[k] < NS ? sq[k] : 0);
-        const int ex = fixed_exp(top[k]);
-        const bool bad = fixed_bad(top[k]);
+        const unsigned own_top = kCluster ? top[k] : top_of(sq[0] < NS ? sq[0] : 0, w / WPG);
+        const int ex = fixed_exp(own_top);
+        const bool bad = fixed_bad(own_top);
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const unsigned d = quad_transpose8(bad ? 0u : fixed_digits(sv[k][g], ex), e);
-          if (own[k]) *reinterpret_cast<unsigned *>(pw[k] + g * U) = d;
+          if (own[k]) *reinterpret_cast<unsigned *>(pw[k] + 64 * g) = d;
         }
-        if (kCluster && w == 0 && e == 0) stop[sq[k]] = top[k];
+        if (kCluster && w % WPG == 0 && e == 0) stop[2 * sq[k] + w / WPG] = own_top;
       }
       lds_barrier();
-      // dh of the block's sequences for the wave's units
-      auto product = [&](int rb, v4i (&acc)[UPW]) {
+      // a group's part of dh of the block's sequences for the wave's units, in digit sums
+      auto product = [&](int rb, int q, v4i (&acc)[UPW]) {
 #pragma unroll
         for (int u = 0; u < UPW; ++u) acc[u] = v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
+        for (int s = 4 * q; s < 4 * q + 4; ++s) {
           const v4i af = *reinterpret_cast<const v4i *>(ar[rb] + 64 * s);
 #pragma unroll
           for (int u = 0; u < UPW; ++u) acc[u] = mfma_i8(af, wf[u][s], acc[u]);
@@ -337,22 +351,30 @@ __global__ __launch_bounds__(512) void lstm_bwd_recurrence_res(BwdArgs a, BresPa
         const unsigned base = (par * p.ntiles + tile) * G * G;
         const unsigned dst = w / 2;
         if (dst < G) {
-          float *x = p.xp + static_cast<size_t>((base + dst * G + m0) * kBresTile) * kBresMember +
+          double *x = p.xp + static_cast<size_t>((base + dst * G + m0) * kBresTile) * kBresMember +
                      64 * (w % 2) + e;
 #pragma unroll
           for (int rb = 0; rb < RB; ++rb) {
-            product(rb, acc);
-            const unsigned tp = stop[4 * rb + grp];
-            const int ex = fixed_exp(tp);
-            const bool bad = fixed_bad(tp);
+            double v[UPW];
 #pragma unroll
-            for (int u = 0; u < UPW; ++u) {
-              const v4i &s = acc[u];
-              const float v = bad ? NAN : fixed_sum(s[0], s[1], s[2], s[3], ex);
-              cluster::store_coherent(
-                  reinterpret_cast<unsigned *>(x + (4 * rb + grp) * kBresMember + 16 * u),
-                  __builtin_bit_cast(unsigned, v));
+            for (int q = 0; q < NG; ++q) {
+              product(rb, q, acc);
+              const unsigned tp = stop[2 * (4 * rb + grp) + q];
+              const int ex = fixed_exp(tp);
+              const bool bad = fixed_bad(tp);
+#pragma unroll
+              for (int u = 0; u < UPW; ++u) {
+                const double f = bad ? static_cast<double>(NAN)
+                                     : fixed_sum(fixed_pair(acc[u][0], acc[u][1]),
+                                                 fixed_pair(acc[u][2], acc[u][3]), ex);
+                v[u] = q == 0 ? f : v[u] + f;
+              }
             }
+#pragma unroll
+            for (int u = 0; u < UPW; ++u)
+              cluster::store_coherent(
+                  reinterpret_cast<unsigned long long *>(x + (4 * rb + grp) * kBresMember + 16 * u),
+                  __builtin_bit_cast(unsigned long long, v[u]));
           }
         }
         cluster::arrive(counter);
@@ -361,40 +383,48 @@ __global__ __launch_bounds__(512) void lstm_bwd_recurrence_res(BwdArgs a, BresPa
         store();
         alive = cluster::wait(counter, epoch * G, p.timeout, p.spin_limit);
         if (!alive) return;
-        const auto xr = cluster::buffer_rsrc(p.xp, 8u * p.ntiles * G * G * kBresTile * kBresMember);
-        float part[NP][4];
+        const auto xr = cluster::buffer_rsrc(p.xp, 16u * p.ntiles * G * G * kBresTile * kBresMember);
+        double part[NP][4];
 #pragma unroll
         for (int k = 0; k < NP; ++k)
 #pragma unroll
           for (unsigned s = 0; s < 4; ++s) {
             const unsigned src = s < G ? s : 0;
             part[k][s] = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(
-                           xr, 4u * (((base + m0 * G + src) * kBresTile + sq[k]) * kBresMember + 16 * w + e),
+                double, __builtin_amdgcn_raw_buffer_load_b64(
+                           xr, 8u * (((base + m0 * G + src) * kBresTile + sq[k]) * kBresMember + 16 * w + e),
                            0, 16 /* sc1: from the coherence point */));
           }
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
-          float v = part[k][0];
+          double v = part[k][0];
 #pragma unroll
           for (unsigned s = 1; s < 4; ++s)
             if (s < G) v += part[k][s];
-          dh[k] = v;
+          dh[k] = static_cast<float>(v);
         }
       } else {
-        product(0, acc);
+        double sum[NP];
+        bool bad = false;
 #pragma unroll
-        for (int k = 0; k < NP; ++k) {
-          int sum[4];
+        for (int q = 0; q < NG; ++q) {
+          product(0, q, acc);
+          bad |= fixed_bad(top[q]);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            sum[q] = acc[k < UPW ? k : 0][q];
-            if constexpr (kMerge)
-              sum[q] = __builtin_amdgcn_permlane32_swap(acc[0][q], acc[UPW - 1][q], false, false)[0];
+          for (int k = 0; k < NP; ++k) {
+            const v4i &d = acc[k < UPW ? k : 0];
+            int lo = fixed_pair(d[0], d[1]), hi = fixed_pair(d[2], d[3]);
+            if constexpr (kMerge) {
+              const v4i &d1 = acc[UPW - 1];
+              lo = __builtin_amdgcn_permlane32_swap(lo, fixed_pair(d1[0], d1[1]), false, false)[0];
+              hi = __builtin_amdgcn_permlane32_swap(hi, fixed_pair(d1[2], d1[3]), false, false)[0];
+            }
+            const double f = fixed_sum(lo, hi, fixed_exp(top[q]));
+            sum[k] = q == 0 ? f : sum[k] + f;
           }
-          dh[k] = fixed_bad(top[k]) ? NAN
-                                    : fixed_sum(sum[0], sum[1], sum[2], sum[3], fixed_exp(top[k]));
         }
+#pragma unroll
+        for (int k = 0; k < NP; ++k) dh[k] = bad ? NAN : static_cast<float>(sum[k]);
       }
     };
 
@@ -437,10 +467,10 @@ static const void *bres_kernel(int H, int ns) {
   return ns == 2 ? bres_kernel<2, CODES>(H) : bres_kernel<4, CODES>(H);
 }
 
-// Fragments and exchange of the form that takes H (v4i elements, floats).
+// Fragments and exchange of the form that takes H (v4i elements, doubles).
 static size_t bres_frags(int H) {
   const size_t U = H > 256 ? kBresMember : H, G = (H + U - 1) / U;
-  return G * (H / 16) * ((4 * U + 63) / 64) * 64;
+  return G * (H / 16) * (4 * ((U + 63) / 64)) * 64;
 }
 static size_t bres_exchange(int B, int H) {
   const size_t G = (H + kBresMember - 1) / kBresMember, nt = (B + kBresTile - 1) / kBresTile;
@@ -453,7 +483,7 @@ static size_t bres_exchange(int B, int H) {
 // workgroup then has a CU of its own, else four; above, clusters of ceil(H / 128) on eight.  A
 // forced poll limit (the timeout tests) asks for the clustered form up to H = 256.
 static int lstm_bwd_res_launch(const BwdArgs &a, const StepParams &sp, const float *whh_q, v4i *frag,
-                               float *xp, unsigned *sync, hipStream_t stream, int **timeout_flag) {
+                               double *xp, unsigned *sync, hipStream_t stream, int **timeout_flag) {
   const int H = a.H, B = a.B;
   const bool clustered = H > 256, codes = a.ckb != nullptr;
   if (H > kMaxHB || std::getenv("RXMET_NO_CLUSTER") != nullptr ||
@@ -465,7 +495,7 @@ static int lstm_bwd_res_launch(const BwdArgs &a, const StepParams &sp, const flo
     if (!fits(sp.gout[g])) return 0;
   // one step's rows are addressed with 31-bit byte offsets (gates: 16 bytes per unit)
   if (16.0 * ((B + 15) / 16 * 16) * H >= 2147483648.0) return 0;
-  if (4.0 * bres_exchange(B, H) >= 2147483648.0) return 0;
+  if (8.0 * bres_exchange(B, H) >= 2147483648.0) return 0;
   BresParams p{};
   for (int g = 0; g < 4; ++g) {
     p.gs[g] = static_cast<float>(sp.gout[g].dscale);
@@ -476,7 +506,7 @@ static int lstm_bwd_res_launch(const BwdArgs &a, const StepParams &sp, const flo
   p.t_s = static_cast<float>(sp.tanh_c.dscale);
   p.t_z = static_cast<float>(sp.tanh_c.zp - (codes ? sp.tanh_c.lo : 0));
   p.frag = frag;
-  const int U = clustered ? kBresMember : H, ksn = (4 * U + 63) / 64;
+  const int U = clustered ? kBresMember : H, ksn = 4 * ((U + 63) / 64);
   p.G = (H + U - 1) / U;
   int device = 0, ncu = 0;
   RXMET_CHECK_HIP(hipGetDevice(&device));

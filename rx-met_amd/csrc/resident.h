@@ -83,14 +83,13 @@ __device__ __forceinline__ unsigned fixed_digits(float v, int ex) {
   return (static_cast<unsigned>(q) + 0x00808080u) ^ 0x00808080u;
 }
 
-// The sum of products from its four digit sums (each exact in fp32, below 2^24 in magnitude), back
-// at the values' scale: the high and the low pair rounded once each, then their sum; within two
-// units in the last place of the exact sum.  (The same in double: 14 more instructions of twice the
-// length per element.)
-__device__ __forceinline__ float fixed_sum(int s0, int s1, int s2, int s3, int ex) {
-  const float hi = __builtin_fmaf(static_cast<float>(s3), 256.0f, static_cast<float>(s2));
-  const float lo = __builtin_fmaf(static_cast<float>(s1), 256.0f, static_cast<float>(s0));
-  return ldexpf(__builtin_fmaf(hi, 65536.0f, lo), -ex);
+// Two neighbouring digit sums over at most 256 products of bytes (each within 2^22) as one integer.
+__device__ __forceinline__ int fixed_pair(int s0, int s1) { return s1 * 256 + s0; }
+
+// The sum of products from the pairs of its four digit sums, back at the values' scale; exact (47
+// bits).  In fp32 the pairs would be rounded, an error that stays where they cancel.
+__device__ __forceinline__ double fixed_sum(int lo, int hi, int ex) {
+  return __builtin_ldexp(__builtin_fma(static_cast<double>(hi), 65536.0, static_cast<double>(lo)), -ex);
 }
 
 }  // namespace rxmet

@@ -112,6 +112,42 @@ def test_resident_backward_matches_oracle(cuda, case):
         assert np.linalg.norm(a.cpu().numpy() - e) <= 1e-5 * (np.linalg.norm(e) + 1e-30), n
 
 
+@pytest.mark.parametrize("case", [(5, 3, 4, 128), (5, 5, 4, 208), (3, 515, 3, 256), (5, 9, 4, 384),
+                                  (4, 19, 3, 512)])
+@pytest.mark.parametrize("small", [1e-5, 1e-9, 1e-20])
+def test_resident_backward_keeps_small_groups(cuda, case, small):
+    """Groups of 64 units of two kinds that W_hh does not couple, the output gradients of the second
+    kind `small` times the first's (a member of a cluster holds one group of each): its dh0, dc0 and
+    its channels of dW_hh and db_hh are as close to the oracle's 64-bit sums as the first's, relative
+    to their own norm (each term within 2^-30 of its group's largest, sums of at most 4 H and T B
+    terms: a few 1e-7)."""
+    T, B, I, H = case
+    print(f"[lstm resident bwd small] {case} {small}", flush=True)
+    args, _, p = _case(T, B, I, H, "default", 16, True, True)
+    second = np.arange(H) // 64 % 2 == 1
+    rows = np.tile(second, 4)
+    args = list(args)
+    args[1] = np.where(rows[:, None] == second[None, :], args[1], np.float32(0))
+    exp_f = LO.forward_quant(*args[:5], p, args[5], args[6], mode=LO.ACT_LIBM_EXACT)
+    g = np.random.default_rng(10)
+    scale = np.where(second, np.float32(small), np.float32(1))
+    go, gh, gc = ((g.standard_normal(s) * 0.1).astype(np.float32) * scale
+                  for s in ((T, B, H), (B, H), (B, H)))
+    exp = LO.backward_quant(exp_f, p, go, gh, gc)
+    Wi, Wh, bi, bh, x, h0, c0 = (_dev(a, cuda) for a in args)
+    prm = _wrap(p)
+    saved = lstm_ops.forward_quant(x, Wi, Wh, bi, bh, h0, c0, prm, True, codes=True)[3]
+    got = lstm_ops.backward_quant(saved, prm, *(_dev(a, cuda) for a in (go, gh, gc)))
+    torch.cuda.synchronize()
+    got = dict(zip(("dx", "dW_ih", "dW_hh", "db_ih", "db_hh", "dh0", "dc0"), got))
+    for kind in (second, ~second):
+        r = np.tile(kind, 4)
+        for n, pick in (("dh0", np.s_[:, kind]), ("dc0", np.s_[:, kind]), ("dW_hh", r), ("db_hh", r)):
+            e, a = (np.asarray(v, np.float64)[pick] for v in (exp[n], got[n].cpu().numpy()))
+            err = np.linalg.norm(a - e) / (np.linalg.norm(e) + 1e-300)
+            assert err <= 1e-5, (n, int(kind.sum()), err)
+
+
 @pytest.mark.parametrize("H", [64, 512])
 def test_resident_backward_keeps_nan_in_its_sequence(cuda, H):
     """A NaN and an infinity in two sequences' output gradients reach every unit's dh0 of those
