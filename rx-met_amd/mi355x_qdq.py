@@ -524,10 +524,8 @@ def quantize_dequantize_minmax(tensor: torch.Tensor, mn: torch.Tensor, mx: torch
             and mx.dtype == torch.float32 and mn.is_contiguous() and mx.is_contiguous()
             and mn.shape == mx.shape and tensor.dtype in _IO_CODE and qmax > qmin):
         return None
-    call = _minmax_call(tensor.shape, tensor.dtype, mn.shape,
-                        None if block_size is None else tuple(block_size), int(qmin), int(qmax),
-                        bool(symmetric), float(sym_offset), float(min_scale),
-                        float(zero_point_shift))
+    call = _call_of(tensor, mn, qmin, qmax, symmetric, min_scale, sym_offset, block_size,
+                    zero_point_shift)
     if call is None:
         return None
     if call.native is not None and tensor.is_contiguous() and _native_node(tensor, mn, mx):
@@ -557,6 +555,16 @@ class _MinMaxCall:
 
     def __init__(self, plan, numerics, native):
         self.plan, self.numerics, self.native = plan, numerics, native
+
+
+def _call_of(tensor, mn, qmin, qmax, symmetric, min_scale, sym_offset, block_size, shift):
+    shape, enc_shape = tensor.shape, mn.shape
+    if torch._C._get_tracing_state() is not None:
+        # a traced tensor's sizes are tensors, which hash by identity
+        shape, enc_shape = (torch.Size(int(d) for d in s) for s in (shape, enc_shape))
+    return _minmax_call(shape, tensor.dtype, enc_shape,
+                        None if block_size is None else tuple(block_size), int(qmin), int(qmax),
+                        bool(symmetric), float(sym_offset), float(min_scale), float(shift))
 
 
 # Keyed by values alone (nothing of a tensor's identity or content); the bound keeps a program
