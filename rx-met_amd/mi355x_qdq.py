@@ -586,11 +586,11 @@ def _minmax_call(shape, dtype, enc_shape, block_size, qmin: int, qmax: int, symm
     if plan.C != math.prod(enc_shape) or t.numel() == 0:
         return None
     scalar = len(enc_shape) == 0 and t.dim() > 0 and internal != dtype
-    native = None
-    if plan.perm is None:  # a permuted layout copies its tensors: the Python Function does that
-        native = _rx.torch_ext().make_plan(list(plan.layout), _IO_CODE[dtype],
-                                           _INTERNAL_CODE[internal], shift, scalar, qmin, qmax,
-                                           symmetric, sym_offset, min_scale)
+    native, ext = None, _rx.torch_ext()
+    # a permuted layout copies its tensors: the Python Function does that
+    if ext is not None and plan.perm is None:
+        native = ext.make_plan(list(plan.layout), _IO_CODE[dtype], _INTERNAL_CODE[internal], shift,
+                               scalar, qmin, qmax, symmetric, sym_offset, min_scale)
     return _MinMaxCall(plan, _numerics(dtype, internal, shift, scalar), native)
 
 

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from pathlib import Path
 from typing import Optional
 
@@ -141,19 +142,22 @@ def load() -> ctypes.CDLL:
 
 def torch_ext():
     """The autograd nodes in C++ (module ``rxmet_torch``, built by build.py), bound to the entry
-    points of the loaded library; raises if it has not been built."""
+    points of the loaded library; None, with one warning, where the module cannot be imported (the
+    Python functions over the same kernels serve then)."""
     global _torch_ext
     if _torch_ext is not None:
-        return _torch_ext
+        return _torch_ext or None
     lib = load()
     import torch  # noqa: F401  (the module's symbols come from PyTorch's libraries)
 
     try:
         import rxmet_torch
     except ImportError as e:
-        raise RxmetError(
-            f"the module rxmet_torch cannot be imported ({e}): build it with "
-            "`python rx-met_amd/build.py`") from e
+        _torch_ext = False
+        warnings.warn(f"the module rxmet_torch cannot be imported ({e}); learnable quantizers run "
+                      "through Python autograd functions, which take the host longer per call. "
+                      "`python rx-met_amd/build.py` builds it", stacklevel=2)
+        return None
     rxmet_torch.bind(*(ctypes.cast(getattr(lib, n), c_ptr).value for n in (
         "rxmet_qdq_forward_minmax", "rxmet_qdq_backward_minmax", "rxmet_qdq_workspace_bytes_ex",
         "rxmet_last_error")))

@@ -4,10 +4,12 @@ import sys
 import warnings
 from pathlib import Path
 
+import pytest
 import torch
 
 sys.path.insert(0, str(Path(__file__).resolve().parents[1] / "rx-met_amd"))
 import mi355x_qdq as Q  # noqa: E402
+import rxmet_lib  # noqa: E402
 
 
 def _call(x, mn):
@@ -32,3 +34,21 @@ def test_traced_calls_share_the_plan_of_their_shape():
     seen.append(_call(torch.zeros(37, 53), mn))
     assert Q._minmax_call.cache_info().currsize == 1
     assert seen[0] is not None and all(c is seen[0] for c in seen)
+
+
+def test_without_the_torch_module(monkeypatch):
+    """Where rxmet_torch cannot be imported the calls warn once and keep the Python Function."""
+    monkeypatch.setattr(rxmet_lib, "_torch_ext", None)
+    monkeypatch.setitem(sys.modules, "rxmet_torch", None)  # its import raises ImportError
+    Q._minmax_call.cache_clear()
+    mn = torch.zeros(5, 1)
+    try:
+        with pytest.warns(UserWarning, match="rxmet_torch"):
+            call = _call(torch.zeros(5, 8), mn)
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            other = _call(torch.zeros(5, 9), mn)
+        for c in (call, other):
+            assert c.plan is not None and c.native is None
+    finally:
+        Q._minmax_call.cache_clear()  # plans without a native node
