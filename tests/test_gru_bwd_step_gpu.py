@@ -32,7 +32,8 @@ def test_stepped_backward(cuda, case, monkeypatch):
     dh_new[0] = 0
     got = _gpu_backward(cuda, fwd, dh_new, qp, T, B, I, H)
     names = ("dx", "dW", "dR", "dbw", "dbr", "dh0")
-    if B <= 600:  # the oracle's cost
+    # the oracle's cost; the last case is the only one of 64 x 64 tiles with two planes
+    if B <= 600 or cfg == "r12-pot2":
         exp = GO.backward_quant(GO.forward_quant(W, R, bw, br, x, qp, h0=h0, training=True), dh_new, qp)
         for name, a in zip(names, got):
             e = exp[name]

@@ -365,7 +365,10 @@ def test_stepped_backward_matches_clustered(cuda, shape, cfg_name, monkeypatch):
     g = np.random.default_rng(14)
     dh_new = (g.standard_normal((T + 1, B, H)) * 1e-2).astype(f32)
     exp = GO.backward_quant(exp_f, dh_new, qp)
+    # a poll limit other than the default selects the clustered form
+    monkeypatch.setenv("RXMET_TEST_SPIN_LIMIT", str((1 << 20) - 1))
     clustered = _gpu_backward(cuda, fwd, dh_new, qp, T, B, I, H)
+    monkeypatch.delenv("RXMET_TEST_SPIN_LIMIT")
     monkeypatch.setenv("RXMET_BWD_STEPPED", "1")
     got = _gpu_backward(cuda, fwd, dh_new, qp, T, B, I, H)
     for name, a, c in zip(("dx", "dW", "dR", "dbw", "dbr", "dh0"), got, clustered):

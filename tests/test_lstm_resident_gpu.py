@@ -112,6 +112,29 @@ def test_resident_backward_matches_oracle(cuda, case):
         assert np.linalg.norm(a.cpu().numpy() - e) <= 1e-5 * (np.linalg.norm(e) + 1e-30), n
 
 
+@pytest.mark.parametrize("case", [(3, 5, 7, 128, "c4", True), (4, 19, 9, 256, "default", True)])
+def test_clustered_backward_matches_oracle(cuda, case, monkeypatch):
+    """The clustered backward, which takes what the resident one declines and which a poll limit
+    other than the default selects up to H = 256: both saved formats, to the bound above."""
+    T, B, I, H, cfg, state = case
+    print(f"[lstm clustered bwd] {case}", flush=True)
+    args, _, p = _case(T, B, I, H, cfg, 18, True, state)
+    exp_f = LO.forward_quant(*args[:5], p, args[5], args[6], mode=LO.ACT_LIBM_EXACT)
+    go = (np.random.default_rng(19).standard_normal((T, B, H)) * 0.1).astype(np.float32)
+    exp = LO.backward_quant(exp_f, p, go, None, None)
+    Wi, Wh, bi, bh, x, h0, c0 = (_dev(a, cuda) for a in args)
+    prm, res = _wrap(p), []
+    monkeypatch.setenv("RXMET_TEST_SPIN_LIMIT", str((1 << 20) - 1))
+    for codes in (False, True):
+        saved = lstm_ops.forward_quant(x, Wi, Wh, bi, bh, h0, c0, prm, True, codes=codes)[3]
+        res.append(lstm_ops.backward_quant(saved, prm, _dev(go, cuda), None, None))
+    torch.cuda.synchronize()
+    for n, a, b in zip(("dx", "dW_ih", "dW_hh", "db_ih", "db_hh", "dh0", "dc0"), *res):
+        assert torch.equal(a, b), n
+        e = np.asarray(exp[n], np.float64)
+        assert np.linalg.norm(a.cpu().numpy() - e) <= 1e-5 * (np.linalg.norm(e) + 1e-30), n
+
+
 @pytest.mark.parametrize("case", [(5, 3, 4, 128), (5, 5, 4, 208), (3, 515, 3, 256), (5, 9, 4, 384),
                                   (4, 19, 3, 512)])
 @pytest.mark.parametrize("small", [1e-5, 1e-9, 1e-20])

@@ -59,9 +59,10 @@ def test_vectors_and_edges_equal_single_elements(cuda, shape, enc, dtype):
 
 # One check for the quotients of a vector: zeros of either sign, values outside the range of the
 # residual steps, infinities and NaN, one in a vector or all of it, and scales outside theirs.
-@pytest.mark.parametrize("scale", [0.013, 2.0 ** -61, 2.0 ** 61, 2.0 ** -60, 2.0 ** 60, 1e-39, 0.0])
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-def test_quotients_of_a_vector_equal_single_ones(cuda, scale, dtype):
+SCALES = [0.013, 2.0 ** -61, 2.0 ** 61, 2.0 ** -60, 2.0 ** 60, 1e-39, 0.0]
+
+
+def _special_vectors(cuda, dtype):
     gen = torch.Generator(device=cuda).manual_seed(11)
     special = torch.tensor([0.0, -0.0, 2.0 ** -40, -2.0 ** -41, 2.0 ** 40, -2.0 ** 41, 1e-45, 3e38,
                             float("inf"), -float("inf"), float("nan"), 6.5e4], device=cuda)
@@ -69,7 +70,17 @@ def test_quotients_of_a_vector_equal_single_ones(cuda, scale, dtype):
     x[1:49, :, 3] = special.repeat_interleave(4)[:, None]       # one of a vector
     x[49:61] = special[:, None, None]                           # all of it
     x = x.flatten().to(dtype)
-    g = torch.randn(x.shape, generator=gen, device=cuda).to(dtype)
+    return x, torch.randn(x.shape, generator=gen, device=cuda).to(dtype)
+
+
+def _bits(t):
+    return t.detach().view(torch.int32 if t.dtype == torch.float32 else torch.int16)
+
+
+@pytest.mark.parametrize("scale", SCALES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_quotients_of_a_vector_equal_single_ones(cuda, scale, dtype):
+    x, g = _special_vectors(cuda, dtype)
     res = []
     for form in (lambda t: t, _off):
         xf = form(x.detach()).requires_grad_()
@@ -77,8 +88,22 @@ def test_quotients_of_a_vector_equal_single_ones(cuda, scale, dtype):
         o = torch.tensor(0.0, device=cuda).requires_grad_()
         y = Q.quantize_dequantize(xf, s, o, -128, 127)
         y.backward(form(g))
-        q = Q.quantize(form(x.detach()), s.detach(), o.detach(), -128, 127) if dtype == torch.float32 else y
-        res.append([t.detach().view(torch.int32 if t.dtype == torch.float32 else torch.int16)
-                    for t in (y, xf.grad, q)])
+        res.append([_bits(t) for t in (y, xf.grad)])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("scale", SCALES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_codes_of_a_vector_equal_single_ones(cuda, scale, dtype):
+    """Quantization, whose quotients of a 16-bit vector share the check too, and its backward."""
+    x, g = _special_vectors(cuda, dtype)
+    res = []
+    for form in (lambda t: t, _off):
+        xf = form(x.detach()).requires_grad_()
+        s = torch.tensor(scale, device=cuda).requires_grad_()
+        q = Q.quantize(xf, s, torch.tensor(0.0, device=cuda), -128, 127)
+        q.backward(form(g.to(q.dtype)))
+        res.append([_bits(t) for t in (q, xf.grad)])
     for a, b in zip(*res):
         assert torch.equal(a, b)
