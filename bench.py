@@ -317,10 +317,11 @@ def _gru_kernel_work(B, T, I, H, D=2, stepped_bwd=False):
     2*M*N*K as counted for the metric; peaks are MI355X's dense figures in TFLOP/s."""
     C = 3 * H
     M = T * B
-    dirs = "both directions in one clustered launch" if D == 2 else "one clustered launch"
-    bwd = ("one direction, stepped: per time step one dh GEMM launch (bf16 MFMA: dq split into "
-           "three bf16 terms against the R codes) and one pointwise launch" if stepped_bwd else
-           f"{dirs} (bf16 MFMA: dq split into three bf16 terms against the R codes)")
+    dirs = (("both directions in one " if D == 2 else "one ") +
+            ("launch, R_q in the registers of a workgroup" if H <= 256 else "clustered launch"))
+    bwd = ("one direction, stepped: one launch per time step (bf16 MFMA: the three bf16 terms of dq "
+           "against the R codes, then the step's pointwise)" if stepped_bwd else
+           f"{dirs} (bf16 MFMA: the three bf16 terms of dq against the R codes)")
     return {
         "gru_fwd_recurrence": (D * 2.0 * M * H * C, INT8_MFMA_PEAK,
                                f"recurrent GEMM R_q.h_q over T steps, {dirs} (int8 MFMA, 16-bit "
@@ -616,8 +617,9 @@ def _lstm_kernel_work(B, T, I, H):
                                 "recurrent GEMM W_hh_q.h_q over T steps (int8 MFMA) with the "
                                 "fused gate / cell / hidden fake-quant"),
         "lstm_bwd_recurrence": (2.0 * M * H * C, INT8_MFMA_PEAK,
-                                "dh GEMM W_hh_q^T.dgates over T steps (int8 MFMA, 3 planes of "
-                                "22-bit block fixed point) with the fused STE pointwise"),
+                                "dh GEMM W_hh_q^T.dgates over T steps (int8 MFMA, four byte "
+                                "digits of 31-bit fixed point per 64 units) with the fused STE "
+                                "pointwise"),
         "lstm_bwd_weight_gemms": (2.0 * M * C * (2 * I + H), BF16_MFMA_PEAK,
                                   "dx, dW_ih, dW_hh GEMMs (float gradient split into three "
                                   "bf16 terms against exact bf16 code planes, MFMA)"),
@@ -1047,8 +1049,8 @@ def _calib_leg(torch, steps: int, warmup: int):
         M = T * B
         rec, gemm = f"{kind}_calibrate_forward", f"{kind}_calibrate_input_gemm"
         work = {rec: (D * 2.0 * M * H * C, FP32_MFMA_PEAK,
-                      "recurrent GEMM h R of every direction over T steps on fp32 MFMA (one "
-                      "clustered launch per direction: gates and statistics fused)"),
+                      "recurrent GEMM h R of every direction over T steps on fp32 MFMA (clustered, "
+                      "a QuantGRU's two directions in one launch: gates and statistics fused)"),
                 gemm: (D * 2.0 * M * C * I, FP32_MFMA_PEAK,
                        "input projection x W of every direction (fp32 MFMA, statistics fused)")}
         dt, p50, p95, kernels, roof = _timed_steps(torch, step, steps, warmup, work,
