@@ -1254,8 +1254,9 @@ static int backward_recurrence_resident(BwdPlan *plans, int ndir, int T, int B, 
               : (codes ? bwd_res_kernel<4, true>(nkb) : bwd_res_kernel<4, false>(nkb));
   const int waves = (H / 16 + kn.upw - 1) / kn.upw;
   const size_t lds = bwd_res_lds(kn.kb, ns, kn.kl, waves, kn.upw);
-  RXMET_CHECK_HIP(hipFuncSetAttribute(kn.fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      static_cast<int>(lds)));
+  if (lds > 64 * 1024)
+    RXMET_CHECK_HIP(hipFuncSetAttribute(kn.fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        static_cast<int>(lds)));
   void *args[] = {&plans[0].ba, &plans[ndir > 1 ? 1 : 0].ba, &nblk, &nkb};
   rxmet::prof::Scope ps__("gru_bwd_recurrence", stream);
   RXMET_CHECK_HIP(hipLaunchKernel(kn.fn, dim3(ndir * nblk), dim3(64 * waves), args, lds, stream));
